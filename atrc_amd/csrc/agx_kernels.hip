@@ -588,24 +588,21 @@ __device__ __forceinline__ bool wt_test(const WtRay &r, V A, V B, V C, float tmi
 }
 
 // ---------------------------------------------------------------- BVH4 (production mode)
-// Slab test of one child box with Atrc's arithmetic, NaN axes ignored (fminf /
-// fmaxf) and the exit distance widened by 2^-21 relative, so that a ray meeting
-// a primitive exactly on its bound is never culled.  Returns the entry
-// distance, or +INF for a miss.
-__device__ __forceinline__ float b4_slab(float lx, float hx, float ly, float hy, float lz, float hz, V o, V inv,
-                                         float tmin, float tmax) {
-    const float nx = inv.x * (lx - o.x), fx = inv.x * (hx - o.x);
-    const float ny = inv.y * (ly - o.y), fy = inv.y * (hy - o.y);
-    const float nz = inv.z * (lz - o.z), fz = inv.z * (hz - o.z);
-    const float t0 = fmaxf(fmaxf(tmin, fminf(nx, fx)), fmaxf(fminf(ny, fy), fminf(nz, fz)));
-    const float t1 = fminf(fminf(tmax, fmaxf(nx, fx)), fminf(fmaxf(ny, fy), fmaxf(nz, fz)));
-    return t0 <= t1 * 1.000000477f ? t0 : INF_F;
-}
-
-// child bound j of a quantized node: origin + byte j of w times the step
-__device__ __forceinline__ float b4_q(float org, uint32_t w, int j, float step) {
-    const float m = float((w >> (8 * j)) & 0xffu) * step;
-    return org + m;
+// A ray as the box tests see it: the reciprocal direction with its magnitude
+// held to 2^80 (so that the products below stay finite for a component that is
+// zero: a plane is then met at +-2^80 times its distance, outside any scene),
+// and which bound of an axis it meets first.
+struct B4Ray {
+    V o, inv;
+    bool nx, ny, nz;  // the ray runs towards smaller x / y / z: the high bound comes first
+};
+__device__ __forceinline__ B4Ray b4_ray(V o, V d) {
+    B4Ray r;
+    r.o = o;
+    constexpr float M = 0x1p80f;
+    r.inv = mk(fminf(fmaxf(1 / d.x, -M), M), fminf(fmaxf(1 / d.y, -M), M), fminf(fmaxf(1 / d.z, -M), M));
+    r.nx = r.inv.x < 0; r.ny = r.inv.y < 0; r.nz = r.inv.z < 0;
+    return r;
 }
 
 struct B4Node {
@@ -613,29 +610,51 @@ struct B4Node {
 };
 __device__ __forceinline__ B4Node b4_load(const float4 *n) { return B4Node{n[0], n[1], n[2], n[3]}; }
 
-// 64-byte node: decode the four children's (conservative) boxes and slab-test them
-__device__ __forceinline__ void b4_children(const B4Node &nd, V o, V inv, float tmin, float tmax, float t[4],
+// Byte j of w as a float (v_cvt_f32_ubyte)
+__device__ __forceinline__ float b4_byte(uint32_t w, int j) { return float((w >> (8 * j)) & 0xffu); }
+
+// 64-byte node: the entry distances of the four children's boxes (+INF where
+// the ray misses) and their codes.  The traversal kernels are bound by vector
+// instructions, so the decode is folded into the slab test: the plane at byte q
+// of an axis is met at t = q (step / d) + (origin - o) / d, one conversion and one FMA
+// where decoding the bound, subtracting o and multiplying takes one conversion and four
+// operations, and the sign of d picks the near and the far bounds once a node instead of
+// a minimum and a maximum a plane (a node visit of 146 vector instructions instead of 225;
+// the 1M-triangle 1920x1080 frame at 64 samples 131.9 -> 122.5 ms, 1280x719 at 8 samples
+// in the watertight mode 10.7 -> 10.0 ms).
+// Conservative: step / d is exact up to 1/d's own rounding (step is a power of
+// two); the offset carries 2 ulp of its own size, so the near offset is
+// lowered and the far one raised by 2^-22 of it (4 ulp); the FMAs and the
+// axes' 1/d differ by at most 4 ulp of t, covered by widening the exit by
+// 2^-21.  Bounds carry the builder's own padding of 2^-20 of their coordinate, which
+// covers the decode's rounding that the builder emulates.  NaN axes (overflow)
+// are ignored by fminf / fmaxf and only cull less.
+__device__ __forceinline__ void b4_children(const B4Node &nd, const B4Ray &r, float tmin, float tmax, float t[4],
                                             uint32_t k[4]) {
     const float4 h = nd.h, cc = nd.cc, qa = nd.qa, qb = nd.qb;
     const uint32_t eb = __float_as_uint(h.w);
-    const float sx = __uint_as_float((eb & 0xffu) << 23), sy = __uint_as_float(((eb >> 8) & 0xffu) << 23),
-                sz = __uint_as_float(((eb >> 16) & 0xffu) << 23);
-    const uint32_t wlx = __float_as_uint(qa.x), whx = __float_as_uint(qa.y), wly = __float_as_uint(qa.z),
-                   why = __float_as_uint(qa.w), wlz = __float_as_uint(qb.x), whz = __float_as_uint(qb.y);
+    const float ax = __uint_as_float((eb & 0xffu) << 23) * r.inv.x,
+                ay = __uint_as_float(((eb >> 8) & 0xffu) << 23) * r.inv.y,
+                az = __uint_as_float(((eb >> 16) & 0xffu) << 23) * r.inv.z;
+    const float bx = (h.x - r.o.x) * r.inv.x, by = (h.y - r.o.y) * r.inv.y, bz = (h.z - r.o.z) * r.inv.z;
+    constexpr float E = 0x1p-22f, W = 1.000000477f;
+    const float bnx = fmaf(-E, fabsf(bx), bx), bny = fmaf(-E, fabsf(by), by), bnz = fmaf(-E, fabsf(bz), bz);
+    const float bfx = fmaf(E, fabsf(bx), bx), bfy = fmaf(E, fabsf(by), by), bfz = fmaf(E, fabsf(bz), bz);
+    const uint32_t lx = __float_as_uint(qa.x), hx = __float_as_uint(qa.y), ly = __float_as_uint(qa.z),
+                   hy = __float_as_uint(qa.w), lz = __float_as_uint(qb.x), hz = __float_as_uint(qb.y);
+    const uint32_t wnx = r.nx ? hx : lx, wfx = r.nx ? lx : hx;
+    const uint32_t wny = r.ny ? hy : ly, wfy = r.ny ? ly : hy;
+    const uint32_t wnz = r.nz ? hz : lz, wfz = r.nz ? lz : hz;
     k[0] = __float_as_uint(cc.x); k[1] = __float_as_uint(cc.y);
     k[2] = __float_as_uint(cc.z); k[3] = __float_as_uint(cc.w);
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-        t[j] = k[j] != BVH4_EMPTY
-                   ? b4_slab(b4_q(h.x, wlx, j, sx), b4_q(h.x, whx, j, sx), b4_q(h.y, wly, j, sy),
-                             b4_q(h.y, why, j, sy), b4_q(h.z, wlz, j, sz), b4_q(h.z, whz, j, sz), o, inv, tmin, tmax)
-                   : INF_F;
-}
-
-// the same for the node at n
-__device__ __forceinline__ void b4_children(const float4 *n, V o, V inv, float tmin, float tmax, float t[4],
-                                            uint32_t k[4]) {
-    b4_children(b4_load(n), o, inv, tmin, tmax, t, k);
+    for (int j = 0; j < 4; ++j) {
+        const float t0 = fmaxf(fmaxf(fmaxf(fmaf(b4_byte(wnx, j), ax, bnx), fmaf(b4_byte(wny, j), ay, bny)),
+                                     fmaf(b4_byte(wnz, j), az, bnz)), tmin);
+        const float t1 = fminf(fminf(fminf(fmaf(b4_byte(wfx, j), ax, bfx), fmaf(b4_byte(wfy, j), ay, bfy)),
+                                     fmaf(b4_byte(wfz, j), az, bfz)), tmax);
+        t[j] = (k[j] != BVH4_EMPTY) & (t0 <= t1 * W) ? t0 : INF_F;
+    }
 }
 
 __device__ __forceinline__ void cswap(float t[4], uint32_t k[4], int a, int b) {
@@ -684,7 +703,8 @@ static_assert((BVH4_RING_CLOSEST & (BVH4_RING_CLOSEST - 1)) == 0 && (BVH4_RING_A
 template <bool STATS, int CAP, bool WT, int TB>
 struct B4Closest {
     static constexpr int SPILL = CAP - BVH4_RING_CLOSEST;  // (node code, entry distance bits)
-    V o, d, inv;
+    B4Ray r;
+    V d;
     float tmin, tmax;
     WtRay wr;
     uint32_t code;
@@ -693,9 +713,9 @@ struct B4Closest {
     HitRec rec;
 
     __device__ __forceinline__ void start(V o_, V d_, float tmin_, float tmax_) {
-        o = o_; d = d_; tmin = tmin_; tmax = tmax_;
-        inv = mk(1 / d.x, 1 / d.y, 1 / d.z);
-        if (WT) wr = wt_ray(o, d);
+        d = d_; tmin = tmin_; tmax = tmax_;
+        r = b4_ray(o_, d_);
+        if (WT) wr = wt_ray(o_, d_);
         code = 0; sp = 0; best_rank = -1;
         rec.ent = -1; rec.prim = -1; rec.t = -1; rec.u = 0; rec.v = 0;
     }
@@ -709,7 +729,7 @@ struct B4Closest {
         if (STATS) c.visits++;
         float t[4];
         uint32_t k[4];
-        b4_children(root, o, inv, tmin, tmax, t, k);
+        b4_children(root, r, tmin, tmax, t, k);
         cswap(t, k, 0, 1); cswap(t, k, 2, 3); cswap(t, k, 0, 2); cswap(t, k, 1, 3); cswap(t, k, 1, 2);
         if (t[0] == INF_F) return true;
         if (t[3] != INF_F)
@@ -729,7 +749,7 @@ struct B4Closest {
             if (STATS) c.visits++;
             float t[4];
             uint32_t k[4];
-            b4_children(N + size_t(code) * BVH4_NODE_VEC4, o, inv, tmin, tmax, t, k);
+            b4_children(b4_load(N + size_t(code) * BVH4_NODE_VEC4), r, tmin, tmax, t, k);
             cswap(t, k, 0, 1); cswap(t, k, 2, 3); cswap(t, k, 0, 2); cswap(t, k, 1, 3); cswap(t, k, 1, 2);
             if (t[0] != INF_F) {
                 if (t[3] != INF_F && sp < CAP)
@@ -754,7 +774,7 @@ struct B4Closest {
                     if (STATS) c.tests++;
                     float tt, uu, vv;
                     const bool hit_tri = WT ? wt_test(wr, mk(p0), mk(p1), mk(p2), tmin, tmax, &tt, &uu, &vv)
-                                            : mt_closest(o, d, tmin, tmax, mk(p0), mk(p1), mk(p2), &tt, &uu, &vv);
+                                            : mt_closest(r.o, d, tmin, tmax, mk(p0), mk(p1), mk(p2), &tt, &uu, &vv);
                     // an exact tie with another entity's hit goes to the entity that
                     // Atrc's aggregate tests later (its tie rank)
                     const int32_t rank = __float_as_int(p2.w);
@@ -769,7 +789,7 @@ struct B4Closest {
                     // against the next float below the current hit distance
                     const int32_t rank = __float_as_int(p2.w);
                     float tb = rank < best_rank ? __uint_as_float(__float_as_uint(tmax) - 1u) : tmax;
-                    if (analytic_closest<STATS>(s.ents[ent], ent, o, d, tmin, &tb, &rec, c)) {
+                    if (analytic_closest<STATS>(s.ents[ent], ent, r.o, d, tmin, &tb, &rec, c)) {
                         tmax = tb;
                         best_rank = rank;
                     }
@@ -805,7 +825,8 @@ __device__ bool b4_closest(const DevScene &s, V o, V d, float tmin, float tmax, 
 template <bool STATS, int CAP, bool WT, int TB>
 struct B4Any {
     static constexpr int SPILL = CAP - BVH4_RING_ANY;
-    V o, d, inv;
+    B4Ray r;
+    V d;
     float tmin, tmax;
     WtRay wr;
     uint32_t code;
@@ -813,9 +834,9 @@ struct B4Any {
     bool occluded;
 
     __device__ __forceinline__ void start(V o_, V d_, float tmin_, float tmax_) {
-        o = o_; d = d_; tmin = tmin_; tmax = tmax_;
-        inv = mk(1 / d.x, 1 / d.y, 1 / d.z);
-        if (WT) wr = wt_ray(o, d);
+        d = d_; tmin = tmin_; tmax = tmax_;
+        r = b4_ray(o_, d_);
+        if (WT) wr = wt_ray(o_, d_);
         code = 0; sp = 0; occluded = false;
     }
 
@@ -826,7 +847,7 @@ struct B4Any {
         if (STATS) c.visits++;
         float t[4];
         uint32_t k[4];
-        b4_children(nd, o, inv, tmin, tmax, t, k);
+        b4_children(nd, r, tmin, tmax, t, k);
         uint32_t next = BVH4_EMPTY;
         for (int j = 0; j < 4; ++j) {
             if (t[j] == INF_F) continue;
@@ -861,11 +882,11 @@ struct B4Any {
                     if (WT) {
                         float tt, uu, vv;
                         if (wt_test(wr, mk(p0), mk(p1), mk(p2), tmin, tmax, &tt, &uu, &vv)) { occluded = true; return true; }
-                    } else if (mt_any(o, d, tmin, tmax, mk(p0), mk(p1), mk(p2))) {
+                    } else if (mt_any(r.o, d, tmin, tmax, mk(p0), mk(p1), mk(p2))) {
                         occluded = true;
                         return true;
                     }
-                } else if (analytic_any<STATS>(s.ents[__float_as_int(p0.w)], o, d, tmin, tmax, c)) {
+                } else if (analytic_any<STATS>(s.ents[__float_as_int(p0.w)], r.o, d, tmin, tmax, c)) {
                     occluded = true;
                     return true;
                 }
