@@ -104,7 +104,8 @@ struct agx_ctx {
     uint32_t g_batch_cap = 0;
     uint64_t g_steps = 0;
     size_t g_wave_cap = 0;
-    size_t g_ms_cap = 0;
+    size_t media_cap = 0, media_nee_cap = 0;  // paths / NEE slots the media buffers hold
+    std::vector<void *> media_allocs;
     std::vector<void *> guide_allocs, guide_wave_allocs;
     hipEvent_t ev[8]{};
     std::vector<hipEvent_t> pool;    // timing / readback events, reused across renders
@@ -135,14 +136,19 @@ struct agx_ctx {
         guide_wave_allocs.clear();
         pb.g_feat = pb.g_out = pb.g_rec = nullptr;
         pb.g_rec_state = nullptr;
-        pb.g_ms = nullptr;
         g_wave_cap = 0;
-        g_ms_cap = 0;
+    }
+    void free_media() {
+        for (void *p : media_allocs) if (p) (void)hipFree(p);
+        media_allocs.clear();
+        pb.g_ms = pb.nee_seg = nullptr;
+        media_cap = media_nee_cap = 0;
     }
     void free_wave() {
         for (void *p : wave_allocs) if (p) (void)hipFree(p);
         wave_allocs.clear();
         free_guide_wave();
+        free_media();
         pb = PathBuffers{};
         counters = nullptr;
         qc_blk = nullptr;
@@ -172,11 +178,15 @@ struct agx_ctx {
         g_wave_cap = n;
         return AGX_OK;
     }
-    // the medium samples of guided renders in media (k_medium_pass)
-    int ensure_guide_media(size_t n) {
-        if (n <= g_ms_cap) return AGX_OK;
-        HIP_TRY(galloc(guide_wave_allocs, &pb.g_ms, 3 * n));
-        g_ms_cap = n;
+    // the medium samples and NEE segments of n paths and L lights in a scene with media (k_media)
+    int ensure_media(size_t n, int L) {
+        const size_t nl = n * size_t(std::max(L, 1));
+        if (n <= media_cap && nl <= media_nee_cap) return AGX_OK;
+        free_media();
+        HIP_TRY(galloc(media_allocs, &pb.g_ms, 3 * n));
+        HIP_TRY(galloc(media_allocs, &pb.nee_seg, nl));
+        media_cap = n;
+        media_nee_cap = nl;
         return AGX_OK;
     }
     // network state; parameters initialised uniform in +-1/sqrt(fan-in) (weights)
@@ -615,13 +625,14 @@ int agx_render(agx_ctx *c, const agx_render_params *p, const volatile int32_t *c
     rc.guide_rec_shift = guide_rec_shift(size_t(per_pass));
     int r = c->ensure_wave(size_t(per_pass), rc.L, wh);
     if (r != AGX_OK) return r;
+    const bool media = (c->ds.features & SF_MEDIA) != 0;
+    if (media && (r = c->ensure_media(size_t(per_pass), rc.L)) != AGX_OK) return r;
     if (guide) {
         if ((r = c->ensure_guide_wave(size_t(per_pass))) != AGX_OK) return r;
         // media: with guiding at medium points, scattering points get their own
-        // network evaluation (k_medium_pass)
+        // network evaluation
         rc.guide_medium_depth = p->guide_medium_depth > 0 ? p->guide_medium_depth : 0;
-        rc.guide_media = ((c->ds.features & SF_MEDIA) && rc.guide_medium_depth > 0) ? 1 : 0;
-        if (rc.guide_media && (r = c->ensure_guide_media(size_t(per_pass))) != AGX_OK) return r;
+        rc.guide_media = (media && rc.guide_medium_depth > 0) ? 1 : 0;
         if (!c->guide_ready || p->guide_reset) {
             if ((r = c->guide_init(p->guide_seed, guide_batch)) != AGX_OK) return r;
         } else if ((r = c->ensure_guide_batch(guide_batch)) != AGX_OK) {
@@ -698,28 +709,28 @@ int agx_render(agx_ctx *c, const agx_render_params *p, const volatile int32_t *c
                 launch_capture_rays(c->pb, 1, c->capture_o[1], c->capture_d[1], c->capture_count + 1,
                                     c->capture_cap, n_shadow_max, c->stream);
             }
+            launch_trace_shadow(c->ds, c->pb, n_shadow_max, stats, c->dcnt + 1, c->stream);
+            if ((r = mark(&e2))) return r;
+            timed.push_back({e0, e1, 0});
+            timed.push_back({e1, e2, 1});
+            if (media) launch_media(c->ds, rc, c->pb, uint32_t(rc.n_paths), c->stream);
             if (guide) {
                 // the network's mixture for every vertex about to be shaded (in media,
                 // at the scattering point the vertex's medium sample reaches)
-                if (rc.guide_media) launch_medium_pass(c->ds, rc, c->pb, uint32_t(rc.n_paths), c->stream);
                 launch_guide_features(c->ds, rc, c->pb, uint32_t(rc.n_paths), c->stream);
                 size_t ef, eg;
                 if ((r = mark(&ef))) return r;
                 launch_guide_infer(c->g_packed, c->g_bias, c->pb.g_feat, c->pb.g_out, cin + 2, uint32_t(rc.n_paths),
                                    c->stream);
                 if ((r = mark(&eg))) return r;
-                timed.push_back({e1, ef, 2});
+                timed.push_back({e2, ef, 2});
                 timed.push_back({ef, eg, 3});
-                e1 = eg;
+                e2 = eg;
             }
-            launch_trace_shadow(c->ds, c->pb, n_shadow_max, stats, c->dcnt + 1, c->stream);
-            if ((r = mark(&e2))) return r;
             launch_reset_counters(cout, c->stream);
             launch_shade(c->ds, rc, c->pb, uint32_t(rc.n_paths), c->stream);
             launch_queue_compact(c->pb, uint32_t(rc.n_paths), rc.L, c->qc_blk, c->stream);
             if ((r = mark(&e3))) return r;
-            timed.push_back({e0, e1, 0});
-            timed.push_back({e1, e2, 1});
             timed.push_back({e2, e3, 2});
             if ((r = readback(cout))) return r;
             std::swap(cin, cout);
@@ -1044,6 +1055,8 @@ int graph_prepare(agx_ctx *c, const agx_render_params *p) {
     const int64_t layer = rc.splat ? int64_t(rc.EW) * rc.EH : wh;
     const int64_t per_pass = plain_pass_size(c, rc, layer, p->spp);
     if (int r = c->ensure_wave(size_t(per_pass), rc.L, wh); r != AGX_OK) return r;
+    if (c->ds.features & SF_MEDIA)
+        if (int r = c->ensure_media(size_t(per_pass), rc.L); r != AGX_OK) return r;
     if (size_t(wh) > c->resolve_cap) {
         if (c->d_resolve) (void)hipFree(c->d_resolve);
         if (c->h_resolve) (void)hipHostFree(c->h_resolve);
@@ -1071,7 +1084,9 @@ int enqueue_render(agx_ctx *c, const agx_render_params *p, hipStream_t st, unsig
     const int64_t total = layer * p->spp;
     const int64_t per_pass = plain_pass_size(c, rc, layer, p->spp);
     if (size_t(per_pass) > c->cap_paths || std::max(rc.L, 1) > c->cap_L || wh > c->cap_wh ||
-        size_t(wh) > c->resolve_cap)
+        size_t(wh) > c->resolve_cap ||
+        ((c->ds.features & SF_MEDIA) &&
+         (size_t(per_pass) > c->media_cap || size_t(per_pass) * size_t(std::max(rc.L, 1)) > c->media_nee_cap)))
         return fail(AGX_E_INVALID_ARG, "graph batch: render buffers not prepared");
     rc.guide_rec_shift = guide_rec_shift(size_t(per_pass));
     const uint32_t n_closest_max = uint32_t(2 * per_pass), n_shadow_max = uint32_t(per_pass * std::max(rc.L, 1));
@@ -1096,6 +1111,7 @@ int enqueue_render(agx_ctx *c, const agx_render_params *p, hipStream_t st, unsig
             launch_count_rays(cin, rays, st);
             launch_trace_closest(c->ds, pb, n_closest_max, false, c->dcnt, st);
             launch_trace_shadow(c->ds, pb, n_shadow_max, false, c->dcnt + 1, st);
+            if (c->ds.features & SF_MEDIA) launch_media(c->ds, rc, pb, uint32_t(rc.n_paths), st);
             launch_reset_counters(cout, st);
             launch_shade(c->ds, rc, pb, uint32_t(rc.n_paths), st);
             launch_queue_compact(pb, uint32_t(rc.n_paths), rc.L, c->qc_blk, st);

@@ -653,7 +653,7 @@ __device__ __forceinline__ void b4_children(const B4Node &nd, const B4Ray &r, fl
                                      fmaf(b4_byte(wnz, j), az, bnz)), tmin);
         const float t1 = fminf(fminf(fminf(fmaf(b4_byte(wfx, j), ax, bfx), fmaf(b4_byte(wfy, j), ay, bfy)),
                                      fmaf(b4_byte(wfz, j), az, bfz)), tmax);
-        t[j] = (k[j] != BVH4_EMPTY) & (t0 <= t1 * W) ? t0 : INF_F;
+        t[j] = ((k[j] != BVH4_EMPTY) & (t0 <= t1 * W)) ? t0 : INF_F;
     }
 }
 
@@ -2123,104 +2123,19 @@ __device__ __forceinline__ V vlerp(V a, V b, float t) { return a + (b - a) * t; 
 // exit test is !(t < t_max) so that a NaN segment length ends the loop at once.
 constexpr int MAX_TRACKING_STEPS = 1 << 20;
 
-// Medium::tr (homogeneous.cpp:48-57, heterogeneous.cpp:52-72); r = the stream the caller designates
-__device__ V medium_tr(const DevScene &s, int32_t mi, V a, V b, Rng &r) {
-    if (mi < 0) return mk(1, 1, 1);
-    const DevMedium &m = s.media[mi];
-    if (m.kind == AGX_MEDIUM_HOMOGENEOUS) {
-        const float d = length(a - b);
-        return mk(expf(-m.st.x * d), expf(-m.st.y * d), expf(-m.st.z * d));
-    }
-    if (m.kind == AGX_MEDIUM_HETEROGENEOUS) {
-        float result = 1, t = 0;
-        const float t_max = length(a - b);
-        for (int step = 0; step < MAX_TRACKING_STEPS; ++step) {
-            t += -logf(1 - r.uniform()) * m.misc.z;
-            if (!(t < t_max)) break;
-            const V unit = xf_point(m.w2l, vlerp(a, b, t / t_max));
-            result *= 1 - tex3d(s, m.density, unit).x / m.misc.y;
-        }
-        return mk(result, result, result);
-    }
-    return mk(1, 1, 1);
-}
-
 struct MScat {
     bool happened;
     V pos, wr, thr;
     float g;
 };
 
-// Medium::sample_scattering (homogeneous.cpp:62-110, heterogeneous.cpp:81-123)
-__device__ MScat medium_sample(const DevScene &s, const DevMedium &m, V a, V b, Rng &r, Rng &rtr, bool indirect,
-                               float eps) {
-    MScat o;
-    o.happened = false;
-    o.thr = mk(1, 1, 1);
-    o.g = 0;
-    if (m.kind == AGX_MEDIUM_HOMOGENEOUS) {
-        const float sam = r.uniform();
-        if (black(mk(m.ss))) {
-            const float d = length(a - b);
-            o.thr = mk(expf(-m.st.x * d), expf(-m.st.y * d), expf(-m.st.z * d));
-            return o;
-        }
-        const float t_max = length(b - a);
-        int ch = int(sam * 3.0f);  // extract_uniform_int(u, 0, 3)
-        if (ch > 2) ch = 2;
-        const float nsam = sam * 3.0f - float(ch);
-        const float stc = ch == 0 ? m.st.x : (ch == 1 ? m.st.y : m.st.z);
-        const float stv = -logf(nsam) / stc;
-        const bool in_medium = stv < t_max;
-        const float tt = smin(stv, t_max);
-        const V trv = mk(expf(-m.st.x * tt), expf(-m.st.y * tt), expf(-m.st.z * tt));
-        const V dens = in_medium ? mk(m.st) * trv : trv;
-        float pdf = 0;
-        pdf += dens.x;
-        pdf += dens.y;
-        pdf += dens.z;
-        pdf /= 3;
-        pdf = smax(pdf, eps);
-        V thr = trv / pdf;
-        if (in_medium) thr = thr * mk(m.ss);
-        o.thr = thr;
-        if (in_medium) {
-            o.happened = true;
-            o.pos = vlerp(a, b, stv / t_max);
-            o.wr = (a - b) / t_max;
-            o.g = m.misc.x;
-        }
-        return o;
-    }
-    if (m.kind == AGX_MEDIUM_HETEROGENEOUS) {
-        const float t_max = length(a - b);
-        float t = 0;
-        for (int step = 0; step < MAX_TRACKING_STEPS; ++step) {
-            t += -logf(1 - r.uniform()) * m.misc.z;
-            if (!(t < t_max)) break;
-            const V pos = vlerp(a, b, t / t_max);
-            const V unit = xf_point(m.w2l, pos);
-            const float dn = tex3d(s, m.density, unit).x;
-            if (r.uniform() < dn / m.misc.y) {
-                o.happened = true;
-                o.pos = pos;
-                o.wr = (a - b) / t_max;
-                o.thr = (m.white_for_indirect && indirect) ? mk(1, 1, 1) : tex3d(s, m.albedo, unit);
-                o.g = tex3d(s, m.g3, unit).x;
-                return o;
-            }
-        }
-        return o;
-    }
-    return o;
-}
-
 __device__ __forceinline__ int32_t medium_side(const DevEntity &e, V d, V n) { return dot(d, n) >= 0 ? e.med_out : e.med_in; }
 
 // resolve the MIS-BSDF ray of the previous vertex (direct_illum.cpp:130-192, 194-253;
 // a medium vertex stores |cos| = 1 and pdf = f, so one formula serves both)
+// (k_media has multiplied the record's f by the transmittance of the ray's segment)
 template <uint32_t F>
-__device__ V resolve_mis(const DevScene &s, const PathBuffers &pb, uint32_t p, uint32_t flags, float eps, Rng &rtr) {
+__device__ V resolve_mis(const DevScene &s, const PathBuffers &pb, uint32_t p, uint32_t flags, float eps) {
     const float4 ma = pb.mis_a[p], mb = pb.mis_b[p];
     const V coef = mk(ma), bf = mk(mb);
     const float absdot = ma.w, pdf = mb.w;
@@ -2243,8 +2158,7 @@ __device__ V resolve_mis(const DevScene &s, const PathBuffers &pb, uint32_t p, u
     const Surf sp = surface_at(s, h, o, d, eps);
     const V lrad = dot(sp.geo.z, sp.wr) > 0 ? mk(e.emit) : mk(0, 0, 0);
     if (black(lrad)) return mk(0, 0, 0);
-    const int32_t med = int32_t(flags >> PF_MIS_MED_SHIFT) - 1;
-    const V f = ((F & SF_MEDIA) ? medium_tr(s, med, o, sp.pos, rtr) : mk(1, 1, 1)) * lrad * bf * absdot;
+    const V f = lrad * bf * absdot;
     if (delta) return coef * (f / pdf);
     const float lpdf = area_light_pdf(e, o, sp.pos, sp.geo.z);
     return coef * (f / (pdf + lpdf));
@@ -2356,17 +2270,244 @@ __device__ void guide_inputs_medium(const DevScene &s, V pos, V wr, float *x) {
     x[7] = (atan2f(w.y, w.x) + PI_F) / (2 * PI_F);
 }
 
-// Guided renders in media: the medium segment of each vertex about to be
-// shaded is sampled here, before inference, so that a scattering point gets a
-// network evaluation of its own.  The draws are the ones k_shade would make
-// first at this vertex (Medium::sample_scattering, path_tracing.cpp:64-76);
-// k_shade takes the stored sample instead of drawing again.
-__global__ void __launch_bounds__(256) k_medium_pass(DevScene s, RenderConst rc, PathBuffers pb) {
+// ---------------------------------------------------------------- media pass
+// A record read through the constant address space
+// at a wave-uniform index, so that its words sit in scalar registers instead of
+// vector ones for the length of a tracking loop.
+template <class T> __device__ __forceinline__ T load_uniform(const T *p) {
+    static_assert(sizeof(T) % 4 == 0, "whole words");
+    using Word = const __attribute__((address_space(4))) uint32_t;
+    Word *w = (Word *)(uintptr_t)p;
+    uint32_t buf[sizeof(T) / 4];
+#pragma unroll
+    for (size_t i = 0; i < sizeof(T) / 4; ++i) buf[i] = w[i];
+    T out;
+    __builtin_memcpy(&out, buf, sizeof(T));
+    return out;
+}
+
+// fn(index) for every distinct medium index among the active lanes, the lanes
+// of one index together; each turn retires at least the first active lane's
+template <class Fn> __device__ __forceinline__ void each_medium(int32_t mi, Fn fn) {
+    for (;;) {
+        const int32_t m0 = __builtin_amdgcn_readfirstlane(mi);
+        if (mi == m0) {
+            fn(m0);
+            return;
+        }
+    }
+}
+
+// Two neighbouring texels of an FP16 or FP32 real grid (x0 and x1 of a row) in
+// one load: the pair at min(x0, w - 2) holds both; at the clamped edges x0 == x1
+// and both are the same half of it.
+__device__ __forceinline__ void texel_pair(const DevScene &s, const DevTex3D &t, size_t row, int xb, bool lo0, bool lo1,
+                                           float *a, float *b) {
+    const size_t i = row + size_t(xb);
+    float p, q;
+    if (t.f16) {
+        _Float16 g[2];
+        __builtin_memcpy(g, s.grids16 + i, 4);
+        p = float(g[0]); q = float(g[1]);
+    } else {
+        float g[2];
+        __builtin_memcpy(g, s.grids + i, 8);
+        p = g[0]; q = g[1];
+    }
+    *a = lo0 ? p : q;
+    *b = lo1 ? p : q;
+}
+
+// first channel of tex3d: the same arithmetic, with the trilinear lookup of a
+// real grid at least two texels wide reading its eight texels as four pairs
+__device__ __forceinline__ float tex3d_x(const DevScene &s, const DevTex3D &t, V uvw) {
+    if (t.kind == AGX_TEX3D_CONSTANT || !t.linear || t.ch != 1 || t.w < 2) return tex3d(s, t, uvw).x;
+    const V q = xf_point(t.xf, uvw);
+    const float u = wrap3(t.wrap[0], q.x), v = wrap3(t.wrap[1], q.y), w = wrap3(t.wrap[2], q.z);
+    const float fu = u * float(t.w) - 0.5f, fv = v * float(t.h) - 0.5f, fw = w * float(t.d) - 0.5f;
+    const float bu = floorf(fu), bv = floorf(fv), bw = floorf(fw);
+    const float du = fu - bu, dv = fv - bv, dw = fw - bw;
+    const int x0 = min(t.w - 1, max(0, int(bu))), x1 = min(t.w - 1, max(0, int(bu) + 1));
+    const int y0 = min(t.h - 1, max(0, int(bv))), y1 = min(t.h - 1, max(0, int(bv) + 1));
+    const int z0 = min(t.d - 1, max(0, int(bw))), z1 = min(t.d - 1, max(0, int(bw) + 1));
+    const int xb = min(x0, t.w - 2);
+    const bool lo0 = x0 == xb, lo1 = x1 == xb;
+    auto row = [&](int y, int z) { return t.offset + (size_t(z) * size_t(t.h) + size_t(y)) * size_t(t.w); };
+    float a0, a1, b0, b1, c0, c1, d0, d1;
+    texel_pair(s, t, row(y0, z0), xb, lo0, lo1, &a0, &a1);
+    texel_pair(s, t, row(y1, z0), xb, lo0, lo1, &b0, &b1);
+    texel_pair(s, t, row(y0, z1), xb, lo0, lo1, &c0, &c1);
+    texel_pair(s, t, row(y1, z1), xb, lo0, lo1, &d0, &d1);
+    auto lerp = [](float a, float b, float k) { return a + (b - a) * k; };
+    const float c00 = lerp(a0, a1, du), c10 = lerp(b0, b1, du), c01 = lerp(c0, c1, du), c11 = lerp(d0, d1, du);
+    const float r = lerp(lerp(c00, c10, dv), lerp(c01, c11, dv), dw);
+    return t.inv_gamma != 1.0f ? powf(r, t.inv_gamma) : r;
+}
+
+// Medium::tr (homogeneous.cpp:48-57, heterogeneous.cpp:52-72) from a to b; r = the
+// stream the caller designates.  With `value` false only the stream advances:
+// the number of ratio-tracking draws depends on the segment's length and the
+// majorant alone, not on the densities met.
+__device__ __forceinline__ V medium_tr(const DevScene &s, int32_t mi, V a, V b, Rng &r, bool value) {
+    V out = mk(1, 1, 1);
+    each_medium(mi, [&](int32_t m0) {
+        const DevMedium *mp = s.media + m0;
+        const int32_t kind = load_uniform(&mp->kind);
+        if (kind == AGX_MEDIUM_HOMOGENEOUS) {
+            const vec4 st = load_uniform(&mp->st);
+            const float d = length(a - b);
+            out = mk(expf(-st.x * d), expf(-st.y * d), expf(-st.z * d));
+        } else if (kind == AGX_MEDIUM_HETEROGENEOUS) {
+            const vec4 misc = load_uniform(&mp->misc);
+            const vec4 w2l[3] = {load_uniform(&mp->w2l[0]), load_uniform(&mp->w2l[1]), load_uniform(&mp->w2l[2])};
+            const DevTex3D density = load_uniform(&mp->density);
+            float result = 1, t = 0;
+            const float t_max = length(a - b);
+            for (int step = 0; step < MAX_TRACKING_STEPS; ++step) {
+                t += -logf(1 - r.uniform()) * misc.z;
+                if (!(t < t_max)) break;
+                if (!value) continue;
+                const V unit = xf_point(w2l, vlerp(a, b, t / t_max));
+                result *= 1 - tex3d_x(s, density, unit) / misc.y;
+            }
+            out = mk(result, result, result);
+        }
+    });
+    return out;
+}
+
+// Medium::sample_scattering (homogeneous.cpp:62-110, heterogeneous.cpp:81-123)
+__device__ __forceinline__ MScat medium_sample(const DevScene &s, int32_t mi, V a, V b, Rng &r, bool indirect, float eps) {
+    MScat o;
+    o.happened = false;
+    o.pos = o.wr = mk(0, 0, 0);
+    o.thr = mk(1, 1, 1);
+    o.g = 0;
+    each_medium(mi, [&](int32_t m0) {
+        const DevMedium *mp = s.media + m0;
+        const int32_t kind = load_uniform(&mp->kind);
+        if (kind == AGX_MEDIUM_HOMOGENEOUS) {
+            const vec4 st = load_uniform(&mp->st), ss = load_uniform(&mp->ss), misc = load_uniform(&mp->misc);
+            const float sam = r.uniform();
+            if (black(mk(ss))) {
+                const float d = length(a - b);
+                o.thr = mk(expf(-st.x * d), expf(-st.y * d), expf(-st.z * d));
+                return;
+            }
+            const float t_max = length(b - a);
+            int ch = int(sam * 3.0f);  // extract_uniform_int(u, 0, 3)
+            if (ch > 2) ch = 2;
+            const float nsam = sam * 3.0f - float(ch);
+            const float stc = ch == 0 ? st.x : (ch == 1 ? st.y : st.z);
+            const float stv = -logf(nsam) / stc;
+            const bool in_medium = stv < t_max;
+            const float tt = smin(stv, t_max);
+            const V trv = mk(expf(-st.x * tt), expf(-st.y * tt), expf(-st.z * tt));
+            const V dens = in_medium ? mk(st) * trv : trv;
+            float pdf = 0;
+            pdf += dens.x;
+            pdf += dens.y;
+            pdf += dens.z;
+            pdf /= 3;
+            pdf = smax(pdf, eps);
+            V thr = trv / pdf;
+            if (in_medium) thr = thr * mk(ss);
+            o.thr = thr;
+            if (in_medium) {
+                o.happened = true;
+                o.pos = vlerp(a, b, stv / t_max);
+                o.wr = (a - b) / t_max;
+                o.g = misc.x;
+            }
+        } else if (kind == AGX_MEDIUM_HETEROGENEOUS) {
+            const vec4 misc = load_uniform(&mp->misc);
+            const vec4 w2l[3] = {load_uniform(&mp->w2l[0]), load_uniform(&mp->w2l[1]), load_uniform(&mp->w2l[2])};
+            const DevTex3D density = load_uniform(&mp->density);
+            const float t_max = length(a - b);
+            float t = 0;
+            for (int step = 0; step < MAX_TRACKING_STEPS; ++step) {
+                t += -logf(1 - r.uniform()) * misc.z;
+                if (!(t < t_max)) break;
+                const V pos = vlerp(a, b, t / t_max);
+                const float dn = tex3d_x(s, density, xf_point(w2l, pos));
+                if (r.uniform() < dn / misc.y) {
+                    o.happened = true;
+                    o.pos = pos;
+                    break;
+                }
+            }
+            if (o.happened) {
+                const V unit = xf_point(w2l, o.pos);
+                o.wr = (a - b) / t_max;
+                o.thr = (load_uniform(&mp->white_for_indirect) && indirect) ? mk(1, 1, 1) : tex3d(s, s.media[m0].albedo, unit);
+                o.g = tex3d(s, s.media[m0].g3, unit).x;
+            }
+        }
+    });
+    return o;
+}
+
+// Scenes with media, once per bounce between the traversals and k_shade: all
+// tracking through media, in a kernel of its own.  Tracking is a chain of
+// dependent texel fetches; inside k_shade (199 VGPRs, two waves per SIMD)
+// nothing hid their latency, and the transmittance of every NEE segment was
+// tracked before its shadow ray was known.  Here, per path:
+//   1. the transmittance of the previous vertex's NEE segments, multiplied
+//      into the pending contributions; for an occluded segment the stream
+//      advances without a lookup (not even that when nothing draws from it again);
+//   2. the transmittance of its MIS-BSDF ray, if that met a light, into the record's f;
+//   3. the medium sample of the segment to the vertex about to be shaded
+//      (Medium::sample_scattering, path_tracing.cpp:64-76), or its absorption
+//      once the scattering count is exhausted, stored for k_shade.
+// Draws: 1 and 2 take the transmittance stream, 3 the main one, each in the
+// order of Atrc's estimator as the oracle restates it.
+// Bound by the latency of the dependent fetches (106 VGPRs, 4 waves per SIMD).
+// The door-gap room with a 256^3 grid, 1024x1024 at 4 samples: 168.0 -> 56.0 ms,
+// of which this kernel 9.0 ms and k_shade 12.1 ms (130 ms with the tracking inside it).
+__global__ void __launch_bounds__(256) k_media(DevScene s, RenderConst rc, PathBuffers pb) {
     const uint32_t n = pb.cnt_in[2];
     const uint32_t tid = blockIdx.x * blockDim.x + threadIdx.x;
     if (tid >= n) return;
     const uint32_t p = pb.q_in[tid];
     uint32_t flags = pb.flags[p] & ~PF_MS;
+    const unsigned long long inc = path_inc(rc, p);
+    if (flags & PF_PENDING) {
+        Rng rtr;
+        rtr.state = pb.rng_tr[p];
+        rtr.inc = inc;
+        const bool later = (flags & (PF_CONT | PF_MIS)) != 0;  // draws that follow this vertex's NEE
+        const size_t nb = size_t(p) * rc.L;
+        int32_t last = rc.L;  // lights from here on need no draw
+        if (!later)
+            while (last > 0 && (pb.nee[nb + last - 1].w == 0.0f || pb.occluded[nb + last - 1])) --last;
+        for (int32_t l = 0; l < last; ++l) {
+            const float4 c = pb.nee[nb + l];
+            if (c.w == 0.0f) continue;
+            const float4 a = pb.nee_seg[nb + l];
+            const int32_t mi = __float_as_int(a.w);
+            if (mi < 0) continue;
+            const bool lit = !pb.occluded[nb + l];
+            const V tr = medium_tr(s, mi, mk(a), mk(pb.sh_o[nb + l]), rtr, lit);
+            if (lit) pb.nee[nb + l] = f4(mk(c) * tr, c.w);
+        }
+        const int32_t med = int32_t(flags >> PF_MIS_MED_SHIFT) - 1;
+        if ((flags & PF_MIS) && med >= 0) {
+            const float4 h4 = pb.hit[2 * p + 1];
+            const int32_t ent = __float_as_int(h4.w);
+            if (ent >= 0 && s.ents[ent].light >= 0) {
+                HitRec h;
+                h.t = h4.x; h.u = h4.y; h.v = h4.z; h.ent = ent; h.prim = pb.hit_prim[2 * p + 1];
+                const V o = mk(pb.ray_o[2 * p + 1]);
+                const Surf sp = surface_at(s, h, o, mk(pb.ray_d[2 * p + 1]), rc.eps);
+                if (dot(sp.geo.z, sp.wr) > 0 && !black(mk(s.ents[ent].emit))) {
+                    const V tr = medium_tr(s, med, o, sp.pos, rtr, true);
+                    const float4 mb = pb.mis_b[p];
+                    pb.mis_b[p] = f4(mk(mb) * tr, mb.w);
+                }
+            }
+        }
+        pb.rng_tr[p] = rtr.state;
+    }
     const float4 h4 = pb.hit[2 * p];
     const int32_t ent = __float_as_int(h4.w);
     if ((flags & PF_CONT) && ent >= 0) {
@@ -2375,19 +2516,30 @@ __global__ void __launch_bounds__(256) k_medium_pass(DevScene s, RenderConst rc,
         h.t = h4.x; h.u = h4.y; h.v = h4.z; h.ent = ent; h.prim = pb.hit_prim[2 * p];
         const V ro = mk(pb.ray_o[2 * p]), rd = mk(pb.ray_d[2 * p]);
         const Surf sp = surface_at(s, h, ro, rd, rc.eps);
-        const DevEntity &e = s.ents[ent];
-        const int32_t mi = medium_side(e, sp.wr, sp.geo.z);
-        if (mi >= 0 && dep.z < s.media[mi].max_scat) {
-            Rng rng, rtr;
+        const int32_t mi = medium_side(s.ents[ent], sp.wr, sp.geo.z);
+        if (mi >= 0) {
+            Rng rng;
             rng.state = pb.rng[p];
-            rtr.state = pb.rng_tr[p];
-            rng.inc = rtr.inc = path_inc(rc, p);
-            const MScat ms = medium_sample(s, s.media[mi], ro, sp.pos, rng, rtr, dep.z > 0, rc.eps);
+            rng.inc = inc;
+            MScat ms;
+            if (dep.z < s.media[mi].max_scat) {
+                ms = medium_sample(s, mi, ro, sp.pos, rng, dep.z > 0, rc.eps);
+            } else {  // medium->ab (absorption only) when the scattering count is exhausted
+                ms.happened = false;
+                ms.pos = ms.wr = mk(0, 0, 0);
+                ms.g = 0;
+                if (s.media[mi].kind == AGX_MEDIUM_HOMOGENEOUS) {
+                    const vec4 sa = s.media[mi].sa;
+                    const float d = length(ro - sp.pos);
+                    ms.thr = mk(expf(-sa.x * d), expf(-sa.y * d), expf(-sa.z * d));
+                } else {
+                    ms.thr = medium_tr(s, mi, ro, sp.pos, rng, true);
+                }
+            }
             pb.g_ms[3 * size_t(p)] = f4(ms.pos, ms.g);
             pb.g_ms[3 * size_t(p) + 1] = f4(ms.thr, ms.happened ? 1.0f : 0.0f);
-            pb.g_ms[3 * size_t(p) + 2] = f4(ms.wr, 0.0f);
+            if (ms.happened) pb.g_ms[3 * size_t(p) + 2] = f4(ms.wr, 0.0f);
             pb.rng[p] = rng.state;
-            pb.rng_tr[p] = rtr.state;
             flags |= PF_MS;
         }
     }
@@ -2403,7 +2555,7 @@ __global__ void __launch_bounds__(256) k_guide_features(DevScene s, RenderConst 
     const float4 h4 = pb.hit[2 * p];
     const int32_t ent = __float_as_int(h4.w);
     const uint32_t flags = pb.flags[p];
-    if ((flags & PF_MS) && pb.g_ms[3 * size_t(p) + 1].w != 0.0f) {
+    if (rc.guide_media && (flags & PF_MS) && pb.g_ms[3 * size_t(p) + 1].w != 0.0f) {
         guide_inputs_medium(s, mk(pb.g_ms[3 * size_t(p)]), mk(pb.g_ms[3 * size_t(p) + 2]), x);
     } else if ((flags & PF_CONT) && ent >= 0) {
         HitRec h;
@@ -2428,16 +2580,12 @@ __global__ void __launch_bounds__(256) k_shade(DevScene s, RenderConst rc, PathB
     const bool fresh = (flags & PF_FRESH) != 0;
     flags &= ~PF_FRESH;
     V L = fresh ? mk(0, 0, 0) : mk(pb.radiance[p]);
-    // the transmittance stream is drawn only in media: vacuum variants neither
-    // load nor store it
-    Rng rtr;
     const bool media = (F & SF_MEDIA) && (s.features & SF_MEDIA);
-    rtr.state = media ? pb.rng_tr[p] : 0ull;
     Rng rng;
     rng.state = pb.rng[p];
-    rng.inc = rtr.inc = path_inc(rc, p);
-    // the medium sample k_medium_pass took for this vertex (guided renders in media)
-    const bool ms_done = (F & SF_GUIDE) && (F & SF_MEDIA) && (flags & PF_MS);
+    rng.inc = path_inc(rc, p);
+    // k_media has sampled the medium segment before this vertex
+    const bool ms_done = media && (flags & PF_MS);
     flags &= ~PF_MS;
     // 1. direct illumination of the previous vertex (path_tracing.cpp:85-97, 134-146)
     if (flags & PF_PENDING) {
@@ -2457,7 +2605,7 @@ __global__ void __launch_bounds__(256) k_shade(DevScene s, RenderConst rc, PathB
             const float4 c = pb.nee[nb + l];
             if (c.w != 0.0f && !pb.occluded[nb + l]) direct = direct + mk(c);
         }
-        if (flags & PF_MIS) direct = direct + resolve_mis<F>(s, pb, p, flags, eps, rtr);
+        if (flags & PF_MIS) direct = direct + resolve_mis<F>(s, pb, p, flags, eps);
         L = L + direct;
         if ((F & SF_GUIDE) && rc.guide_record && guide_recording(rc, p) && !black(direct)) {
             // light reaching the previous vertex arrives at every earlier recorded
@@ -2478,7 +2626,6 @@ __global__ void __launch_bounds__(256) k_shade(DevScene s, RenderConst rc, PathB
     if (!(flags & PF_CONT)) {
         pb.radiance[p] = f4(L, 0);
         pb.flags[p] = flags;
-        if (media) pb.rng_tr[p] = rtr.state;
         return;
     }
     flags &= ~PF_CONT;
@@ -2506,7 +2653,6 @@ __global__ void __launch_bounds__(256) k_shade(DevScene s, RenderConst rc, PathB
         }
         pb.radiance[p] = f4(L, 0);
         pb.flags[p] = flags;
-        if (media) pb.rng_tr[p] = rtr.state;
         return;
     }
     HitRec h;
@@ -2522,125 +2668,112 @@ __global__ void __launch_bounds__(256) k_shade(DevScene s, RenderConst rc, PathB
     bool cont = false;
     bool push_mis = false;
     uint32_t shadow_mask = 0;  // bit l: the shadow ray of light l is traced
-    // medium between the ray origin and the hit (path_tracing.cpp:64-119)
-    const int32_t mi = (F & SF_MEDIA) ? medium_side(e, sp.wr, sp.geo.z) : -1;
+    // medium between the ray origin and the hit (path_tracing.cpp:64-119), sampled by k_media:
+    // a scattering point, or the throughput of the segment
+    const int32_t mi = media ? medium_side(e, sp.wr, sp.geo.z) : -1;
     bool scattered = false;
-    if ((F & SF_MEDIA) && mi >= 0) {
-        const DevMedium &m = s.media[mi];
-        if (dep.z < m.max_scat) {
-            MScat ms;
-            if (ms_done) {
-                const float4 a = pb.g_ms[3 * size_t(p)], b4 = pb.g_ms[3 * size_t(p) + 1], c4 = pb.g_ms[3 * size_t(p) + 2];
-                ms.pos = mk(a); ms.g = a.w; ms.thr = mk(b4); ms.happened = b4.w != 0.0f; ms.wr = mk(c4);
-            } else {
-                ms = medium_sample(s, m, ro, sp.pos, rng, rtr, dep.z > 0, eps);
+    if ((F & SF_MEDIA) && ms_done) {
+        const float4 ma = pb.g_ms[3 * size_t(p)], mb = pb.g_ms[3 * size_t(p) + 1], mc = pb.g_ms[3 * size_t(p) + 2];
+        MScat ms;
+        ms.pos = mk(ma); ms.g = ma.w; ms.thr = mk(mb); ms.happened = mb.w != 0.0f; ms.wr = mk(mc);
+        coef = coef * ms.thr;
+        if (ms.happened) {
+            scattered = true;
+            dep.z += 1;
+            // NEE at the medium point: area lights only; the environment draws nothing
+            // (trace_nomis samples no light)
+            for (int32_t l = 0; l < (rc.nomis ? 0 : rc.L); ++l) {
+                const size_t slot = size_t(p) * rc.L + l;
+                const int32_t li = s.lights[l];
+                pb.nee[slot] = make_float4(0, 0, 0, 0);
+                if (li < 0) continue;
+                float s5[5];
+                for (int k = 0; k < 5; ++k) s5[k] = rng.uniform();
+                const DevEntity &le = s.ents[li];
+                const LightSmp ls = area_light_sample(s, le, ms.pos, s5[0], s5[1], s5[3], eps);
+                const V rad = mk(le.emit);
+                if (black(rad) || ls.pdf == 0.0f) continue;
+                const V tl = normalize(ls.pos - ms.pos);
+                const float fp = hg_eval(ms.g, tl, ms.wr);
+                if (fp == 0.0f) continue;
+                const V f = rad * mk(fp, fp, fp);
+                pb.nee[slot] = f4(coef * (f / (ls.pdf + fp)), 1.0f);
+                pb.nee_seg[slot] = f4(ms.pos, __int_as_float(mi));
+                pending = true;
+                // Scene::visible(light, point): from the light towards the point
+                const float dis = length(ls.pos - ms.pos);
+                put_shadow(pb, slot, ls.pos, normalize(ms.pos - ls.pos), eps, dis - eps);
+                shadow_mask |= 1u << l;
             }
-            coef = coef * ms.thr;
-            if (ms.happened) {
-                scattered = true;
-                dep.z += 1;
-                // NEE at the medium point: area lights only; the environment draws nothing
-                // (trace_nomis samples no light)
-                for (int32_t l = 0; l < (rc.nomis ? 0 : rc.L); ++l) {
-                    const size_t slot = size_t(p) * rc.L + l;
-                    const int32_t li = s.lights[l];
-                    pb.nee[slot] = make_float4(0, 0, 0, 0);
-                    if (li < 0) continue;
-                    float s5[5];
-                    for (int k = 0; k < 5; ++k) s5[k] = rng.uniform();
-                    const DevEntity &le = s.ents[li];
-                    const LightSmp ls = area_light_sample(s, le, ms.pos, s5[0], s5[1], s5[3], eps);
-                    const V rad = mk(le.emit);
-                    if (black(rad) || ls.pdf == 0.0f) continue;
-                    const V tl = normalize(ls.pos - ms.pos);
-                    const float fp = hg_eval(ms.g, tl, ms.wr);
-                    if (fp == 0.0f) continue;
-                    const V f = medium_tr(s, mi, ms.pos, ls.pos, rtr) * rad * mk(fp, fp, fp);
-                    pb.nee[slot] = f4(coef * (f / (ls.pdf + fp)), 1.0f);
+            if (!rc.nomis) {  // MIS-BSDF ray with the phase function (direct_illum.cpp:194-253)
+                const float u0 = rng.uniform(), u1 = rng.uniform();
+                (void)rng.uniform();
+                V dir;
+                float f;
+                hg_sample(ms.g, ms.wr, u0, u1, &dir, &f);
+                if (f != 0.0f) {
+                    dir = normalize(dir);
+                    pb.ray_o[2 * p + 1] = f4(ms.pos, 0.0f);
+                    pb.ray_d[2 * p + 1] = f4(dir, INF_F);
+                    pb.mis_a[p] = f4(coef, 1.0f);
+                    pb.mis_b[p] = make_float4(f, f, f, f);
+                    flags |= PF_MIS | (uint32_t(mi + 1) << PF_MIS_MED_SHIFT);
                     pending = true;
-                    // Scene::visible(light, point): from the light towards the point
-                    const float dis = length(ls.pos - ms.pos);
-                    put_shadow(pb, slot, ls.pos, normalize(ms.pos - ls.pos), eps, dis - eps);
-                    shadow_mask |= 1u << l;
-                }
-                if (!rc.nomis) {  // MIS-BSDF ray with the phase function (direct_illum.cpp:194-253)
-                    const float u0 = rng.uniform(), u1 = rng.uniform();
-                    (void)rng.uniform();
-                    V dir;
-                    float f;
-                    hg_sample(ms.g, ms.wr, u0, u1, &dir, &f);
-                    if (f != 0.0f) {
-                        dir = normalize(dir);
-                        pb.ray_o[2 * p + 1] = f4(ms.pos, 0.0f);
-                        pb.ray_d[2 * p + 1] = f4(dir, INF_F);
-                        pb.mis_a[p] = f4(coef, 1.0f);
-                        pb.mis_b[p] = make_float4(f, f, f, f);
-                        flags |= PF_MIS | (uint32_t(mi + 1) << PF_MIS_MED_SHIFT);
-                        pending = true;
-                        push_mis = true;
-                    }
-                }
-                if ((F & SF_GUIDE) && rc.guide && dep.x <= rc.guide_medium_depth) {
-                    // guided: one-sample mixture of the learned density (probability
-                    // alpha) and the phase function, weighted by the mixture density
-                    const float usel = rng.uniform();
-                    const float u0 = rng.uniform(), u1 = rng.uniform(), u2 = rng.uniform();
-                    const float *G = pb.g_out + size_t(tid) * GUIDE_ROW;
-                    const float a = rc.guide_alpha;
-                    V dir;
-                    float fp;
-                    if (usel < a) {
-                        dir = guide_sample(G, u0, u1, u2);
-                        fp = hg_eval(ms.g, dir, ms.wr);
-                    } else {
-                        hg_sample(ms.g, ms.wr, u0, u1, &dir, &fp);
-                        dir = normalize(dir);
-                    }
-                    const float pdf = a * guide_pdf(G, dir) + (1 - a) * fp;  // the phase function's pdf is its value
-                    if (fp != 0.0f && !(pdf < eps) && isfinite(pdf)) {
-                        pb.ray_o[2 * p] = f4(ms.pos, 0.0f);
-                        pb.ray_d[2 * p] = f4(dir, INF_F);
-                        coef = coef * (fp / pdf);
-                        dep.x += 1;
-                        if (dep.x <= rc.max_depth) {
-                            cont = true;
-                            if (dep.x > rc.min_depth) {
-                                if (rng.uniform() > rc.cont_prob) cont = false;
-                                else coef = coef / rc.cont_prob;
-                            }
-                        }
-                        if (cont && rc.guide_record && guide_recording(rc, p))
-                            guide_record(pb, rc, p, tid, dir, pdf, coef, fp);
-                    }
-                } else {  // phase-function continuation (path_tracing.cpp:99-108; trace_nomis :285-296
-                   // samples around the surface hit's wr, tests only f and keeps the direction as sampled)
-                    const float u0 = rng.uniform(), u1 = rng.uniform();
-                    (void)rng.uniform();
-                    V dir;
-                    float f;
-                    hg_sample(ms.g, rc.nomis ? sp.wr : ms.wr, u0, u1, &dir, &f);
-                    if (f != 0.0f && (rc.nomis || !(f < eps))) {
-                        pb.ray_o[2 * p] = f4(ms.pos, 0.0f);
-                        pb.ray_d[2 * p] = f4(rc.nomis ? dir : normalize(dir), INF_F);
-                        coef = coef * (mk(f, f, f) / f);
-                        dep.x += 1;
-                        if (dep.x <= rc.max_depth) {
-                            cont = true;
-                            if (dep.x > rc.min_depth) {
-                                if (rng.uniform() > rc.cont_prob) cont = false;
-                                else coef = coef / rc.cont_prob;
-                            }
-                        }
-                    }
+                    push_mis = true;
                 }
             }
-        } else {
-            // medium->ab (absorption only) when the scattering count is exhausted
-            if (m.kind == AGX_MEDIUM_HOMOGENEOUS) {
-                const float d = length(ro - sp.pos);
-                coef = coef * mk(expf(-m.sa.x * d), expf(-m.sa.y * d), expf(-m.sa.z * d));
-            } else {
-                coef = coef * medium_tr(s, mi, ro, sp.pos, rng);
+            if ((F & SF_GUIDE) && rc.guide && dep.x <= rc.guide_medium_depth) {
+                // guided: one-sample mixture of the learned density (probability
+                // alpha) and the phase function, weighted by the mixture density
+                const float usel = rng.uniform();
+                const float u0 = rng.uniform(), u1 = rng.uniform(), u2 = rng.uniform();
+                const float *G = pb.g_out + size_t(tid) * GUIDE_ROW;
+                const float a = rc.guide_alpha;
+                V dir;
+                float fp;
+                if (usel < a) {
+                    dir = guide_sample(G, u0, u1, u2);
+                    fp = hg_eval(ms.g, dir, ms.wr);
+                } else {
+                    hg_sample(ms.g, ms.wr, u0, u1, &dir, &fp);
+                    dir = normalize(dir);
+                }
+                const float pdf = a * guide_pdf(G, dir) + (1 - a) * fp;  // the phase function's pdf is its value
+                if (fp != 0.0f && !(pdf < eps) && isfinite(pdf)) {
+                    pb.ray_o[2 * p] = f4(ms.pos, 0.0f);
+                    pb.ray_d[2 * p] = f4(dir, INF_F);
+                    coef = coef * (fp / pdf);
+                    dep.x += 1;
+                    if (dep.x <= rc.max_depth) {
+                        cont = true;
+                        if (dep.x > rc.min_depth) {
+                            if (rng.uniform() > rc.cont_prob) cont = false;
+                            else coef = coef / rc.cont_prob;
+                        }
+                    }
+                    if (cont && rc.guide_record && guide_recording(rc, p))
+                        guide_record(pb, rc, p, tid, dir, pdf, coef, fp);
+                }
+            } else {  // phase-function continuation (path_tracing.cpp:99-108; trace_nomis :285-296
+               // samples around the surface hit's wr, tests only f and keeps the direction as sampled)
+                const float u0 = rng.uniform(), u1 = rng.uniform();
+                (void)rng.uniform();
+                V dir;
+                float f;
+                hg_sample(ms.g, rc.nomis ? sp.wr : ms.wr, u0, u1, &dir, &f);
+                if (f != 0.0f && (rc.nomis || !(f < eps))) {
+                    pb.ray_o[2 * p] = f4(ms.pos, 0.0f);
+                    pb.ray_d[2 * p] = f4(rc.nomis ? dir : normalize(dir), INF_F);
+                    coef = coef * (mk(f, f, f) / f);
+                    dep.x += 1;
+                    if (dep.x <= rc.max_depth) {
+                        cont = true;
+                        if (dep.x > rc.min_depth) {
+                            if (rng.uniform() > rc.cont_prob) cont = false;
+                            else coef = coef / rc.cont_prob;
+                        }
+                    }
+                }
             }
         }
     }
@@ -2668,9 +2801,8 @@ __global__ void __launch_bounds__(256) k_shade(DevScene s, RenderConst rc, PathB
                         const V tl = normalize(ls.pos - sp.pos);
                         const V f = bsdf_eval<F>(b, tl, sp.wr);
                         if (!black(f)) {
-                            const V trv = (F & SF_MEDIA) ? medium_tr(s, medium_side(e, tl, sp.geo.z), ls.pos, sp.pos, rtr)
-                                                         : mk(1, 1, 1);
-                            const V ff = trv * rad * f * fabsf(cosv(tl, sp.geo.z));
+                            const V ff = rad * f * fabsf(cosv(tl, sp.geo.z));
+                            if (media) pb.nee_seg[slot] = f4(ls.pos, __int_as_float(medium_side(e, tl, sp.geo.z)));
                             const float bp = bsdf_pdf<F>(b, tl, sp.wr);
                             contrib = coef * (ff / (ls.pdf + bp));
                             valid = true;
@@ -2691,6 +2823,7 @@ __global__ void __launch_bounds__(256) k_shade(DevScene s, RenderConst rc, PathB
                         const float bp = bsdf_pdf<F>(b, tl, sp.wr);
                         contrib = coef * (ff / (epdf + bp));
                         valid = true;
+                        if (media) pb.nee_seg[slot] = make_float4(0, 0, 0, __int_as_float(-1));  // no transmittance
                         // Scene::visible(A, B): [eps, |A-B| - eps] along normalize(B - A)
                         so = sp.pos; sd = normalize(lpos - sp.pos); tmax = length(sp.pos - lpos) - eps;
                     }
@@ -2787,7 +2920,6 @@ __global__ void __launch_bounds__(256) k_shade(DevScene s, RenderConst rc, PathB
     pb.depth[p] = dep;
     pb.flags[p] = flags;
     pb.rng[p] = rng.state;
-    if (media) pb.rng_tr[p] = rtr.state;
 }
 
 // ---------------------------------------------------------------- queue compaction
@@ -3292,10 +3424,9 @@ void launch_queue_compact(const PathBuffers &pb, uint32_t max_n, int L, uint4 *b
     if (nb) hipLaunchKernelGGL(k_queue_scatter, dim3(nb), dim3(QC_THREADS), 0, st, pb, nl, blk);
 }
 
-void launch_medium_pass(const DevScene &s, const RenderConst &rc, const PathBuffers &pb, uint32_t max_n,
-                        hipStream_t st) {
+void launch_media(const DevScene &s, const RenderConst &rc, const PathBuffers &pb, uint32_t max_n, hipStream_t st) {
     if (!max_n) return;
-    hipLaunchKernelGGL(k_medium_pass, dim3(grid_of(max_n, 256)), dim3(256), 0, st, s, rc, pb);
+    hipLaunchKernelGGL(k_media, dim3(grid_of(max_n, 256)), dim3(256), 0, st, s, rc, pb);
 }
 
 void launch_guide_features(const DevScene &s, const RenderConst &rc, const PathBuffers &pb, uint32_t max_n,
