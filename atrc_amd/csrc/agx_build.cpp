@@ -869,6 +869,11 @@ int build_host_scene(const agx_scene_desc &desc, HostScene *out, std::string *er
                 o[0] = S.blas_prims[3 * size_t(slot)];
                 o[1] = S.blas_prims[3 * size_t(slot) + 1];
                 o[2] = S.blas_prims[3 * size_t(slot) + 2];
+            } else if (S.ents[ref_ent[r]].kind == AGX_GEOM_QUAD && !watertight) {
+                const DevEntity &q = S.ents[ref_ent[r]];
+                o[0] = q.a;
+                o[1] = q.b_a;
+                o[2] = q.c_a;
             } else {
                 o[0] = o[1] = o[2] = vec4{0, 0, 0, 0};
             }

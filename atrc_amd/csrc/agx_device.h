@@ -35,7 +35,8 @@ constexpr int MAX_LIGHTS = 16;
 // BVH4_LEAF | (count - 1) << 27 | first primitive.  A primitive is 3 vec4:
 //   (A, entity), (B - A, slot), (C - A, tie rank); slot = index into
 //   blas_prims/blas_info of a mesh triangle, or BVH4_ANALYTIC for a whole
-//   analytic entity; tie rank = DevEntity::tie_rank of the entity.  In the
+//   analytic entity (a quad's record holds its A, B - A, C - A, the others zeros);
+//   tie rank = DevEntity::tie_rank of the entity.  In the
 //   watertight mode a mesh triangle is (A, entity), (B, slot), (C, tie rank)
 //   with the mesh's own vertex coordinates, and a quad is two primitives
 //   (A, entity), (B, BVH4_QUAD_ABC), (C, rank) and (A, entity), (C, BVH4_QUAD_ACD), (D, rank).

@@ -692,6 +692,16 @@ __device__ __forceinline__ E ring_pop(E *col, const E *spill, int &sp) {
 static_assert((BVH4_RING_CLOSEST & (BVH4_RING_CLOSEST - 1)) == 0 && (BVH4_RING_ANY & (BVH4_RING_ANY - 1)) == 0,
               "ring sizes are powers of two");
 
+// A quad's record carries its first triangle (A, B - A, C - A), so that quads
+// take the lanes' common triangle test instead of the entity switch: walls are
+// what most rays of a room test, and a wave ran the node, triangle and entity
+// code one after another for its lanes.  The other analytic records hold zeros
+// there, and so does a quad whose B - A is zero: those go through the entity.
+__device__ __forceinline__ bool b4_inline_quad(float4 p1) {
+    return __float_as_uint(p1.w) == BVH4_ANALYTIC &&
+           (__float_as_uint(p1.x) | __float_as_uint(p1.y) | __float_as_uint(p1.z)) != 0;
+}
+
 // Closest hit over the BVH4: children visited near-first, pending children
 // kept with their entry distance and skipped once a closer hit is known.
 // ring = this lane's column of a [BVH4_RING_CLOSEST][TB] LDS array.  The state
@@ -769,19 +779,37 @@ struct B4Closest {
                 const float4 p0 = P[3 * size_t(i)], p1 = P[3 * size_t(i) + 1], p2 = P[3 * size_t(i) + 2];
                 const int32_t ent = __float_as_int(p0.w);
                 const uint32_t slot = __float_as_uint(p1.w);
-                if (slot < BVH4_QUAD_ACD || (WT && slot != BVH4_ANALYTIC)) {
-                    // a mesh triangle, or (watertight mode) one triangle of a quad
+                const bool quad = !WT && b4_inline_quad(p1);
+                if (slot < BVH4_QUAD_ACD || (WT && slot != BVH4_ANALYTIC) || quad) {
+                    // a mesh triangle, a quad (its first triangle, then its second), or
+                    // (watertight mode) one triangle of a quad
                     if (STATS) c.tests++;
+                    const int32_t rank = __float_as_int(p2.w);
+                    int32_t prim = (WT && slot >= BVH4_QUAD_ACD) ? (slot == BVH4_QUAD_ABC ? 0 : 1) : int32_t(slot);
                     float tt, uu, vv;
-                    const bool hit_tri = WT ? wt_test(wr, mk(p0), mk(p1), mk(p2), tmin, tmax, &tt, &uu, &vv)
-                                            : mt_closest(r.o, d, tmin, tmax, mk(p0), mk(p1), mk(p2), &tt, &uu, &vv);
+                    bool hit_tri;
+                    if (WT) {
+                        hit_tri = wt_test(wr, mk(p0), mk(p1), mk(p2), tmin, tmax, &tt, &uu, &vv);
+                    } else {
+                        // a quad of a lower-ranked entity must hit strictly closer: its tests run
+                        // against the next float below the current hit distance
+                        const float lim = quad && rank < best_rank ? __uint_as_float(__float_as_uint(tmax) - 1u) : tmax;
+                        hit_tri = mt_closest(r.o, d, tmin, lim, mk(p0), mk(p1), mk(p2), &tt, &uu, &vv);
+                        if (quad) {
+                            prim = 0;
+                            if (!hit_tri) {
+                                if (STATS) c.tests++;
+                                hit_tri = mt_closest(r.o, d, tmin, lim, mk(p0), mk(p2), mk(s.ents[ent].d_a), &tt, &uu, &vv);
+                                prim = 1;
+                            }
+                        }
+                    }
                     // an exact tie with another entity's hit goes to the entity that
                     // Atrc's aggregate tests later (its tie rank)
-                    const int32_t rank = __float_as_int(p2.w);
                     if (hit_tri && (tt < tmax || ent == rec.ent || rank > best_rank)) {
                         tmax = tt;
                         rec.t = tt; rec.u = uu; rec.v = vv; rec.ent = ent;
-                        rec.prim = (WT && slot >= BVH4_QUAD_ACD) ? (slot == BVH4_QUAD_ABC ? 0 : 1) : int32_t(slot);
+                        rec.prim = prim;
                         best_rank = rank;
                     }
                 } else {
@@ -877,7 +905,8 @@ struct B4Any {
                 // leave it unused; triangles need it)
                 const float4 p0 = P[3 * size_t(i)], p1 = P[3 * size_t(i) + 1], p2 = P[3 * size_t(i) + 2];
                 const uint32_t slot = __float_as_uint(p1.w);
-                if (slot < BVH4_QUAD_ACD || (WT && slot != BVH4_ANALYTIC)) {
+                const bool quad = !WT && b4_inline_quad(p1);
+                if (slot < BVH4_QUAD_ACD || (WT && slot != BVH4_ANALYTIC) || quad) {
                     if (STATS) c.tests++;
                     if (WT) {
                         float tt, uu, vv;
@@ -885,6 +914,12 @@ struct B4Any {
                     } else if (mt_any(r.o, d, tmin, tmax, mk(p0), mk(p1), mk(p2))) {
                         occluded = true;
                         return true;
+                    } else if (quad) {
+                        if (STATS) c.tests++;
+                        if (mt_any(r.o, d, tmin, tmax, mk(p0), mk(p2), mk(s.ents[__float_as_int(p0.w)].d_a))) {
+                            occluded = true;
+                            return true;
+                        }
                     }
                 } else if (analytic_any<STATS>(s.ents[__float_as_int(p0.w)], r.o, d, tmin, tmax, c)) {
                     occluded = true;
