@@ -659,20 +659,8 @@ int agx_render(agx_ctx *c, const agx_render_params *p, const volatile int32_t *c
         HIP_TRY(hipEventRecord(e, c->stream));
         return AGX_OK;
     };
-    // Queue sizes are read back asynchronously into a pinned ring; the host
-    // checks termination two bounces behind, so the GPU never idles waiting.
-    struct Readback { size_t ev; int slot; };
-    std::vector<Readback> reads;
-    int ring_next = 0;
-    auto readback = [&](const uint32_t *dev) -> int {
-        const int slot = ring_next++ % agx_ctx::RING;
-        HIP_TRY(hipMemcpyAsync(c->h_counters + 4 * slot, dev, 4 * sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream));
-        size_t e;
-        if (int rr = mark(&e)) return rr;
-        reads.push_back({e, slot});
-        return AGX_OK;
-    };
-    const uint32_t n_closest_max = uint32_t(2 * per_pass), n_shadow_max = uint32_t(per_pass * std::max(rc.L, 1));
+    // Every bounce's queue sizes are written into a slot of a pinned ring by the kernel that
+    // makes the queues; the host reads a slot after the event that follows it.
     const int max_bounces = p->max_depth + std::max(p->specular_depth, 0) + 2;
     if (max_bounces + 1 > agx_ctx::RING)
         return fail(AGX_E_UNSUPPORTED, "max_depth + specular_depth too large (at most " +
@@ -689,58 +677,76 @@ int agx_render(agx_ctx *c, const agx_render_params *p, const volatile int32_t *c
         launch_reset_counters(cout, c->stream);
         c->pb.cnt_out = cout;
         launch_raygen(c->ds, rc, c->pb, c->stream);
+        // raygen queues every camera path, or (roulette at depth 1) those it counts
+        const bool all_queued = rc.min_depth >= 1 && rc.max_depth >= 1;
+        if (!all_queued) {
+            HIP_TRY(hipMemcpyAsync(c->h_counters, cout, 4 * sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream));
+        } else {
+            c->h_counters[0] = c->h_counters[2] = uint32_t(rc.n_paths);
+            c->h_counters[1] = c->h_counters[3] = 0;
+        }
         if ((r = mark(&b))) return r;
         timed.push_back({a, b, 2});
-        if ((r = readback(cout))) return r;
         st.paths += uint64_t(rc.n_paths);
-        const size_t first_read = reads.size() - 1;
+        // done[k] = the event after which slot k of the pinned ring holds the queue
+        // sizes that bounce k consumes (and the start of bounce k)
+        std::vector<size_t> done(1, b);
+        uint32_t alive = uint32_t(rc.n_paths);  // at least the paths that the coming bounce shades
+        int bounces = 0;
         std::swap(cin, cout);
         std::swap(c->pb.q_in, c->pb.q_out);
         for (int bounce = 0; bounce < max_bounces; ++bounce) {
             c->pb.cnt_in = cin;
             c->pb.cnt_out = cout;
-            size_t e0, e1, e2, e3;
-            if ((r = mark(&e0))) return r;
-            launch_trace_closest(c->ds, c->pb, n_closest_max, stats, c->dcnt, c->stream);
+            // grids for the paths known to be left, not for the pass's capacity: blocks
+            // without work cost about a microsecond a thousand, 0.1 ms a launch of
+            // 33 million paths.  Camera paths have no MIS or shadow rays yet.
+            const uint32_t n_closest = bounce == 0 ? alive : 2 * alive;
+            const uint32_t n_shadow = bounce == 0 ? 0 : alive * uint32_t(std::max(rc.L, 0));
+            size_t e0 = done.back(), e1, e2, e3;
+            launch_trace_closest(c->ds, c->pb, n_closest, stats, c->dcnt, c->stream);
             if ((r = mark(&e1))) return r;
             if (c->capture_count) {
                 launch_capture_rays(c->pb, 0, c->capture_o[0], c->capture_d[0], c->capture_count, c->capture_cap,
-                                    n_closest_max, c->stream);
+                                    n_closest, c->stream);
                 launch_capture_rays(c->pb, 1, c->capture_o[1], c->capture_d[1], c->capture_count + 1,
-                                    c->capture_cap, n_shadow_max, c->stream);
+                                    c->capture_cap, n_shadow, c->stream);
             }
-            launch_trace_shadow(c->ds, c->pb, n_shadow_max, stats, c->dcnt + 1, c->stream);
-            if ((r = mark(&e2))) return r;
             timed.push_back({e0, e1, 0});
-            timed.push_back({e1, e2, 1});
-            if (media) launch_media(c->ds, rc, c->pb, uint32_t(rc.n_paths), c->stream);
+            e2 = e1;
+            st.trace_closest_launches += 1;
+            if (n_shadow) {
+                launch_trace_shadow(c->ds, c->pb, n_shadow, stats, c->dcnt + 1, c->stream);
+                if ((r = mark(&e2))) return r;
+                timed.push_back({e1, e2, 1});
+                st.trace_shadow_launches += 1;
+            }
+            if (media) launch_media(c->ds, rc, c->pb, alive, c->stream);
             if (guide) {
                 // the network's mixture for every vertex about to be shaded (in media,
                 // at the scattering point the vertex's medium sample reaches)
-                launch_guide_features(c->ds, rc, c->pb, uint32_t(rc.n_paths), c->stream);
+                launch_guide_features(c->ds, rc, c->pb, alive, c->stream);
                 size_t ef, eg;
                 if ((r = mark(&ef))) return r;
-                launch_guide_infer(c->g_packed, c->g_bias, c->pb.g_feat, c->pb.g_out, cin + 2, uint32_t(rc.n_paths),
-                                   c->stream);
+                launch_guide_infer(c->g_packed, c->g_bias, c->pb.g_feat, c->pb.g_out, cin + 2, alive, c->stream);
                 if ((r = mark(&eg))) return r;
                 timed.push_back({e2, ef, 2});
                 timed.push_back({ef, eg, 3});
                 e2 = eg;
             }
-            launch_reset_counters(cout, c->stream);
-            launch_shade(c->ds, rc, c->pb, uint32_t(rc.n_paths), c->stream);
-            launch_queue_compact(c->pb, uint32_t(rc.n_paths), rc.L, c->qc_blk, c->stream);
+            launch_shade(c->ds, rc, c->pb, alive, c->stream);
+            launch_queue_compact(c->pb, alive, rc.L, c->qc_blk, c->h_counters + 4 * (bounce + 1), c->stream);
             if ((r = mark(&e3))) return r;
             timed.push_back({e2, e3, 2});
-            if ((r = readback(cout))) return r;
+            done.push_back(e3);
+            bounces = bounce + 1;
             std::swap(cin, cout);
             std::swap(c->pb.q_in, c->pb.q_out);
-            // the queue produced two bounces ago: if it was empty, everything since is a no-op
-            if (bounce >= 1) {
-                const Readback &rb = reads[first_read + size_t(bounce)];
-                HIP_TRY(hipEventSynchronize(c->pool[rb.ev]));
-                if (c->h_counters[4 * rb.slot + 2] == 0) break;
-            }
+            // what this bounce consumes is known by now (the bounce before it wrote it), so
+            // the GPU, busy with this bounce, does not wait for the host
+            HIP_TRY(hipEventSynchronize(c->pool[done[size_t(bounce)]]));
+            alive = std::min(alive, c->h_counters[4 * bounce + 2]);
+            if (alive == 0) break;  // this bounce was a no-op, and so would be the rest
             if (cancel_flag && *cancel_flag) { cancelled = true; break; }
         }
         if (cancelled) break;
@@ -779,18 +785,13 @@ int agx_render(agx_ctx *c, const agx_render_params *p, const volatile int32_t *c
             st.guide_samples += std::min<uint32_t>(guide_samples_h, guide_batch);
             st.guide_trained += uint64_t(guide_valid_h) * uint64_t(guide_steps);
         }
-        // sum the ray queue sizes of this pass (every read has completed)
-        for (size_t k = first_read; k < reads.size(); ++k) {
-            const uint32_t *q = c->h_counters + 4 * reads[k].slot;
+        // sum the ray queue sizes of this pass
+        for (int k = 0; k <= bounces; ++k) {
+            const uint32_t *q = c->h_counters + 4 * k;
             st.closest_rays += q[0];
             st.shadow_rays += q[1];
-            if (guide && k + 1 < reads.size()) st.guide_rows += q[2];  // shaded by the next bounce
+            if (guide && k < bounces) st.guide_rows += q[2];
         }
-        // every bounce launched both traversal kernels (an empty queue exits at once)
-        st.trace_closest_launches += uint64_t(reads.size() - first_read - 1);
-        st.trace_shadow_launches += uint64_t(reads.size() - first_read - 1);
-        reads.resize(first_read);
-        ring_next = 0;
         if (cancel_flag && *cancel_flag) cancelled = true;
     }
     HIP_TRY(hipEventRecord(c->ev[1], c->stream));
@@ -1089,7 +1090,7 @@ int enqueue_render(agx_ctx *c, const agx_render_params *p, hipStream_t st, unsig
          (size_t(per_pass) > c->media_cap || size_t(per_pass) * size_t(std::max(rc.L, 1)) > c->media_nee_cap)))
         return fail(AGX_E_INVALID_ARG, "graph batch: render buffers not prepared");
     rc.guide_rec_shift = guide_rec_shift(size_t(per_pass));
-    const uint32_t n_closest_max = uint32_t(2 * per_pass), n_shadow_max = uint32_t(per_pass * std::max(rc.L, 1));
+    const uint32_t n_closest_max = uint32_t(2 * per_pass), n_shadow_max = uint32_t(per_pass * std::max(rc.L, 0));
     // without delta surfaces no bounce extends the depth (path_tracing.cpp:155-162),
     // so the specular allowance adds only empty launches
     const int spec = (c->ds.features & SF_DELTA) ? std::max(p->specular_depth, 0) : 0;
@@ -1109,12 +1110,11 @@ int enqueue_render(agx_ctx *c, const agx_render_params *p, hipStream_t st, unsig
             pb.cnt_in = cin;
             pb.cnt_out = cout;
             launch_count_rays(cin, rays, st);
-            launch_trace_closest(c->ds, pb, n_closest_max, false, c->dcnt, st);
-            launch_trace_shadow(c->ds, pb, n_shadow_max, false, c->dcnt + 1, st);
+            launch_trace_closest(c->ds, pb, bounce == 0 ? uint32_t(rc.n_paths) : n_closest_max, false, c->dcnt, st);
+            if (bounce > 0) launch_trace_shadow(c->ds, pb, n_shadow_max, false, c->dcnt + 1, st);
             if (c->ds.features & SF_MEDIA) launch_media(c->ds, rc, pb, uint32_t(rc.n_paths), st);
-            launch_reset_counters(cout, st);
             launch_shade(c->ds, rc, pb, uint32_t(rc.n_paths), st);
-            launch_queue_compact(pb, uint32_t(rc.n_paths), rc.L, c->qc_blk, st);
+            launch_queue_compact(pb, uint32_t(rc.n_paths), rc.L, c->qc_blk, nullptr, st);
             std::swap(cin, cout);
             std::swap(pb.q_in, pb.q_out);
         }

@@ -3020,8 +3020,9 @@ __global__ void __launch_bounds__(QC_THREADS) k_queue_count(PathBuffers pb, uint
     }
 }
 
-// one block: blk[b] <- exclusive prefix of the block counts; cnt_out[0..2] <- totals
-__global__ void __launch_bounds__(1024) k_queue_scan(PathBuffers pb, uint4 *blk) {
+// one block: blk[b] <- exclusive prefix of the block counts; cnt_out[0..2] <- totals, and
+// the same into host (pinned memory, may be null)
+__global__ void __launch_bounds__(1024) k_queue_scan(PathBuffers pb, uint4 *blk, uint32_t *host) {
     const uint32_t n = pb.cnt_in[2];
     const uint32_t nb = (n + QC_SPAN - 1) / QC_SPAN;
     __shared__ uint32_t wsum[3][16];
@@ -3048,6 +3049,11 @@ __global__ void __launch_bounds__(1024) k_queue_scan(PathBuffers pb, uint4 *blk)
         pb.cnt_out[0] = carry[0];
         pb.cnt_out[1] = carry[1];
         pb.cnt_out[2] = carry[2];
+        if (host) {
+            host[0] = carry[0];
+            host[1] = carry[1];
+            host[2] = carry[2];
+        }
     }
 }
 
@@ -3451,11 +3457,12 @@ void launch_shade(const DevScene &s, const RenderConst &rc, const PathBuffers &p
 
 uint32_t queue_compact_blocks(uint32_t max_n) { return (max_n + QC_SPAN - 1) / QC_SPAN + 1; }
 
-void launch_queue_compact(const PathBuffers &pb, uint32_t max_n, int L, uint4 *blk, hipStream_t st) {
+void launch_queue_compact(const PathBuffers &pb, uint32_t max_n, int L, uint4 *blk, uint32_t *host_counts,
+                          hipStream_t st) {
     const uint32_t nb = (max_n + QC_SPAN - 1) / QC_SPAN;
     const uint32_t nl = uint32_t(L > 0 ? L : 0);
     if (nb) hipLaunchKernelGGL(k_queue_count, dim3(nb), dim3(QC_THREADS), 0, st, pb, nl, blk);
-    hipLaunchKernelGGL(k_queue_scan, dim3(1), dim3(1024), 0, st, pb, blk);
+    hipLaunchKernelGGL(k_queue_scan, dim3(1), dim3(1024), 0, st, pb, blk, host_counts);
     if (nb) hipLaunchKernelGGL(k_queue_scatter, dim3(nb), dim3(QC_THREADS), 0, st, pb, nl, blk);
 }
 

@@ -1,0 +1,54 @@
+"""The render loop's launch decisions: passes whose first bounce is thinned by
+roulette (queues counted on the device), scenes without lights (no shadow
+launches) and images of a few paths, path for path against the oracle; the ray
+counts are those of the queues and the same in every pass split.
+"""
+import numpy as np
+import pytest
+
+from atrc_amd import capi, scenes
+
+from test_gpu_render_parity import _path_parity
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("accel", [capi.ACCEL_ATRC, capi.ACCEL_BVH4, capi.ACCEL_BVH4_WATERTIGHT])
+@pytest.mark.parametrize("W,H", [(1, 1), (13, 5), (65, 63)])
+@pytest.mark.parametrize("min_depth", [0, 2])
+def test_small_images_path_parity(gpu_ctx, W, H, min_depth, accel):
+    s, cam, tr = scenes.cornell_box()
+    s.accel = accel
+    # a single path may round to another decision: small images must agree on all but one
+    _path_parity(gpu_ctx, s, cam, dict(tr, min_depth=min_depth), W, H, f"small {W}x{H} min_depth {min_depth}",
+                 min_frac=min(0.97, 1 - 1.5 / (W * H)))
+
+
+def test_no_lights(gpu_ctx):
+    s, cam, tr = scenes.cornell_box()
+    s.entities[-1].emit = (0.0, 0.0, 0.0)
+    s.accel = capi.ACCEL_BVH4
+    desc, keep = s.to_desc()
+    gpu_ctx.upload_scene(desc)
+    print("[launches] cornell without its light", flush=True)
+    g = gpu_ctx.render(scenes.render_params(40, 30, 4, cam, seed=3, **tr))
+    st = gpu_ctx.stats()
+    assert not g["image"].any() and st["shadow_rays"] == 0 and st["trace_shadow_launches"] == 0
+    assert st["closest_rays"] > 40 * 30 * 4
+
+
+def test_ray_counts_add_up(gpu_ctx):
+    """The rays of one render are those of its samples rendered one at a time."""
+    s, cam, tr = scenes.cornell_box()
+    s.accel = capi.ACCEL_BVH4
+    desc, keep = s.to_desc()
+    gpu_ctx.upload_scene(desc)
+    print("[launches] ray counts of 3 samples, together and apart", flush=True)
+    acc = np.zeros(3, np.int64)
+    for k in range(3):
+        gpu_ctx.render(scenes.render_params(70, 51, 1, cam, seed=3, sample_begin=k, **tr))
+        st = gpu_ctx.stats()
+        acc += [st["closest_rays"], st["shadow_rays"], st["paths"]]
+    gpu_ctx.render(scenes.render_params(70, 51, 3, cam, seed=3, **tr))
+    st = gpu_ctx.stats()
+    assert [st["closest_rays"], st["shadow_rays"], st["paths"]] == acc.tolist()
