@@ -475,12 +475,23 @@ static int upload_host_scene(agx_ctx *c, const HostScene &hs) {
     DevScene ds{};
     DevEntity *ents = nullptr;
     DevMaterial *mats = nullptr;
-    vec4 *bn = nullptr, *bp = nullptr, *bi = nullptr, *tn = nullptr, *b4n = nullptr, *b4p = nullptr;
-    int32_t *tp = nullptr, *ai = nullptr;
+    vec4 *bn = nullptr, *bp = nullptr, *bi = nullptr, *tn = nullptr, *b4n = nullptr, *b4p = nullptr, *ar = nullptr;
+    int32_t *ai = nullptr;
     float *ap = nullptr, *gr = nullptr, *etx = nullptr, *epr = nullptr, *eap = nullptr;
     int32_t *eai = nullptr;
     DevMedium *md = nullptr;
     auto track = [&](void *p) { if (p) c->scene_allocs.push_back(p); };
+    // the aggregate's entities with what their visit needs first (Atrc's structures only)
+    std::vector<vec4> refs;
+    if (hs.accel == AGX_ACCEL_ATRC) {
+        const bool tree = hs.aggregate == AGX_AGGREGATE_BVH;
+        refs.resize(tree ? hs.tlas_prims.size() : hs.ents.size());
+        for (size_t k = 0; k < refs.size(); ++k) {
+            const uint32_t i = tree ? uint32_t(hs.tlas_prims[k]) : uint32_t(k);
+            const uint32_t w[4] = {i, uint32_t(hs.ents[i].kind), hs.ents[i].node_base, 0};
+            std::memcpy(&refs[k], w, sizeof(w));
+        }
+    }
     hipError_t e = hipSuccess;
     if (e == hipSuccess) { e = upload(&ents, hs.ents, c->stream); track(ents); }
     if (e == hipSuccess) { e = upload(&etx, hs.env_texels, c->stream); track(etx); }
@@ -492,7 +503,7 @@ static int upload_host_scene(agx_ctx *c, const HostScene &hs) {
     if (e == hipSuccess) { e = upload(&bp, hs.blas_prims, c->stream); track(bp); }
     if (e == hipSuccess) { e = upload(&bi, hs.blas_info, c->stream); track(bi); }
     if (e == hipSuccess) { e = upload(&tn, hs.tlas_nodes, c->stream); track(tn); }
-    if (e == hipSuccess) { e = upload(&tp, hs.tlas_prims, c->stream); track(tp); }
+    if (e == hipSuccess) { e = upload(&ar, refs, c->stream); track(ar); }
     if (e == hipSuccess) { e = upload(&ap, hs.alias_prob, c->stream); track(ap); }
     if (e == hipSuccess) { e = upload(&ai, hs.alias_idx, c->stream); track(ai); }
     if (e == hipSuccess) { e = upload(&md, hs.media, c->stream); track(md); }
@@ -513,7 +524,7 @@ static int upload_host_scene(agx_ctx *c, const HostScene &hs) {
     ds.blas_prims = bp;
     ds.blas_info = bi;
     ds.tlas_nodes = tn;
-    ds.tlas_prims = tp;
+    ds.agg_refs = ar;
     ds.alias_prob = ap;
     ds.alias_idx = ai;
     ds.media = md;
@@ -545,15 +556,6 @@ static int upload_host_scene(agx_ctx *c, const HostScene &hs) {
     ds.n_ent = int32_t(hs.ents.size());
     ds.aggregate = hs.aggregate;
     ds.n_lights = int32_t(hs.lights.size());
-    // stack entries needed: TLAS pending nodes (depth + 1) + BLAS (depth + 1) + 1
-    // The per-thread private stack is the default: at 44 VGPRs it keeps 8 waves per
-    // SIMD, while the 32 KiB LDS column per block caps occupancy at 5 (measured
-    // on the 1M-triangle scene: closest-hit 83.8 ms private vs 99.5 ms LDS for 8 spp).
-    // AGX_TRAVERSAL_STACK=lds selects the LDS column when the depths fit it.
-    ds.lds_stack = 0;
-    if (const char *e = std::getenv("AGX_TRAVERSAL_STACK"))
-        if (std::string(e) == "lds")
-            ds.lds_stack = (hs.max_tlas_depth + 1) + (hs.max_blas_depth + 1) + 1 <= LDS_STACK ? 1 : 0;
     ds.env_kind = hs.env_kind;
     for (int i = 0; i < MAX_LIGHTS; ++i) ds.lights[i] = i < ds.n_lights ? hs.lights[size_t(i)] : -2;
     ds.sky_top = hs.sky_top;

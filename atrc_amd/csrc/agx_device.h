@@ -8,7 +8,7 @@
 //   blas_prims float4[3*P]             (a.xyz, original id) (b-a, 0) (c-a, 0)        48 B / triangle
 //   blas_info  float4[6*P]             interpolated normal / uv deltas and frame      96 B / triangle
 //   tlas_nodes float4[2*T]             entity BVH: (low.xyz, left|leaf-start) (high.xyz, right|leaf-end)
-//   tlas_prims int32[]                 entity indices referenced by TLAS leaves
+//   agg_refs   uint4[]                 entities of the TLAS leaves: (entity, kind, root node of a mesh, 0)
 //   alias_prob/alias_idx               per-mesh triangle-area alias tables (emissive meshes)
 //   lights     int32[L]                Atrc light order: -1 = environment, else entity index
 #pragma once
@@ -60,7 +60,6 @@ constexpr int BVH4_RING_CLOSEST = 8;
 constexpr int BVH4_RING_ANY = 16;
 constexpr int BLAS_STACK = 96;               // >= max BLAS depth + 2 (checked at upload)
 constexpr int TLAS_STACK = 64;
-constexpr int LDS_STACK = 32;                // LDS stack column per thread (TLAS + BLAS entries)
 
 // DevEntity::flags
 constexpr int32_t EF_NO_DENOISE = 1;
@@ -144,7 +143,8 @@ struct DevScene {
     const vec4 *blas_prims;
     const vec4 *blas_info;
     const vec4 *tlas_nodes;
-    const int32_t *tlas_prims;
+    const vec4 *agg_refs;  // entities in the order of the aggregate (native: list order; BVH: leaf order):
+                           // uint bits (entity, AGX_GEOM_*, root node of a mesh, 0)
     const float *alias_prob;
     const int32_t *alias_idx;
     const DevMedium *media;
@@ -154,7 +154,6 @@ struct DevScene {
     int32_t aggregate;     // AGX_AGGREGATE_*
     int32_t n_lights;
     int32_t env_kind;
-    int32_t lds_stack;     // 1: TLAS depth + BLAS depth fit the LDS stack column
     int32_t accel;         // AGX_ACCEL_*
     int32_t bvh4_large_stack;  // 1: the BVH4 is too deep for BVH4_STACK_SMALL
     uint32_t features;     // SF_* the scene uses (media, Disney, delta materials)

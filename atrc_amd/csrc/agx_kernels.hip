@@ -249,105 +249,57 @@ struct HitRec {
     int32_t ent, prim;
 };
 
-// threads per block of the traversal kernels (the Atrc-mode LDS stack columns hold 256)
+// threads per block of the traversal kernels outside the BVH4 modes
 constexpr unsigned TRACE_BLOCK = 256;
-static_assert(TRACE_BLOCK <= 256 && TRACE_BLOCK % 64 == 0, "traversal block: whole waves, at most the LDS columns");
 
-// Traversal stacks.  TLAS and BLAS share one stack: a BLAS traversal uses the
-// entries above the TLAS entries pending at its entity.  LdsStack keeps one
-// column per thread in LDS ([depth][thread], conflict-free at equal depth);
-// PrivStack is the private-memory fallback for scenes whose BVH depth exceeds
-// the LDS column (chosen at upload).
-struct LdsStack {
-    uint32_t *col;  // &lds[0][threadIdx.x]
-    int top;
-    __device__ __forceinline__ void push(uint32_t v) { col[top * 256] = v; ++top; }
-    __device__ __forceinline__ uint32_t pop() { --top; return col[top * 256]; }
-};
-struct PrivStack {
-    uint32_t s[BLAS_STACK + TLAS_STACK];
-    int top;
-    __device__ __forceinline__ void push(uint32_t v) { s[top++] = v; }
-    __device__ __forceinline__ uint32_t pop() { return s[--top]; }
-};
-
-// UntransformedTriangleBVH::closest_intersection (triangle_bvh.cpp:403-488)
-template <bool STATS, class Stack>
-__device__ bool blas_closest(const DevScene &s, const DevEntity &e, V o, V d, float tmin, float tmax, HitRec *h,
-                             Counts &c, Stack &stk) {
-    const V inv = mk(1 / d.x, 1 / d.y, 1 / d.z);
-    const uint32_t root = e.node_base;
-    float te;
-    if (STATS) c.visits++;
-    if (!slab(ld(s.blas_nodes[2 * root]), ld(s.blas_nodes[2 * root + 1]), o, inv, tmin, tmax, &te)) return false;
-    const int bottom = stk.top;
-    stk.push(root);
-    float best = INF_F, bu = 0, bv = 0;
-    uint32_t bslot = 0;
-    while (stk.top > bottom) {
-        const uint32_t ni = stk.pop();
-        const float4 lo = ld(s.blas_nodes[2 * ni]), hi = ld(s.blas_nodes[2 * ni + 1]);
-        const uint32_t start = fbits(lo.w), end = fbits(hi.w);
-        if (start != INTERIOR) {
-            for (uint32_t i = start; i < end; ++i) {
-                if (STATS) c.tests++;
-                const vec4 p0 = s.blas_prims[3 * i], p1 = s.blas_prims[3 * i + 1], p2 = s.blas_prims[3 * i + 2];
-                float tt, uu, vv;
-                if (mt_closest(o, d, tmin, tmax, mk(p0), mk(p1), mk(p2), &tt, &uu, &vv)) {
-                    best = tt; bu = uu; bv = vv; bslot = i;
-                    tmax = tt;
-                }
-            }
-        } else {
-            const uint32_t l = ni + 1, r = end;
-            float tl, tr;
-            if (STATS) c.visits += 2;
-            const bool al = slab(ld(s.blas_nodes[2 * l]), ld(s.blas_nodes[2 * l + 1]), o, inv, tmin, tmax, &tl);
-            const bool ar = slab(ld(s.blas_nodes[2 * r]), ld(s.blas_nodes[2 * r + 1]), o, inv, tmin, tmax, &tr);
-            if (al && ar) {
-                if (tl < tr) { stk.push(r); stk.push(l); }
-                else { stk.push(l); stk.push(r); }
-            } else if (al) {
-                stk.push(l);
-            } else if (ar) {
-                stk.push(r);
-            }
-        }
-    }
-    if (isinf(best)) return false;
-    h->t = best; h->u = bu; h->v = bv; h->prim = int32_t(bslot);
-    return true;
+// Per-lane traversal stack whose newest S entries live in an LDS ring and
+// whose older entries spill to a private array.  The ring is a
+// [slot][TB] array (TB = threads per block), so the lanes of a wave touch consecutive words at
+// any mix of depths and never conflict on a bank; an entry reaches private
+// memory only while the stack is deeper than S.  A push onto a full ring moves
+// the oldest ring entry (the same slot) out to the spill array, and a pop that
+// leaves the stack at depth >= S brings it back, so the ring always holds the
+// top min(depth, S) entries.  Each lane touches only its own column: no
+// barrier is needed.  (Free functions over separate locals, so that the depth
+// and the column address stay in registers.)
+template <int S, int TB, class E>
+__device__ __forceinline__ void ring_push(E *col, E *spill, int &sp, E e) {
+    const int slot = sp & (S - 1);
+    if (sp >= S) spill[sp - S] = col[slot * TB];
+    col[slot * TB] = e;
+    ++sp;
+}
+template <int S, int TB, class E>
+__device__ __forceinline__ E ring_pop(E *col, const E *spill, int &sp) {
+    --sp;
+    const int slot = sp & (S - 1);
+    const E e = col[slot * TB];
+    if (sp >= S) col[slot * TB] = spill[sp - S];
+    return e;
 }
 
-// UntransformedTriangleBVH::has_intersection (triangle_bvh.cpp:363-401)
-template <bool STATS, class Stack>
-__device__ bool blas_any(const DevScene &s, const DevEntity &e, V o, V d, float tmin, float tmax, Counts &c,
-                         Stack &stk) {
-    const V inv = mk(1 / d.x, 1 / d.y, 1 / d.z);
-    const uint32_t root = e.node_base;
-    float te;
-    if (STATS) c.visits++;
-    if (!slab(ld(s.blas_nodes[2 * root]), ld(s.blas_nodes[2 * root + 1]), o, inv, tmin, tmax, &te)) return false;
-    const int bottom = stk.top;
-    stk.push(root);
-    while (stk.top > bottom) {
-        const uint32_t ni = stk.pop();
-        const float4 lo = ld(s.blas_nodes[2 * ni]), hi = ld(s.blas_nodes[2 * ni + 1]);
-        const uint32_t start = fbits(lo.w), end = fbits(hi.w);
-        if (start != INTERIOR) {
-            for (uint32_t i = start; i < end; ++i) {
-                if (STATS) c.tests++;
-                const vec4 p0 = s.blas_prims[3 * i], p1 = s.blas_prims[3 * i + 1], p2 = s.blas_prims[3 * i + 2];
-                if (mt_any(o, d, tmin, tmax, mk(p0), mk(p1), mk(p2))) { stk.top = bottom; return true; }
-            }
-        } else {
-            const uint32_t l = ni + 1, r = end;
-            if (STATS) c.visits += 2;
-            if (slab(ld(s.blas_nodes[2 * l]), ld(s.blas_nodes[2 * l + 1]), o, inv, tmin, tmax, &te)) stk.push(l);
-            if (slab(ld(s.blas_nodes[2 * r]), ld(s.blas_nodes[2 * r + 1]), o, inv, tmin, tmax, &te)) stk.push(r);
-        }
-    }
-    return false;
+// ---------------------------------------------------------------- Atrc's structures
+// TLAS and BLAS share one stack: a BLAS traversal uses the entries above the
+// TLAS entries pending at its entity.  An entry is what its node's visit needs:
+// (first primitive, end) of a leaf, (BLAS_NODE | index, right child) of an
+// interior node, so a popped node is not loaded again, and the child that
+// comes off the stack next is not pushed at all.  These launches are bound by the chain of one
+// ray's dependent loads (few rays, 1.4 waves per SIMD at 400x300x8): a step of it
+// was a pop from private memory, the node's load and its children's loads one after another,
+// and is now the children's loads (24 spheres, 403x301 at 8 samples, four planes: 7.05 -> 5.64 ms,
+// and 4.50 ms with the loop structure of scene_query).
+constexpr uint32_t BLAS_NODE = 0x80000000u;
+constexpr int ATRC_RING = 8;
+constexpr int ATRC_SPILL = BLAS_STACK + TLAS_STACK - ATRC_RING;
+
+struct BlasRef {  // a node about to be visited
+    uint32_t idx, start, end;
+};
+__device__ __forceinline__ uint2 pack_blas(const BlasRef &n) {
+    return make_uint2(n.start == INTERIOR ? n.idx | BLAS_NODE : n.start, n.end);
+}
+__device__ __forceinline__ BlasRef unpack_blas(uint2 e) {
+    return (e.x & BLAS_NODE) ? BlasRef{e.x & ~BLAS_NODE, INTERIOR, e.y} : BlasRef{0, e.x, e.y};
 }
 
 // sphere_aux.h:10-16
@@ -416,18 +368,6 @@ __device__ bool analytic_closest(const DevEntity &e, int32_t ei, V o, V d, float
     }
 }
 
-// Closest hit of one entity; on success *tmax is lowered to the hit distance.
-template <bool STATS, class Stack>
-__device__ bool entity_closest(const DevScene &s, int32_t ei, V o, V d, float tmin, float *tmax, HitRec *h,
-                               Counts &c, Stack &stk) {
-    const DevEntity &e = s.ents[ei];
-    if (e.kind != AGX_GEOM_TRIANGLE_BVH) return analytic_closest<STATS>(e, ei, o, d, tmin, tmax, h, c);
-    if (!blas_closest<STATS>(s, e, o, d, tmin, *tmax, h, c, stk)) return false;
-    h->ent = ei;
-    *tmax = h->t;
-    return true;
-}
-
 template <bool STATS>
 __device__ bool analytic_any(const DevEntity &e, V o, V d, float tmin, float tmax, Counts &c) {
     switch (e.kind) {
@@ -463,73 +403,122 @@ __device__ bool analytic_any(const DevEntity &e, V o, V d, float tmin, float tma
     }
 }
 
-template <bool STATS, class Stack>
-__device__ bool entity_any(const DevScene &s, int32_t ei, V o, V d, float tmin, float tmax, Counts &c, Stack &stk) {
-    const DevEntity &e = s.ents[ei];
-    if (e.kind != AGX_GEOM_TRIANGLE_BVH) return analytic_any<STATS>(e, o, d, tmin, tmax, c);
-    return blas_any<STATS>(s, e, o, d, tmin, tmax, c, stk);
-}
-
 // AABB::intersect (common.h:384-395) with std::min/max operand order
 __device__ __forceinline__ bool tlas_box(float4 lo, float4 hi, V o, V inv, float tmin, float tmax) {
     float te;
     return slab(lo, hi, o, inv, tmin, tmax, &te);
 }
 
-// Scene closest hit: NativeAggregate (native_aggregate.cpp:31-45) or EntityBVH
-// (entity_bvh.cpp:141-172, left subtree before right, node bound tested on entry).
-template <bool STATS, class Stack>
-__device__ bool scene_closest(const DevScene &s, V o, V d, float tmin, float tmax, HitRec *h, Counts &c, Stack &stk) {
+// Scene queries over Atrc's structures: closest hit (ANY = false; *h holds it)
+// or any hit.  Aggregates: NativeAggregate (native_aggregate.cpp:31-45: every entity in
+// order) or EntityBVH (entity_bvh.cpp:141-172: left subtree before right, node bound
+// tested on entry).  Meshes: UntransformedTriangleBVH::closest_intersection
+// (triangle_bvh.cpp:403-488: the nearer child first) and has_intersection (:363-401:
+// the right child first).  ring = this lane's column of an [ATRC_RING][TB] LDS array.
+//
+// The lanes of a wave meet different entities after different numbers of
+// steps.  The outer loop takes every lane to its next mesh (or its end); the inner loop
+// steps through the meshes until fewer than half of those lanes are still inside one,
+// so that a lane waits for at most the slower half of its wave.
+template <bool STATS, int TB, bool ANY>
+__device__ bool scene_query(const DevScene &s, V o, V d, float tmin, float tmax, HitRec *h, Counts &c, uint2 *ring) {
+    uint2 spill[ATRC_SPILL];
+    const uint4 *refs = reinterpret_cast<const uint4 *>(s.agg_refs);
+    const V inv = mk(1 / d.x, 1 / d.y, 1 / d.z);
+    const bool tree = s.aggregate == AGX_AGGREGATE_BVH;
     bool hit = false;
-    stk.top = 0;
-    if (s.aggregate == AGX_AGGREGATE_BVH) {
-        const V inv = mk(1 / d.x, 1 / d.y, 1 / d.z);
-        stk.push(0);
-        while (stk.top > 0) {
-            const uint32_t ni = stk.pop();
+    int sp = 0;
+    uint32_t ni = 0;                               // TLAS node to visit next
+    uint32_t i = 0, end = tree ? 0 : uint32_t(s.n_ent);  // aggregate entries still to test
+    bool last = !tree;                             // no TLAS node is left once they are tested
+    // the mesh the lane is inside: node to visit, entity, stack depth at its root
+    bool inside = false;
+    BlasRef n{0, 0, 0};
+    int32_t ent = -1;
+    int bottom = 0;
+    for (;;) {
+        while (!inside) {  // to the next mesh whose root the ray enters
+            float te;
+            if (i < end) {
+                const uint4 ref = refs[i++];
+                if (int32_t(ref.y) == AGX_GEOM_TRIANGLE_BVH) {
+                    if (STATS) c.visits++;
+                    const float4 lo = ld(s.blas_nodes[2 * ref.z]), hi = ld(s.blas_nodes[2 * ref.z + 1]);
+                    if (slab(lo, hi, o, inv, tmin, tmax, &te)) {
+                        n = BlasRef{ref.z, fbits(lo.w), fbits(hi.w)};
+                        ent = int32_t(ref.x);
+                        bottom = sp;
+                        inside = true;
+                    }
+                } else if (ANY) {
+                    if (analytic_any<STATS>(s.ents[ref.x], o, d, tmin, tmax, c)) return true;
+                } else {
+                    hit = analytic_closest<STATS>(s.ents[ref.x], int32_t(ref.x), o, d, tmin, &tmax, h, c) || hit;
+                }
+                continue;
+            }
+            if (last) return hit;
             const float4 lo = ld(s.tlas_nodes[2 * ni]), hi = ld(s.tlas_nodes[2 * ni + 1]);
             if (STATS) c.visits++;
-            if (!tlas_box(lo, hi, o, inv, tmin, tmax)) continue;
-            const uint32_t a = fbits(lo.w), b = fbits(hi.w);
-            if (a & TLAS_LEAF) {
-                for (uint32_t i = a & ~TLAS_LEAF; i < b; ++i)
-                    hit = entity_closest<STATS>(s, s.tlas_prims[i], o, d, tmin, &tmax, h, c, stk) || hit;
-            } else {
-                stk.push(b);
-                stk.push(a);
+            if (tlas_box(lo, hi, o, inv, tmin, tmax)) {
+                const uint32_t a = fbits(lo.w), b = fbits(hi.w);
+                if (!(a & TLAS_LEAF)) {
+                    ring_push<ATRC_RING, TB>(ring, spill, sp, make_uint2(b, 0));
+                    ni = a;
+                    continue;
+                }
+                i = a & ~TLAS_LEAF;
+                end = b;
             }
+            if (sp == 0) last = true;
+            else ni = ring_pop<ATRC_RING, TB>(ring, spill, sp).x;
         }
-    } else {
-        for (int32_t i = 0; i < s.n_ent; ++i) hit = entity_closest<STATS>(s, i, o, d, tmin, &tmax, h, c, stk) || hit;
-    }
-    return hit;
-}
-
-template <bool STATS, class Stack>
-__device__ bool scene_any(const DevScene &s, V o, V d, float tmin, float tmax, Counts &c, Stack &stk) {
-    stk.top = 0;
-    if (s.aggregate == AGX_AGGREGATE_BVH) {
-        const V inv = mk(1 / d.x, 1 / d.y, 1 / d.z);
-        stk.push(0);
-        while (stk.top > 0) {
-            const uint32_t ni = stk.pop();
-            const float4 lo = ld(s.tlas_nodes[2 * ni]), hi = ld(s.tlas_nodes[2 * ni + 1]);
-            if (STATS) c.visits++;
-            if (!tlas_box(lo, hi, o, inv, tmin, tmax)) continue;
-            const uint32_t a = fbits(lo.w), b = fbits(hi.w);
-            if (a & TLAS_LEAF) {
-                for (uint32_t i = a & ~TLAS_LEAF; i < b; ++i)
-                    if (entity_any<STATS>(s, s.tlas_prims[i], o, d, tmin, tmax, c, stk)) return true;
+        const int lanes = __popcll(__ballot(true));
+        do {
+            bool pop = true;
+            if (n.start != INTERIOR) {
+                // the next primitive's rows are in flight while one is tested
+                const vec4 *P = s.blas_prims + 3 * size_t(n.start < n.end ? n.start : 0);
+                vec4 p0 = P[0], p1 = P[1], p2 = P[2];
+                for (uint32_t k = n.start; k < n.end; ++k) {
+                    P += k + 1 < n.end ? 3 : 0;
+                    const vec4 q0 = P[0], q1 = P[1], q2 = P[2];
+                    if (STATS) c.tests++;
+                    if (ANY) {
+                        if (mt_any(o, d, tmin, tmax, mk(p0), mk(p1), mk(p2))) return true;
+                    } else {
+                        float tt, uu, vv;
+                        // (a hit at infinite distance is none, triangle_bvh.cpp:480)
+                        if (mt_closest(o, d, tmin, tmax, mk(p0), mk(p1), mk(p2), &tt, &uu, &vv) && !isinf(tt)) {
+                            h->t = tt; h->u = uu; h->v = vv; h->prim = int32_t(k); h->ent = ent;
+                            tmax = tt;
+                            hit = true;
+                        }
+                    }
+                    p0 = q0; p1 = q1; p2 = q2;
+                }
             } else {
-                stk.push(b);
-                stk.push(a);
+                const uint32_t l = n.idx + 1, r = n.end;
+                float tl, tr;
+                if (STATS) c.visits += 2;
+                const float4 llo = ld(s.blas_nodes[2 * l]), lhi = ld(s.blas_nodes[2 * l + 1]);
+                const float4 rlo = ld(s.blas_nodes[2 * r]), rhi = ld(s.blas_nodes[2 * r + 1]);
+                const bool al = slab(llo, lhi, o, inv, tmin, tmax, &tl);
+                const bool ar = slab(rlo, rhi, o, inv, tmin, tmax, &tr);
+                const BlasRef L{l, fbits(llo.w), fbits(lhi.w)}, R{r, fbits(rlo.w), fbits(rhi.w)};
+                if (al | ar) {
+                    const bool left = al && (!ar || (!ANY && tl < tr));
+                    if (al & ar) ring_push<ATRC_RING, TB>(ring, spill, sp, pack_blas(left ? R : L));
+                    n = left ? L : R;
+                    pop = false;
+                }
             }
-        }
-        return false;
+            if (pop) {
+                inside = sp != bottom;
+                if (inside) n = unpack_blas(ring_pop<ATRC_RING, TB>(ring, spill, sp));
+            }
+        } while (inside && 2 * __popcll(__ballot(inside)) >= lanes);
     }
-    for (int32_t i = 0; i < s.n_ent; ++i)
-        if (entity_any<STATS>(s, i, o, d, tmin, tmax, c, stk)) return true;
-    return false;
 }
 
 // ---------------------------------------------------------------- watertight triangle test
@@ -664,32 +653,8 @@ __device__ __forceinline__ void cswap(float t[4], uint32_t k[4], int a, int b) {
     }
 }
 
-// Per-lane traversal stack whose newest S entries live in an LDS ring and
-// whose older entries spill to a private array.  The ring is a
-// [slot][TB] array (TB = threads per block), so the lanes of a wave touch consecutive words at
-// any mix of depths and never conflict on a bank; an entry reaches private
-// memory only while the stack is deeper than S.  A push onto a full ring moves
-// the oldest ring entry (the same slot) out to the spill array, and a pop that
-// leaves the stack at depth >= S brings it back, so the ring always holds the
-// top min(depth, S) entries.  Each lane touches only its own column: no
-// barrier is needed.  (Free functions over separate locals, so that the depth
-// and the column address stay in registers.)
-template <int S, int TB, class E>
-__device__ __forceinline__ void ring_push(E *col, E *spill, int &sp, E e) {
-    const int slot = sp & (S - 1);
-    if (sp >= S) spill[sp - S] = col[slot * TB];
-    col[slot * TB] = e;
-    ++sp;
-}
-template <int S, int TB, class E>
-__device__ __forceinline__ E ring_pop(E *col, const E *spill, int &sp) {
-    --sp;
-    const int slot = sp & (S - 1);
-    const E e = col[slot * TB];
-    if (sp >= S) col[slot * TB] = spill[sp - S];
-    return e;
-}
-static_assert((BVH4_RING_CLOSEST & (BVH4_RING_CLOSEST - 1)) == 0 && (BVH4_RING_ANY & (BVH4_RING_ANY - 1)) == 0,
+static_assert((BVH4_RING_CLOSEST & (BVH4_RING_CLOSEST - 1)) == 0 && (BVH4_RING_ANY & (BVH4_RING_ANY - 1)) == 0 &&
+                  (ATRC_RING & (ATRC_RING - 1)) == 0,
               "ring sizes are powers of two");
 
 // A quad's record carries its first triangle (A, B - A, C - A), so that quads
@@ -941,32 +906,24 @@ __device__ bool b4_any(const DevScene &s, V o, V d, float tmin, float tmax, Coun
     return q.occluded;
 }
 
-// Traversal variants: Atrc's structures with the private or the LDS stack, or
-// the BVH4 with the small or the large stack (LDS ring + private spill), with
-// Atrc's triangle test or the watertight one.
-enum { TM_ATRC_PRIV = 0, TM_ATRC_LDS = 1, TM_B4_SMALL = 2, TM_B4_LARGE = 3, TM_B4W_SMALL = 4, TM_B4W_LARGE = 5 };
+// Traversal variants: Atrc's structures, or the BVH4 with the small or the
+// large stack, with Atrc's triangle test or the watertight one.
+enum { TM_ATRC = 0, TM_B4_SMALL = 2, TM_B4_LARGE = 3, TM_B4W_SMALL = 4, TM_B4W_LARGE = 5 };
 
-// LDS words per thread of a traversal kernel: the Atrc-mode LDS column, or
-// the BVH4 rings (the closest-hit ring of (code, distance) pairs and the
-// any-hit ring of codes share the space; k_trace_rays runs either).
+// LDS words per thread of a traversal kernel: the BVH4 rings (the closest-hit
+// ring of (code, distance) pairs and the any-hit ring of codes share the space;
+// k_trace_rays runs either) or the ring of Atrc's structures.
 constexpr int lds_stack_words(int tm) {
-    return tm == TM_ATRC_LDS ? LDS_STACK
-                             : (tm >= TM_B4_SMALL ? (2 * BVH4_RING_CLOSEST > BVH4_RING_ANY ? 2 * BVH4_RING_CLOSEST
-                                                                                          : BVH4_RING_ANY)
-                                                  : 1);
+    return tm == TM_ATRC ? 2 * ATRC_RING
+                         : (2 * BVH4_RING_CLOSEST > BVH4_RING_ANY ? 2 * BVH4_RING_CLOSEST : BVH4_RING_ANY);
 }
 
-// lds = the block's [lds_stack_words(TM)][TB] word array (the Atrc-mode LDS
-// column needs TB = 256)
+// lds = the block's [lds_stack_words(TM)][TB] word array
 template <bool STATS, int TM, int TB>
 __device__ __forceinline__ bool query_closest(const DevScene &s, V o, V d, float tmin, float tmax, HitRec *h,
                                               Counts &c, uint32_t *lds) {
-    if constexpr (TM == TM_ATRC_LDS) {
-        LdsStack stk{lds + threadIdx.x, 0};
-        return scene_closest<STATS>(s, o, d, tmin, tmax, h, c, stk);
-    } else if constexpr (TM == TM_ATRC_PRIV) {
-        PrivStack stk;
-        return scene_closest<STATS>(s, o, d, tmin, tmax, h, c, stk);
+    if constexpr (TM == TM_ATRC) {
+        return scene_query<STATS, TB, false>(s, o, d, tmin, tmax, h, c, reinterpret_cast<uint2 *>(lds) + threadIdx.x);
     } else if constexpr (TM == TM_B4_SMALL || TM == TM_B4W_SMALL) {
         return b4_closest<STATS, BVH4_STACK_SMALL, TM == TM_B4W_SMALL, TB>(s, o, d, tmin, tmax, h, c,
                                                                         reinterpret_cast<uint2 *>(lds) + threadIdx.x);
@@ -979,12 +936,8 @@ __device__ __forceinline__ bool query_closest(const DevScene &s, V o, V d, float
 template <bool STATS, int TM, int TB>
 __device__ __forceinline__ bool query_any(const DevScene &s, V o, V d, float tmin, float tmax, Counts &c,
                                           uint32_t *lds) {
-    if constexpr (TM == TM_ATRC_LDS) {
-        LdsStack stk{lds + threadIdx.x, 0};
-        return scene_any<STATS>(s, o, d, tmin, tmax, c, stk);
-    } else if constexpr (TM == TM_ATRC_PRIV) {
-        PrivStack stk;
-        return scene_any<STATS>(s, o, d, tmin, tmax, c, stk);
+    if constexpr (TM == TM_ATRC) {
+        return scene_query<STATS, TB, true>(s, o, d, tmin, tmax, nullptr, c, reinterpret_cast<uint2 *>(lds) + threadIdx.x);
     } else if constexpr (TM == TM_B4_SMALL || TM == TM_B4W_SMALL) {
         return b4_any<STATS, BVH4_STACK_SMALL, TM == TM_B4W_SMALL, TB>(s, o, d, tmin, tmax, c, lds + threadIdx.x);
     } else {
@@ -992,7 +945,7 @@ __device__ __forceinline__ bool query_any(const DevScene &s, V o, V d, float tmi
     }
 }
 
-// The block's traversal stack memory in LDS (one word when the variant has none)
+// The block's traversal stack memory in LDS
 #define AGX_LDS_COLUMN(TM, TB)                                                 \
     __shared__ __align__(16) uint32_t lds_stack_[lds_stack_words(TM) * (TB)]; \
     uint32_t *lds_col = lds_stack_
@@ -1822,7 +1775,7 @@ __device__ __forceinline__ int32_t xcd_block(uint32_t n) {
 // the latency of its node fetches, and the default allocation (66 VGPRs) left
 // room for seven; eight fit in 64 without spilling.
 template <bool STATS, int TM, int TB>
-__global__ void __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(8, 8))) k_trace_closest(DevScene s, PathBuffers pb, DevCounters *cnt) {
+__global__ void __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(TM == TM_ATRC ? 5 : 8, 8))) k_trace_closest(DevScene s, PathBuffers pb, DevCounters *cnt) {
     const uint32_t n = pb.cnt_in[0];
     const int32_t lb = xcd_block<TB>(n);
     if (lb < 0) return;  // whole block past the queue
@@ -3412,10 +3365,8 @@ void launch_raygen(const DevScene &s, const RenderConst &rc, const PathBuffers &
                 if (s.bvh4_large_stack) AGX_LAUNCH_TM(K, TM_B4W_LARGE, 256, grid, st, __VA_ARGS__);\
                 else AGX_LAUNCH_TM(K, TM_B4W_SMALL, 256, grid, st, __VA_ARGS__);                  \
             }                                                                                     \
-        } else if (s.lds_stack) {                                                                 \
-            AGX_LAUNCH_TM(K, TM_ATRC_LDS, 256, grid, st, __VA_ARGS__);                            \
         } else {                                                                                  \
-            AGX_LAUNCH_TM(K, TM_ATRC_PRIV, 256, grid, st, __VA_ARGS__);                           \
+            AGX_LAUNCH_TM(K, TM_ATRC, 256, grid, st, __VA_ARGS__);                                \
         }                                                                                         \
     } while (0)
 
