@@ -418,8 +418,8 @@ __device__ __forceinline__ bool tlas_box(float4 lo, float4 hi, V o, V inv, float
 //
 // The lanes of a wave meet different entities after different numbers of
 // steps.  The outer loop takes every lane to its next mesh (or its end); the inner loop
-// steps through the meshes until fewer than half of those lanes are still inside one,
-// so that a lane waits for at most the slower half of its wave.
+// steps through the meshes until fewer than an eighth of those lanes are still inside
+// one (400x300x8: 4.50 ms at an eighth, 4.57 at a quarter, 4.73 at a half, 5.09 at three quarters).
 template <bool STATS, int TB, bool ANY>
 __device__ bool scene_query(const DevScene &s, V o, V d, float tmin, float tmax, HitRec *h, Counts &c, uint2 *ring) {
     uint2 spill[ATRC_SPILL];
@@ -517,7 +517,7 @@ __device__ bool scene_query(const DevScene &s, V o, V d, float tmin, float tmax,
                 inside = sp != bottom;
                 if (inside) n = unpack_blas(ring_pop<ATRC_RING, TB>(ring, spill, sp));
             }
-        } while (inside && 2 * __popcll(__ballot(inside)) >= lanes);
+        } while (inside && 8 * __popcll(__ballot(inside)) >= lanes);
     }
 }
 
@@ -670,11 +670,12 @@ __device__ __forceinline__ bool b4_inline_quad(float4 p1) {
 // Closest hit over the BVH4: children visited near-first, pending children
 // kept with their entry distance and skipped once a closer hit is known.
 // ring = this lane's column of a [BVH4_RING_CLOSEST][TB] LDS array.  The state
-// of one lane's traversal: start() takes a ray, step() does one node visit, or
-// one leaf and the pops that follow it, and returns true once the traversal is
-// over (hit() then tells whether it found a hit, rec the hit).  The stack
-// entries below the ring live in the caller's spill array (a separate local,
-// so that the state itself stays in registers).
+// of one lane's traversal: start() takes a ray, node_step() visits an interior
+// node, leaf_step() tests a leaf, each with the pops that follow, and they return
+// true once the traversal is over (hit() then tells whether it found a hit, rec
+// the hit); b4_run drives them.  The stack entries below the ring live in the
+// caller's spill array (a separate local, so that the state itself stays in
+// registers).
 template <bool STATS, int CAP, bool WT, int TB>
 struct B4Closest {
     static constexpr int SPILL = CAP - BVH4_RING_CLOSEST;  // (node code, entry distance bits)
@@ -696,107 +697,118 @@ struct B4Closest {
     }
     __device__ __forceinline__ bool hit() const { return best_rank >= 0; }
 
-    // The first step, with the root node's rows already loaded (the root is
-    // always an interior node): its entered children are pushed farthest
-    // first and the nearest becomes the current node.  True if the ray enters
-    // none (the traversal is over).
-    __device__ __forceinline__ bool visit_root(const B4Node &root, Counts &c, uint2 *ring, uint2 (&spill)[SPILL]) {
+    __device__ __forceinline__ bool at_leaf() const { return (code & BVH4_LEAF) != 0; }
+
+    // Visit of an interior node whose rows are loaded: its entered children are
+    // pushed farthest first and the nearest becomes the current node (true), or
+    // none is entered (false: the caller pops).
+    __device__ __forceinline__ bool visit(const B4Node &nd, Counts &c, uint2 *ring, uint2 (&spill)[SPILL]) {
         if (STATS) c.visits++;
         float t[4];
         uint32_t k[4];
-        b4_children(root, r, tmin, tmax, t, k);
+        b4_children(nd, r, tmin, tmax, t, k);
         cswap(t, k, 0, 1); cswap(t, k, 2, 3); cswap(t, k, 0, 2); cswap(t, k, 1, 3); cswap(t, k, 1, 2);
-        if (t[0] == INF_F) return true;
-        if (t[3] != INF_F)
+        if (t[0] == INF_F) return false;
+        if (t[3] != INF_F && sp < CAP)
             ring_push<BVH4_RING_CLOSEST, TB>(ring, spill, sp, make_uint2(k[3], __float_as_uint(t[3])));
-        if (t[2] != INF_F)
+        if (t[2] != INF_F && sp < CAP)
             ring_push<BVH4_RING_CLOSEST, TB>(ring, spill, sp, make_uint2(k[2], __float_as_uint(t[2])));
-        if (t[1] != INF_F)
+        if (t[1] != INF_F && sp < CAP)
             ring_push<BVH4_RING_CLOSEST, TB>(ring, spill, sp, make_uint2(k[1], __float_as_uint(t[1])));
         code = k[0];
-        return false;
+        return true;
     }
-
-    __device__ __forceinline__ bool step(const DevScene &s, Counts &c, uint2 *ring, uint2 (&spill)[SPILL]) {
-        const float4 *N = reinterpret_cast<const float4 *>(s.b4_nodes);
-        const float4 *P = reinterpret_cast<const float4 *>(s.b4_prims);
-        if (!(code & BVH4_LEAF)) {
-            if (STATS) c.visits++;
-            float t[4];
-            uint32_t k[4];
-            b4_children(b4_load(N + size_t(code) * BVH4_NODE_VEC4), r, tmin, tmax, t, k);
-            cswap(t, k, 0, 1); cswap(t, k, 2, 3); cswap(t, k, 0, 2); cswap(t, k, 1, 3); cswap(t, k, 1, 2);
-            if (t[0] != INF_F) {
-                if (t[3] != INF_F && sp < CAP)
-                    ring_push<BVH4_RING_CLOSEST, TB>(ring, spill, sp, make_uint2(k[3], __float_as_uint(t[3])));
-                if (t[2] != INF_F && sp < CAP)
-                    ring_push<BVH4_RING_CLOSEST, TB>(ring, spill, sp, make_uint2(k[2], __float_as_uint(t[2])));
-                if (t[1] != INF_F && sp < CAP)
-                    ring_push<BVH4_RING_CLOSEST, TB>(ring, spill, sp, make_uint2(k[1], __float_as_uint(t[1])));
-                code = k[0];
-                return false;
-            }
-        } else {
-            const uint32_t first = code & BVH4_FIRST_MASK, cnt = ((code >> 27) & 15u) + 1;
-            for (uint32_t i = first; i < first + cnt; ++i) {
-                // the record's three rows in flight together (the third does not
-                // wait for the slot test: every kind of record uses it)
-                const float4 p0 = P[3 * size_t(i)], p1 = P[3 * size_t(i) + 1], p2 = P[3 * size_t(i) + 2];
-                const int32_t ent = __float_as_int(p0.w);
-                const uint32_t slot = __float_as_uint(p1.w);
-                const bool quad = !WT && b4_inline_quad(p1);
-                if (slot < BVH4_QUAD_ACD || (WT && slot != BVH4_ANALYTIC) || quad) {
-                    // a mesh triangle, a quad (its first triangle, then its second), or
-                    // (watertight mode) one triangle of a quad
-                    if (STATS) c.tests++;
-                    const int32_t rank = __float_as_int(p2.w);
-                    int32_t prim = (WT && slot >= BVH4_QUAD_ACD) ? (slot == BVH4_QUAD_ABC ? 0 : 1) : int32_t(slot);
-                    float tt, uu, vv;
-                    bool hit_tri;
-                    if (WT) {
-                        hit_tri = wt_test(wr, mk(p0), mk(p1), mk(p2), tmin, tmax, &tt, &uu, &vv);
-                    } else {
-                        // a quad of a lower-ranked entity must hit strictly closer: its tests run
-                        // against the next float below the current hit distance
-                        const float lim = quad && rank < best_rank ? __uint_as_float(__float_as_uint(tmax) - 1u) : tmax;
-                        hit_tri = mt_closest(r.o, d, tmin, lim, mk(p0), mk(p1), mk(p2), &tt, &uu, &vv);
-                        if (quad) {
-                            prim = 0;
-                            if (!hit_tri) {
-                                if (STATS) c.tests++;
-                                hit_tri = mt_closest(r.o, d, tmin, lim, mk(p0), mk(p2), mk(s.ents[ent].d_a), &tt, &uu, &vv);
-                                prim = 1;
-                            }
-                        }
-                    }
-                    // an exact tie with another entity's hit goes to the entity that
-                    // Atrc's aggregate tests later (its tie rank)
-                    if (hit_tri && (tt < tmax || ent == rec.ent || rank > best_rank)) {
-                        tmax = tt;
-                        rec.t = tt; rec.u = uu; rec.v = vv; rec.ent = ent;
-                        rec.prim = prim;
-                        best_rank = rank;
-                    }
-                } else {
-                    // a lower-ranked entity must hit strictly closer: its test runs
-                    // against the next float below the current hit distance
-                    const int32_t rank = __float_as_int(p2.w);
-                    float tb = rank < best_rank ? __uint_as_float(__float_as_uint(tmax) - 1u) : tmax;
-                    if (analytic_closest<STATS>(s.ents[ent], ent, r.o, d, tmin, &tb, &rec, c)) {
-                        tmax = tb;
-                        best_rank = rank;
-                    }
-                }
-            }
-        }
-        // next pending child that may still hold a closer hit
+    // the next pending child that may still hold a closer hit; true once none is left
+    __device__ __forceinline__ bool pop_next(uint2 *ring, uint2 (&spill)[SPILL]) {
         for (;;) {
             if (sp == 0) return true;
             const uint2 e = ring_pop<BVH4_RING_CLOSEST, TB>(ring, spill, sp);
             if (__uint_as_float(e.y) <= tmax) { code = e.x; return false; }
         }
     }
+    __device__ __forceinline__ bool node_step(const DevScene &s, Counts &c, uint2 *ring, uint2 (&spill)[SPILL]) {
+        const float4 *N = reinterpret_cast<const float4 *>(s.b4_nodes);
+        if (visit(b4_load(N + size_t(code) * BVH4_NODE_VEC4), c, ring, spill)) return false;
+        return pop_next(ring, spill);
+    }
+    __device__ __forceinline__ bool leaf_step(const DevScene &s, Counts &c, uint2 *ring, uint2 (&spill)[SPILL]) {
+        const float4 *P = reinterpret_cast<const float4 *>(s.b4_prims);
+        const uint32_t first = code & BVH4_FIRST_MASK, cnt = ((code >> 27) & 15u) + 1;
+        for (uint32_t i = first; i < first + cnt; ++i) {
+            // the record's three rows in flight together (the third does not
+            // wait for the slot test: every kind of record uses it)
+            const float4 p0 = P[3 * size_t(i)], p1 = P[3 * size_t(i) + 1], p2 = P[3 * size_t(i) + 2];
+            const int32_t ent = __float_as_int(p0.w);
+            const uint32_t slot = __float_as_uint(p1.w);
+            const bool quad = !WT && b4_inline_quad(p1);
+            if (slot < BVH4_QUAD_ACD || (WT && slot != BVH4_ANALYTIC) || quad) {
+                // a mesh triangle, a quad (its first triangle, then its second), or
+                // (watertight mode) one triangle of a quad
+                if (STATS) c.tests++;
+                const int32_t rank = __float_as_int(p2.w);
+                int32_t prim = (WT && slot >= BVH4_QUAD_ACD) ? (slot == BVH4_QUAD_ABC ? 0 : 1) : int32_t(slot);
+                float tt, uu, vv;
+                bool hit_tri;
+                if (WT) {
+                    hit_tri = wt_test(wr, mk(p0), mk(p1), mk(p2), tmin, tmax, &tt, &uu, &vv);
+                } else {
+                    // a quad of a lower-ranked entity must hit strictly closer: its tests run
+                    // against the next float below the current hit distance
+                    const float lim = quad && rank < best_rank ? __uint_as_float(__float_as_uint(tmax) - 1u) : tmax;
+                    hit_tri = mt_closest(r.o, d, tmin, lim, mk(p0), mk(p1), mk(p2), &tt, &uu, &vv);
+                    if (quad) {
+                        prim = 0;
+                        if (!hit_tri) {
+                            if (STATS) c.tests++;
+                            hit_tri = mt_closest(r.o, d, tmin, lim, mk(p0), mk(p2), mk(s.ents[ent].d_a), &tt, &uu, &vv);
+                            prim = 1;
+                        }
+                    }
+                }
+                // an exact tie with another entity's hit goes to the entity that
+                // Atrc's aggregate tests later (its tie rank)
+                if (hit_tri && (tt < tmax || ent == rec.ent || rank > best_rank)) {
+                    tmax = tt;
+                    rec.t = tt; rec.u = uu; rec.v = vv; rec.ent = ent;
+                    rec.prim = prim;
+                    best_rank = rank;
+                }
+            } else {
+                // a lower-ranked entity must hit strictly closer: its test runs
+                // against the next float below the current hit distance
+                const int32_t rank = __float_as_int(p2.w);
+                float tb = rank < best_rank ? __uint_as_float(__float_as_uint(tmax) - 1u) : tmax;
+                if (analytic_closest<STATS>(s.ents[ent], ent, r.o, d, tmin, &tb, &rec, c)) {
+                    tmax = tb;
+                    best_rank = rank;
+                }
+            }
+        }
+        return pop_next(ring, spill);
+    }
 };
+
+// The rest of a traversal (done = it is over already).  A wave whose lanes are
+// at nodes and at leaves would run both codes, one after the other, at every
+// step: instead the lanes at nodes go on until fewer than half of the wave's
+// live lanes are at one, then every lane at a leaf tests it.  Both limits were
+// timed: to the last lane at a node is slower than step by step on the
+// 1M-triangle frame, a half is best there, and rooms gain 13 % at any limit from a
+// half to an eighth (1920x1080x64 116.3 -> 113.7 ms, door-gap room guided training
+// 36.2 -> 31.3 ms, fog 53.6 -> 49.9 ms, Cornell-like 1.74 -> 1.63 ms).
+template <class Q, class Ring, class Spill>
+__device__ __forceinline__ void b4_run(Q &q, bool done, const DevScene &s, Counts &c, Ring *ring, Spill &spill) {
+    while (!done) {
+        const int live = __popcll(__ballot(true));
+        bool go = !q.at_leaf();
+        while (go) {
+            done = q.node_step(s, c, ring, spill);
+            go = !done && !q.at_leaf();
+            if (2 * __popcll(__ballot(go)) < live) go = false;
+        }
+        if (!done && q.at_leaf()) done = q.leaf_step(s, c, ring, spill);
+    }
+}
 
 template <bool STATS, int CAP, bool WT, int TB>
 __device__ bool b4_closest(const DevScene &s, V o, V d, float tmin, float tmax, HitRec *h, Counts &c,
@@ -805,16 +817,13 @@ __device__ bool b4_closest(const DevScene &s, V o, V d, float tmin, float tmax, 
     uint2 spill[B4Closest<STATS, CAP, WT, TB>::SPILL];
     q.start(o, d, tmin, tmax);
     q.rec = *h;
-    while (!q.step(s, c, ring, spill)) {
-    }
+    b4_run(q, false, s, c, ring, spill);
     *h = q.rec;
     return q.hit();
 }
 
 // Any hit over the BVH4; ring = this lane's column of a [BVH4_RING_ANY][TB]
-// LDS array.  The same shape as B4Closest: step() does one node visit, or one
-// leaf and the pop after it, and returns true once the traversal is over
-// (occluded then tells whether it found a hit).
+// LDS array.  The same shape as B4Closest (occluded tells whether it found a hit).
 template <bool STATS, int CAP, bool WT, int TB>
 struct B4Any {
     static constexpr int SPILL = CAP - BVH4_RING_ANY;
@@ -832,6 +841,8 @@ struct B4Any {
         if (WT) wr = wt_ray(o_, d_);
         code = 0; sp = 0; occluded = false;
     }
+
+    __device__ __forceinline__ bool at_leaf() const { return (code & BVH4_LEAF) != 0; }
 
     // Visit of an interior node whose rows are loaded: the first child the ray
     // enters becomes the current node and the others are pushed (true), or
@@ -858,38 +869,38 @@ struct B4Any {
         return false;
     }
 
-    __device__ __forceinline__ bool step(const DevScene &s, Counts &c, uint32_t *ring, uint32_t (&spill)[SPILL]) {
+    __device__ __forceinline__ bool node_step(const DevScene &s, Counts &c, uint32_t *ring, uint32_t (&spill)[SPILL]) {
         const float4 *N = reinterpret_cast<const float4 *>(s.b4_nodes);
+        if (visit(b4_load(N + size_t(code) * BVH4_NODE_VEC4), c, ring, spill)) return false;
+        return pop_next(ring, spill);
+    }
+    __device__ __forceinline__ bool leaf_step(const DevScene &s, Counts &c, uint32_t *ring, uint32_t (&spill)[SPILL]) {
         const float4 *P = reinterpret_cast<const float4 *>(s.b4_prims);
-        if (!(code & BVH4_LEAF)) {
-            if (visit(b4_load(N + size_t(code) * BVH4_NODE_VEC4), c, ring, spill)) return false;
-        } else {
-            const uint32_t first = code & BVH4_FIRST_MASK, cnt = ((code >> 27) & 15u) + 1;
-            for (uint32_t i = first; i < first + cnt; ++i) {
-                // the third row is loaded with the others (analytic records
-                // leave it unused; triangles need it)
-                const float4 p0 = P[3 * size_t(i)], p1 = P[3 * size_t(i) + 1], p2 = P[3 * size_t(i) + 2];
-                const uint32_t slot = __float_as_uint(p1.w);
-                const bool quad = !WT && b4_inline_quad(p1);
-                if (slot < BVH4_QUAD_ACD || (WT && slot != BVH4_ANALYTIC) || quad) {
-                    if (STATS) c.tests++;
-                    if (WT) {
-                        float tt, uu, vv;
-                        if (wt_test(wr, mk(p0), mk(p1), mk(p2), tmin, tmax, &tt, &uu, &vv)) { occluded = true; return true; }
-                    } else if (mt_any(r.o, d, tmin, tmax, mk(p0), mk(p1), mk(p2))) {
-                        occluded = true;
-                        return true;
-                    } else if (quad) {
-                        if (STATS) c.tests++;
-                        if (mt_any(r.o, d, tmin, tmax, mk(p0), mk(p2), mk(s.ents[__float_as_int(p0.w)].d_a))) {
-                            occluded = true;
-                            return true;
-                        }
-                    }
-                } else if (analytic_any<STATS>(s.ents[__float_as_int(p0.w)], r.o, d, tmin, tmax, c)) {
+        const uint32_t first = code & BVH4_FIRST_MASK, cnt = ((code >> 27) & 15u) + 1;
+        for (uint32_t i = first; i < first + cnt; ++i) {
+            // the third row is loaded with the others (analytic records
+            // leave it unused; triangles need it)
+            const float4 p0 = P[3 * size_t(i)], p1 = P[3 * size_t(i) + 1], p2 = P[3 * size_t(i) + 2];
+            const uint32_t slot = __float_as_uint(p1.w);
+            const bool quad = !WT && b4_inline_quad(p1);
+            if (slot < BVH4_QUAD_ACD || (WT && slot != BVH4_ANALYTIC) || quad) {
+                if (STATS) c.tests++;
+                if (WT) {
+                    float tt, uu, vv;
+                    if (wt_test(wr, mk(p0), mk(p1), mk(p2), tmin, tmax, &tt, &uu, &vv)) { occluded = true; return true; }
+                } else if (mt_any(r.o, d, tmin, tmax, mk(p0), mk(p1), mk(p2))) {
                     occluded = true;
                     return true;
+                } else if (quad) {
+                    if (STATS) c.tests++;
+                    if (mt_any(r.o, d, tmin, tmax, mk(p0), mk(p2), mk(s.ents[__float_as_int(p0.w)].d_a))) {
+                        occluded = true;
+                        return true;
+                    }
                 }
+            } else if (analytic_any<STATS>(s.ents[__float_as_int(p0.w)], r.o, d, tmin, tmax, c)) {
+                occluded = true;
+                return true;
             }
         }
         return pop_next(ring, spill);
@@ -901,8 +912,7 @@ __device__ bool b4_any(const DevScene &s, V o, V d, float tmin, float tmax, Coun
     B4Any<STATS, CAP, WT, TB> q;
     uint32_t spill[B4Any<STATS, CAP, WT, TB>::SPILL];
     q.start(o, d, tmin, tmax);
-    while (!q.step(s, c, ring, spill)) {
-    }
+    b4_run(q, false, s, c, ring, spill);
     return q.occluded;
 }
 
@@ -1796,9 +1806,7 @@ __global__ void __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(TM == T
             Q q;
             uint2 spill[Q::SPILL];
             q.start(mk(o4), mk(d4), o4.w, d4.w);
-            if (!q.visit_root(root, c, ring, spill))
-                while (!q.step(s, c, ring, spill)) {
-                }
+            b4_run(q, q.visit(root, c, ring, spill) ? false : q.pop_next(ring, spill), s, c, ring, spill);
             found = q.hit();
             pb.hit[ri] = make_float4(q.rec.t, q.rec.u, q.rec.v, __int_as_float(found ? q.rec.ent : -1));
             pb.hit_prim[ri] = q.rec.prim;
@@ -1839,8 +1847,7 @@ __global__ void __launch_bounds__(TB) k_trace_shadow(DevScene s, PathBuffers pb,
             Q q;
             uint32_t spill[Q::SPILL];
             q.start(mk(o4), mk(d4), d4.w, o4.w);
-            bool done = q.visit(root, c, ring, spill) ? false : q.pop_next(ring, spill);
-            while (!done) done = q.step(s, c, ring, spill);
+            b4_run(q, q.visit(root, c, ring, spill) ? false : q.pop_next(ring, spill), s, c, ring, spill);
             occ = q.occluded;
             pb.occluded[ri] = occ ? 1 : 0;
         }
