@@ -796,10 +796,14 @@ struct B4Closest {
 // 1M-triangle frame, a half is best there, and rooms gain 13 % at any limit from a
 // half to an eighth (1920x1080x64 116.3 -> 113.7 ms, door-gap room guided training
 // 36.2 -> 31.3 ms, fog 53.6 -> 49.9 ms, Cornell-like 1.74 -> 1.63 ms).
-template <class Q, class Ring, class Spill>
-__device__ __forceinline__ void b4_run(Q &q, bool done, const DevScene &s, Counts &c, Ring *ring, Spill &spill) {
+// RUNS: returns early, with lanes' traversals unfinished, once at most `few` of
+// the wave's lanes are live; the result is done of each lane.
+template <bool RUNS, class Q, class Ring, class Spill>
+__device__ __forceinline__ bool b4_run(Q &q, bool done, const DevScene &s, Counts &c, Ring *ring, Spill &spill,
+                                       int few = 0) {
     while (!done) {
         const int live = __popcll(__ballot(true));
+        if (RUNS && live <= few) break;
         bool go = !q.at_leaf();
         while (go) {
             done = q.node_step(s, c, ring, spill);
@@ -808,6 +812,7 @@ __device__ __forceinline__ void b4_run(Q &q, bool done, const DevScene &s, Count
         }
         if (!done && q.at_leaf()) done = q.leaf_step(s, c, ring, spill);
     }
+    return done;
 }
 
 template <bool STATS, int CAP, bool WT, int TB>
@@ -817,7 +822,7 @@ __device__ bool b4_closest(const DevScene &s, V o, V d, float tmin, float tmax, 
     uint2 spill[B4Closest<STATS, CAP, WT, TB>::SPILL];
     q.start(o, d, tmin, tmax);
     q.rec = *h;
-    b4_run(q, false, s, c, ring, spill);
+    b4_run<false>(q, false, s, c, ring, spill);
     *h = q.rec;
     return q.hit();
 }
@@ -912,7 +917,7 @@ __device__ bool b4_any(const DevScene &s, V o, V d, float tmin, float tmax, Coun
     B4Any<STATS, CAP, WT, TB> q;
     uint32_t spill[B4Any<STATS, CAP, WT, TB>::SPILL];
     q.start(o, d, tmin, tmax);
-    b4_run(q, false, s, c, ring, spill);
+    b4_run<false>(q, false, s, c, ring, spill);
     return q.occluded;
 }
 
@@ -1750,8 +1755,8 @@ __device__ BSmp bsdf_sample(const Bsdf &b, V wo, float su, float sv, float sw, f
 }
 
 // ---------------------------------------------------------------- wave-level counter reduction
-__device__ __forceinline__ void flush_counts(const Counts &c, bool ok, DevCounters *cnt) {
-    uint32_t v = c.visits, t = c.tests, h = ok ? 1u : 0u;
+__device__ __forceinline__ void flush_counts(const Counts &c, uint32_t hits, DevCounters *cnt) {
+    uint32_t v = c.visits, t = c.tests, h = hits;
     for (int off = 32; off > 0; off >>= 1) {
         v += __shfl_xor(v, off);
         t += __shfl_xor(t, off);
@@ -1806,7 +1811,7 @@ __global__ void __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(TM == T
             Q q;
             uint2 spill[Q::SPILL];
             q.start(mk(o4), mk(d4), o4.w, d4.w);
-            b4_run(q, q.visit(root, c, ring, spill) ? false : q.pop_next(ring, spill), s, c, ring, spill);
+            b4_run<false>(q, q.visit(root, c, ring, spill) ? false : q.pop_next(ring, spill), s, c, ring, spill);
             found = q.hit();
             pb.hit[ri] = make_float4(q.rec.t, q.rec.u, q.rec.v, __int_as_float(found ? q.rec.ent : -1));
             pb.hit_prim[ri] = q.rec.prim;
@@ -1821,7 +1826,7 @@ __global__ void __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(TM == T
         pb.hit[ri] = make_float4(h.t, h.u, h.v, __int_as_float(h.ent));
         pb.hit_prim[ri] = h.prim;
     }
-    if (STATS) flush_counts(c, found, cnt);
+    if (STATS) flush_counts(c, found ? 1u : 0u, cnt);
 }
 
 template <bool STATS, int TM, int TB>
@@ -1847,7 +1852,7 @@ __global__ void __launch_bounds__(TB) k_trace_shadow(DevScene s, PathBuffers pb,
             Q q;
             uint32_t spill[Q::SPILL];
             q.start(mk(o4), mk(d4), d4.w, o4.w);
-            b4_run(q, q.visit(root, c, ring, spill) ? false : q.pop_next(ring, spill), s, c, ring, spill);
+            b4_run<false>(q, q.visit(root, c, ring, spill) ? false : q.pop_next(ring, spill), s, c, ring, spill);
             occ = q.occluded;
             pb.occluded[ri] = occ ? 1 : 0;
         }
@@ -1857,7 +1862,118 @@ __global__ void __launch_bounds__(TB) k_trace_shadow(DevScene s, PathBuffers pb,
         occ = query_any<STATS, TM, TB>(s, mk(o4), mk(d4), d4.w, o4.w, c, lds_col);
         pb.occluded[ri] = occ ? 1 : 0;
     }
-    if (STATS) flush_counts(c, false, cnt);
+    if (STATS) flush_counts(c, 0u, cnt);
+}
+
+// Large BVH4 queues: a wave takes a run of 64 to 512 consecutive rays and gives
+// its idle lanes the run's next ones whenever at least REFILL_IDLE lanes have
+// finished (or all have).  With one ray a lane, a wave lasts as long as its
+// longest ray: on the 1M-triangle frame 14 of 64 lanes took part in the average vector instruction,
+// and these kernels are bound by those.  The run is the wave's own, so nothing
+// is shared: no atomics, and rays stay in queue order within a wave.  A new ray
+// starts at the root like any lane at a node, so its first visit runs with the
+// others' (a root visit of its own for the few new lanes cost 4 ms a frame).  The state
+// needs 77 registers against 64: six waves per SIMD, with no spill.
+// Runs of n / 2^19 rounds (at most 8) keep several waves for every slot of the chip; queues of
+// less than REFILL_MIN rays would leave slots empty while long runs end, and take
+// one ray a lane at eight waves.  1M-triangle 1920x1080x64 frame: closest hit 46.1 ->
+// 37.3 ms, any hit 19.9 -> 17.0; fog room 1024x1024x4: 20.9 -> 16.7 and 5.6 -> 5.0 (17.2 and 5.6
+// with runs only from 2^22 rays).  Refilling at 16 idle lanes is the same
+// within 0.4 ms, at 48 it costs 1.4.
+constexpr int REFILL_IDLE = 24;
+constexpr uint32_t REFILL_MIN = 1u << 21;
+constexpr unsigned REFILL_BLOCK = 128;
+__device__ __forceinline__ uint32_t refill_run(uint32_t n) { return 64u * min(8u, max(1u, n >> 19)); }
+
+// this wave's part [*first, *last) of a queue of n rays (empty past the queue);
+// blocks are mapped to the XCDs as xcd_block does
+__device__ __forceinline__ void refill_range(uint32_t n, uint32_t *first, uint32_t *last) {
+    const uint32_t run = refill_run(n);
+    const int32_t lb = xcd_block<REFILL_BLOCK>((n + run - 1) / run * 64u);
+    *first = *last = 0;
+    if (lb < 0) return;
+    const uint32_t w = __builtin_amdgcn_readfirstlane(uint32_t(lb) * (REFILL_BLOCK / 64) + (threadIdx.x >> 6));
+    *first = min(n, w * run);
+    *last = min(n, *first + run);
+}
+
+// Traverses the rays [next, last) of the wave: load(i, q) starts traversal q on
+// ray i, store(i, q) takes its result.  Every turn of the loop either starts rays of the
+// run, which is finite, or ends every traversal in flight.
+template <class Q, class Ring, class Spill, class Load, class Store>
+__device__ __forceinline__ void refill_traverse(uint32_t next, uint32_t last, const DevScene &s, Counts &c, Ring *ring,
+                                                Spill &spill, Load load, Store store) {
+    Q q;
+    const uint32_t lane = __lane_id();
+    uint32_t ray = 0;
+    bool done = true, own = false;
+    while (next < last || __ballot(!done)) {
+        const unsigned long long idle = __ballot(done);
+        if (done && own) {
+            store(ray, q);
+            own = false;
+        }
+        if (next < last) {
+            const uint32_t i = next + uint32_t(__popcll(idle & ((1ull << lane) - 1ull)));
+            if (done && i < last) {
+                ray = load(i, q);
+                done = false;
+                own = true;
+            }
+            next += uint32_t(__popcll(idle));
+        }
+        done = b4_run<true>(q, done, s, c, ring, spill, next < last ? 64 - REFILL_IDLE : 0);
+    }
+    if (own) store(ray, q);
+}
+
+template <bool STATS, int TM, int TB>
+__global__ void __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(6, 8))) k_trace_closest_runs(DevScene s, PathBuffers pb, DevCounters *cnt) {
+    uint32_t next, last;
+    refill_range(pb.cnt_in[0], &next, &last);
+    if (next >= last) return;
+    AGX_LDS_COLUMN(TM, TB);
+    constexpr int CAP = (TM == TM_B4_LARGE || TM == TM_B4W_LARGE) ? BVH4_STACK_LARGE : BVH4_STACK_SMALL;
+    using Q = B4Closest<STATS, CAP, TM == TM_B4W_SMALL || TM == TM_B4W_LARGE, TB>;
+    uint2 spill[Q::SPILL];
+    Counts c;
+    uint32_t hits = 0;
+    refill_traverse<Q>(
+        next, last, s, c, reinterpret_cast<uint2 *>(lds_col) + threadIdx.x, spill,
+        [&](uint32_t i, Q &q) {
+            const uint32_t ri = pb.q_closest[i];
+            const float4 o4 = pb.ray_o[ri], d4 = pb.ray_d[ri];
+            q.start(mk(o4), mk(d4), o4.w, d4.w);
+            return ri;
+        },
+        [&](uint32_t ri, const Q &q) {
+            if (STATS) hits += q.hit() ? 1u : 0u;
+            pb.hit[ri] = make_float4(q.rec.t, q.rec.u, q.rec.v, __int_as_float(q.hit() ? q.rec.ent : -1));
+            pb.hit_prim[ri] = q.rec.prim;
+        });
+    if (STATS) flush_counts(c, hits, cnt);
+}
+
+template <bool STATS, int TM, int TB>
+__global__ void __launch_bounds__(TB) k_trace_shadow_runs(DevScene s, PathBuffers pb, DevCounters *cnt) {
+    uint32_t next, last;
+    refill_range(pb.cnt_in[1], &next, &last);
+    if (next >= last) return;
+    AGX_LDS_COLUMN(TM, TB);
+    constexpr int CAP = (TM == TM_B4_LARGE || TM == TM_B4W_LARGE) ? BVH4_STACK_LARGE : BVH4_STACK_SMALL;
+    using Q = B4Any<STATS, CAP, TM == TM_B4W_SMALL || TM == TM_B4W_LARGE, TB>;
+    uint32_t spill[Q::SPILL];
+    Counts c;
+    refill_traverse<Q>(
+        next, last, s, c, lds_col + threadIdx.x, spill,
+        [&](uint32_t i, Q &q) {
+            const uint32_t ri = pb.q_shadow[i];
+            const float4 o4 = pb.sh_o[ri], d4 = pb.sh_d[ri];
+            q.start(mk(o4), mk(d4), d4.w, o4.w);
+            return ri;
+        },
+        [&](uint32_t ri, const Q &q) { pb.occluded[ri] = q.occluded ? 1 : 0; });
+    if (STATS) flush_counts(c, 0u, cnt);
 }
 
 __global__ void __launch_bounds__(256) k_raygen(DevScene s, RenderConst rc, PathBuffers pb) {
@@ -3305,7 +3421,7 @@ __global__ void __launch_bounds__(TB) k_trace_rays(DevScene s, const float4 *o, 
             }
         }
     }
-    if (STATS) flush_counts(c, found, cnt);
+    if (STATS) flush_counts(c, found ? 1u : 0u, cnt);
 }
 
 // Copies the rays of the current closest-hit (which = 0) or any-hit (1) queue,
@@ -3383,15 +3499,45 @@ inline unsigned trace_block_of(const DevScene &s) {
     return (b4 && s.trace_block == 128) ? 128u : TRACE_BLOCK;
 }
 
+// the run kernels for queues that may hold REFILL_MIN rays (BVH4 modes)
+#define AGX_LAUNCH_RUNS(K, grid, st, ...)                                                         \
+    do {                                                                                          \
+        if (s.accel == AGX_ACCEL_BVH4) {                                                          \
+            if (s.bvh4_large_stack) AGX_LAUNCH_TM(K, TM_B4_LARGE, REFILL_BLOCK, grid, st, __VA_ARGS__); \
+            else AGX_LAUNCH_TM(K, TM_B4_SMALL, REFILL_BLOCK, grid, st, __VA_ARGS__);              \
+        } else {                                                                                  \
+            if (s.bvh4_large_stack) AGX_LAUNCH_TM(K, TM_B4W_LARGE, REFILL_BLOCK, grid, st, __VA_ARGS__); \
+            else AGX_LAUNCH_TM(K, TM_B4W_SMALL, REFILL_BLOCK, grid, st, __VA_ARGS__);             \
+        }                                                                                         \
+    } while (0)
+// Blocks for any queue of n <= max_n rays: it has ceil(n / refill_run(n)) waves, at
+// most 2^14 while runs grow with n (2 x 2^19 / 64, just below the second round)
+// and n / 512 once they are longest; xcd_block wants 7 blocks more
+inline unsigned runs_grid(uint32_t max_n) {
+    const uint32_t waves = std::max(1u << 14, (max_n + 511u) / 512u);
+    return (waves + REFILL_BLOCK / 64 - 1) / (REFILL_BLOCK / 64) + 8;
+}
+inline bool use_runs(const DevScene &s, uint32_t max_n) {
+    return (s.accel == AGX_ACCEL_BVH4 || s.accel == AGX_ACCEL_BVH4_WATERTIGHT) && max_n >= REFILL_MIN;
+}
+
 void launch_trace_closest(const DevScene &s, const PathBuffers &pb, uint32_t max_n, bool stats, DevCounters *cnt,
                           hipStream_t st) {
     if (!max_n) return;
+    if (use_runs(s, max_n)) {
+        AGX_LAUNCH_RUNS(k_trace_closest_runs, dim3(runs_grid(max_n)), st, s, pb, cnt);
+        return;
+    }
     const unsigned tb = trace_block_of(s);
     AGX_LAUNCH_STACKED(k_trace_closest, tb, dim3(grid_of(max_n, tb) + 7), st, s, pb, cnt);
 }
 void launch_trace_shadow(const DevScene &s, const PathBuffers &pb, uint32_t max_n, bool stats, DevCounters *cnt,
                          hipStream_t st) {
     if (!max_n) return;
+    if (use_runs(s, max_n)) {
+        AGX_LAUNCH_RUNS(k_trace_shadow_runs, dim3(runs_grid(max_n)), st, s, pb, cnt);
+        return;
+    }
     const unsigned tb = trace_block_of(s);
     AGX_LAUNCH_STACKED(k_trace_shadow, tb, dim3(grid_of(max_n, tb) + 7), st, s, pb, cnt);
 }
