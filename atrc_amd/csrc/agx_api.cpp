@@ -591,6 +591,7 @@ int agx_render(agx_ctx *c, const agx_render_params *p, const volatile int32_t *c
     const auto t_call = std::chrono::steady_clock::now();
     RenderConst rc{};
     if (int r0 = fill_render_const(c, p, &rc); r0 != AGX_OK) return r0;
+    rc.aov = albedo || normal || denoise ? 1 : 0;
     const bool guide = p->guide != 0;
     const bool guide_train = guide && p->guide_train != 0;
     const uint32_t guide_batch = p->guide_batch > 0 ? uint32_t(p->guide_batch) : 65536u;
@@ -648,7 +649,7 @@ int agx_render(agx_ctx *c, const agx_render_params *p, const volatile int32_t *c
     st.prim_bytes = 48;
     st.info_bytes = 96;
     if (stats) HIP_TRY(hipMemsetAsync(c->dcnt, 0, 2 * sizeof(DevCounters), c->stream));
-    launch_film_clear(c->pb, wh, c->stream);
+    launch_film_clear(rc, c->pb, wh, c->stream);
     HIP_TRY(hipEventRecord(c->ev[0], c->stream));
     // Timing events: (start, end, kind) per launch group; read after the render.
     struct Timed { size_t a, b; int kind; };
@@ -830,7 +831,7 @@ int agx_render(agx_ctx *c, const agx_render_params *p, const volatile int32_t *c
             c->resolve_cap = size_t(wh);
         }
         float *dout = c->d_resolve, *hout = c->h_resolve;
-        launch_film_resolve(c->pb, wh, dout, dout + 3 * wh, dout + 6 * wh, dout + 9 * wh, c->stream);
+        launch_film_resolve(rc, c->pb, wh, dout, dout + 3 * wh, dout + 6 * wh, dout + 9 * wh, c->stream);
         hipError_t e = hipSuccess;
         struct Plane { float *user; size_t off, n; };
         const Plane planes[4] = {{rgb, 0, 3}, {albedo, 3, 3}, {normal, 6, 3}, {denoise, 9, 1}};
@@ -1098,7 +1099,7 @@ int enqueue_render(agx_ctx *c, const agx_render_params *p, hipStream_t st, unsig
     const int spec = (c->ds.features & SF_DELTA) ? std::max(p->specular_depth, 0) : 0;
     const int max_bounces = p->max_depth + spec + 2;
     PathBuffers pb = c->pb;
-    launch_film_clear(pb, wh, st);
+    launch_film_clear(rc, pb, wh, st);
     for (int64_t base = 0; base < total; base += per_pass) {
         rc.work_base = base;
         rc.n_paths = int32_t(std::min<int64_t>(per_pass, total - base));
@@ -1123,7 +1124,7 @@ int enqueue_render(agx_ctx *c, const agx_render_params *p, hipStream_t st, unsig
         launch_film(rc, pb, st);
     }
     float *dout = c->d_resolve;
-    launch_film_resolve(pb, wh, dout, dout + 3 * wh, dout + 6 * wh, dout + 9 * wh, st);
+    launch_film_resolve(rc, pb, wh, dout, dout + 3 * wh, dout + 6 * wh, dout + 9 * wh, st);
     return AGX_OK;
 }
 

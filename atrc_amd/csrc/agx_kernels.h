@@ -10,8 +10,8 @@ namespace agx {
 // Per-path state (structure of arrays, N = paths in flight).
 struct PathBuffers {
     float4 *coef;        // [N] path throughput
-    float4 *radiance;    // [N] accumulated radiance
-    float4 *gb_albedo;   // [N] (albedo.xyz, denoise)
+    float4 *radiance;    // [N] accumulated radiance (unless PF_DARK)
+    float4 *gb_albedo;   // [N] (albedo.xyz, denoise), with RenderConst::aov
     float4 *gb_normal;   // [N]
     unsigned long long *rng;     // [N] PCG32 state (the increment is derived from the path id)
     unsigned long long *rng_tr;  // [N] second stream: ratio-tracking transmittance draws
@@ -76,6 +76,7 @@ enum : uint32_t {
     PF_MIS_DELTA = 16u,  // the MIS-BSDF sample was a delta lobe
     PF_FRESH = 32u,      // camera path not shaded yet: radiance 0, depth (1, 1, 0, 0) and the
                          // depth-1 throughput are implied (k_raygen does not store them)
+    PF_DARK = 128u,      // the path's radiance is zero (not stored)
     PF_MS = 64u,         // k_media sampled the medium segment before this vertex into g_ms
     PF_MIS_MED_SHIFT = 16u,  // bits 16..31: 1 + medium index the MIS-BSDF ray travels through (0 = void)
 };
@@ -100,7 +101,7 @@ struct RenderConst {
     int32_t guide_record;  // 1: guided vertices of the recording paths keep training records
     uint32_t guide_rec_shift;  // recording paths: (p + guide_rec_rot) % 2^shift == 0, record slot p >> shift
     uint32_t guide_rec_rot;    // varies per pass so that every pixel records in turn
-    int32_t pad2;
+    int32_t aov;           // 1: the caller takes albedo, normal or denoise planes; 0: the image alone
     // wide film filters (box wider than a pixel, Gaussian): every sample splats
     // onto the pixels of its render tile (tile x tile pixels, Atrc's
     // task_grid_size) as Atrc's apply_image_filter reaches them; the sampled
@@ -152,9 +153,9 @@ void launch_copy_calibration(const float4 *src, float4 *dst, uint64_t n, hipStre
 void launch_capture_rays(const PathBuffers &pb, int which, float4 *o, float4 *d, uint32_t *count, uint32_t cap,
                          uint32_t max_n, hipStream_t st);
 void launch_film(const RenderConst &rc, const PathBuffers &pb, hipStream_t st);
-void launch_film_clear(const PathBuffers &pb, int64_t wh, hipStream_t st);
-void launch_film_resolve(const PathBuffers &pb, int64_t wh, float *rgb, float *albedo, float *normal, float *denoise,
-                         hipStream_t st);
+void launch_film_clear(const RenderConst &rc, const PathBuffers &pb, int64_t wh, hipStream_t st);
+void launch_film_resolve(const RenderConst &rc, const PathBuffers &pb, int64_t wh, float *rgb, float *albedo,
+                         float *normal, float *denoise, hipStream_t st);
 // parity hook: rays in device memory, results to device memory
 // Staging of agx_trace_rays_noalloc: a file-scope device array of
 // NOALLOC_MAX_RAYS rays (84 B each: packed rays, raw inputs, outputs) that the

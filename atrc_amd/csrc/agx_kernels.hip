@@ -2052,9 +2052,11 @@ __global__ void __launch_bounds__(256) k_raygen(DevScene s, RenderConst rc, Path
     }
     const bool launch = alive && 1 <= rc.max_depth;
     if (!launch) {  // a launched path gets its G-buffer and radiance from k_shade at depth 1
-        pb.gb_albedo[p] = make_float4(0, 0, 0, 1);
-        pb.gb_normal[p] = make_float4(0, 0, 0, 0);
-        pb.radiance[p] = make_float4(0, 0, 0, 0);
+        if (rc.aov) {
+            pb.gb_albedo[p] = make_float4(0, 0, 0, 1);
+            pb.gb_normal[p] = make_float4(0, 0, 0, 0);
+        }
+        flags |= PF_DARK;
     }
     if (launch) {
         flags |= PF_CONT | PF_FRESH;
@@ -2721,8 +2723,20 @@ __global__ void __launch_bounds__(256) k_guide_features(DevScene s, RenderConst 
     dst[1] = make_float4(x[4], x[5], x[6], x[7]);
 }
 
+// 128-thread blocks: a block's slot is free again when two waves end instead of four,
+// worth 5 % of shading in the lens scene (full variant), 1 % on the 1M-triangle frame
+constexpr unsigned SHADE_BLOCK = 128;
+
+// stores the radiance of path p and returns its flags: most paths have gathered none
+// yet after their first vertex, and a flag says so in place of 16 bytes written here and read at the next vertex
+__device__ __forceinline__ uint32_t put_radiance(const PathBuffers &pb, uint32_t p, V L, uint32_t flags) {
+    if (black(L)) return flags | PF_DARK;
+    pb.radiance[p] = f4(L, 0);
+    return flags & ~PF_DARK;
+}
+
 template <uint32_t F>
-__global__ void __launch_bounds__(256) k_shade(DevScene s, RenderConst rc, PathBuffers pb) {
+__global__ void __launch_bounds__(SHADE_BLOCK) k_shade(DevScene s, RenderConst rc, PathBuffers pb) {
     const uint32_t n = pb.cnt_in[2];
     const uint32_t tid = blockIdx.x * blockDim.x + threadIdx.x;
     if (tid >= n) return;
@@ -2732,7 +2746,7 @@ __global__ void __launch_bounds__(256) k_shade(DevScene s, RenderConst rc, PathB
     // a fresh camera path: nothing stored yet but its flags, rays and stream
     const bool fresh = (flags & PF_FRESH) != 0;
     flags &= ~PF_FRESH;
-    V L = fresh ? mk(0, 0, 0) : mk(pb.radiance[p]);
+    V L = (fresh || (flags & PF_DARK)) ? mk(0, 0, 0) : mk(pb.radiance[p]);
     const bool media = (F & SF_MEDIA) && (s.features & SF_MEDIA);
     Rng rng;
     rng.state = pb.rng[p];
@@ -2777,8 +2791,7 @@ __global__ void __launch_bounds__(256) k_shade(DevScene s, RenderConst rc, PathB
         flags &= (1u << PF_MIS_MED_SHIFT) - 1u;
     }
     if (!(flags & PF_CONT)) {
-        pb.radiance[p] = f4(L, 0);
-        pb.flags[p] = flags;
+        pb.flags[p] = put_radiance(pb, p, L, flags);
         return;
     }
     flags &= ~PF_CONT;
@@ -2800,12 +2813,11 @@ __global__ void __launch_bounds__(256) k_shade(DevScene s, RenderConst rc, PathB
     const V ro = mk(pb.ray_o[2 * p]), rd = mk(pb.ray_d[2 * p]);
     if (ent < 0) {  // path_tracing.cpp:41-49 (trace_nomis, :250-256: at every depth)
         if ((dep.x == 1 || rc.nomis) && s.env_kind != AGX_ENV_NONE) L = L + coef * env_radiance<F>(s, rd);
-        if (dep.x == 1) {  // the camera ray escaped: empty G-buffer (k_raygen leaves it to this branch)
+        if (dep.x == 1 && rc.aov) {  // the camera ray escaped: empty G-buffer (k_raygen leaves it to this branch)
             pb.gb_normal[p] = make_float4(0, 0, 0, 0);
             pb.gb_albedo[p] = make_float4(0, 0, 0, 1);
         }
-        pb.radiance[p] = f4(L, 0);
-        pb.flags[p] = flags;
+        pb.flags[p] = put_radiance(pb, p, L, flags);
         return;
     }
     HitRec h;
@@ -2813,7 +2825,7 @@ __global__ void __launch_bounds__(256) k_shade(DevScene s, RenderConst rc, PathB
     const Surf sp = surface_at(s, h, ro, rd, eps);
     const DevEntity &e = s.ents[ent];
     const Bsdf b = make_bsdf(s.mats[e.material], sp, eps);
-    if (dep.x == 1) {  // :54-60
+    if (dep.x == 1 && rc.aov) {  // :54-60
         pb.gb_normal[p] = f4(sp.user.z, 0);
         pb.gb_albedo[p] = f4(b.albedo, (e.flags & EF_NO_DENOISE) ? 0.0f : 1.0f);
     }
@@ -3063,7 +3075,7 @@ __global__ void __launch_bounds__(256) k_shade(DevScene s, RenderConst rc, PathB
         }
     }
     if (pending) flags |= PF_PENDING;
-    pb.radiance[p] = f4(L, 0);
+    flags = put_radiance(pb, p, L, flags);
     if (cont) flags |= PF_CONT;
     // the rays of this vertex: 2p (PF_CONT), 2p + 1 (PF_MIS) and the shadow rays of
     // the lights in shadow_mask; k_queue_* build the queues from these after the launch
@@ -3304,18 +3316,43 @@ __device__ __forceinline__ void neumaier(float *sum, float *comp, float x) {
     *sum = t;
 }
 
+// Film channels: rgb, and with the caller's planes asked for (AOV) albedo,
+// normal and the denoise weight as well
+template <bool AOV> constexpr int FILM_CH = AOV ? 10 : 3;
+
+// One sample's channels into a pixel's sums
+template <bool AOV>
+__device__ __forceinline__ void film_add(const PathBuffers &pb, int64_t slot, V v, float w, float (&sum)[FILM_CH<AOV>],
+                                         float (&cmp)[FILM_CH<AOV>]) {
+    neumaier(&sum[0], &cmp[0], w * v.x);
+    neumaier(&sum[1], &cmp[1], w * v.y);
+    neumaier(&sum[2], &cmp[2], w * v.z);
+    if constexpr (AOV) {
+        const float4 a = pb.gb_albedo[slot], n = pb.gb_normal[slot];
+        const float vals[7] = {a.x, a.y, a.z, n.x, n.y, n.z, a.w};
+#pragma unroll
+        for (int k = 0; k < 7; ++k) neumaier(&sum[3 + k], &cmp[3 + k], w * vals[k]);
+    }
+}
+__device__ __forceinline__ V film_radiance(const PathBuffers &pb, int64_t slot, uint32_t flags) {
+    return (flags & PF_DARK) ? mk(0, 0, 0) : mk(pb.radiance[slot]);
+}
+__device__ __forceinline__ bool finite3(V v) { return isfinite(v.x) && isfinite(v.y) && isfinite(v.z); }
+
+// The pixel's sums stay in registers over the samples of the pass and are
+// written back once (the same operations in the same order as updates in memory).
+template <bool AOV>
 __global__ void __launch_bounds__(256) k_film(RenderConst rc, PathBuffers pb) {
+    constexpr int CH = FILM_CH<AOV>;
     const int64_t wh = int64_t(rc.W) * rc.H;
     const int64_t cover = rc.n_paths < wh ? int64_t(rc.n_paths) : wh;
     const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (i >= cover) return;
     const int64_t pixel = (rc.work_base + i) % wh;
     const int64_t layers = rc.n_paths >= wh ? int64_t(rc.n_paths) / wh : 1;
-    // the pixel's sums stay in registers over the layers of the pass and are
-    // written back once (same operations in the same order as per-layer updates)
-    float sum[10], cmp[10];
+    float sum[CH], cmp[CH];
 #pragma unroll
-    for (int k = 0; k < 10; ++k) {
+    for (int k = 0; k < CH; ++k) {
         sum[k] = pb.film_sum[k * wh + pixel];
         cmp[k] = pb.film_comp[k * wh + pixel];
     }
@@ -3323,17 +3360,15 @@ __global__ void __launch_bounds__(256) k_film(RenderConst rc, PathBuffers pb) {
     for (int64_t j = 0; j < layers; ++j) {
         const int64_t slot = j * wh + i;
         if (slot >= rc.n_paths) break;
-        if (!(pb.flags[slot] & PF_KEEP)) continue;
-        const float4 v = pb.radiance[slot];
-        if (!(isfinite(v.x) && isfinite(v.y) && isfinite(v.z))) continue;
-        const float4 a = pb.gb_albedo[slot], n = pb.gb_normal[slot];
-        const float vals[10] = {v.x, v.y, v.z, a.x, a.y, a.z, n.x, n.y, n.z, a.w};
-#pragma unroll
-        for (int k = 0; k < 10; ++k) neumaier(&sum[k], &cmp[k], vals[k]);
+        const uint32_t flags = pb.flags[slot];
+        if (!(flags & PF_KEEP)) continue;
+        const V v = film_radiance(pb, slot, flags);
+        if (!finite3(v)) continue;
+        film_add<AOV>(pb, slot, v, 1.0f, sum, cmp);
         count += 1.0f;
     }
 #pragma unroll
-    for (int k = 0; k < 10; ++k) {
+    for (int k = 0; k < CH; ++k) {
         pb.film_sum[k * wh + pixel] = sum[k];
         pb.film_comp[k * wh + pixel] = cmp[k];
     }
@@ -3367,7 +3402,9 @@ __device__ __forceinline__ float atrc_filter_rel(int32_t x, int32_t lo, int32_t 
     return d > r ? -1.0f : d;
 }
 
+template <bool AOV>
 __global__ void __launch_bounds__(256) k_film_splat(RenderConst rc, PathBuffers pb) {
+    constexpr int CH = FILM_CH<AOV>;
     const int64_t wh = int64_t(rc.W) * rc.H;
     const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (i >= wh) return;
@@ -3380,7 +3417,12 @@ __global__ void __launch_bounds__(256) k_film_splat(RenderConst rc, PathBuffers 
     const int64_t first_sample = int64_t(rc.sample_begin) + rc.work_base / ewh;
     const float r = rc.filter_r;
     const int32_t reach = int32_t(floorf(r + 0.5f));
-    float *sum = pb.film_sum, *cmp = pb.film_comp;
+    float sum[CH], cmp[CH];
+#pragma unroll
+    for (int k = 0; k < CH; ++k) {
+        sum[k] = pb.film_sum[k * wh + i];
+        cmp[k] = pb.film_comp[k * wh + i];
+    }
     float wsum = pb.film_count[i];  // running weight sum, one addition per sample in sample order
     for (int64_t j = 0; j < layers; ++j) {
         for (int32_t qy = y - reach; qy <= y + reach; ++qy) {
@@ -3389,8 +3431,8 @@ __global__ void __launch_bounds__(256) k_film_splat(RenderConst rc, PathBuffers 
                 if (qx < -rc.border0 || qx >= rc.W + rc.border1) continue;
                 const int64_t q = int64_t(qy + rc.border0) * rc.EW + (qx + rc.border0);
                 const int64_t slot = j * ewh + q;
-                const float4 v = pb.radiance[slot];
-                if (!(isfinite(v.x) && isfinite(v.y) && isfinite(v.z))) continue;
+                const V v = film_radiance(pb, slot, pb.flags[slot]);
+                if (!finite3(v)) continue;
                 Rng rs = rng_seed(rc.seed, path_seq((unsigned long long)q, (unsigned long long)(first_sample + j)));
                 const float sx = float(qx) + rs.uniform(), sy = float(qy) + rs.uniform();
                 const float xr = atrc_filter_rel(x, tx0, tx1, r, sx), yr = atrc_filter_rel(y, ty0, ty1, r, sy);
@@ -3399,36 +3441,43 @@ __global__ void __launch_bounds__(256) k_film_splat(RenderConst rc, PathBuffers 
                                       ? gauss1(xr, rc.filter_alpha, rc.filter_exp) * gauss1(yr, rc.filter_alpha,
                                                                                               rc.filter_exp)
                                       : 1.0f;
-                const float4 a = pb.gb_albedo[slot], n = pb.gb_normal[slot];
-                const float vals[10] = {v.x, v.y, v.z, a.x, a.y, a.z, n.x, n.y, n.z, a.w};
-                for (int k = 0; k < 10; ++k) neumaier(&sum[k * wh + i], &cmp[k * wh + i], wgt * vals[k]);
+                film_add<AOV>(pb, slot, v, wgt, sum, cmp);
                 wsum += wgt;
             }
         }
     }
+#pragma unroll
+    for (int k = 0; k < CH; ++k) {
+        pb.film_sum[k * wh + i] = sum[k];
+        pb.film_comp[k * wh + i] = cmp[k];
+    }
     pb.film_count[i] = wsum;
 }
 
-__global__ void k_film_clear(PathBuffers pb, int64_t wh) {
+__global__ void k_film_clear(PathBuffers pb, int64_t wh, int channels) {
     const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (i >= wh) return;
-    for (int k = 0; k < 10; ++k) { pb.film_sum[k * wh + i] = 0; pb.film_comp[k * wh + i] = 0; }
+    for (int k = 0; k < channels; ++k) { pb.film_sum[k * wh + i] = 0; pb.film_comp[k * wh + i] = 0; }
     pb.film_count[i] = 0;
 }
 
+template <bool AOV>
 __global__ void k_film_resolve(PathBuffers pb, int64_t wh, float *rgb, float *albedo, float *normal, float *denoise) {
+    constexpr int CH = FILM_CH<AOV>;
     const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
     if (i >= wh) return;
     const float c = pb.film_count[i];
     const float inv = c > 0 ? 1.0f / c : 1.0f;
-    float v[10];
-    for (int k = 0; k < 10; ++k) v[k] = (pb.film_sum[k * wh + i] + pb.film_comp[k * wh + i]) * inv;
+    float v[CH];
+    for (int k = 0; k < CH; ++k) v[k] = (pb.film_sum[k * wh + i] + pb.film_comp[k * wh + i]) * inv;
     for (int k = 0; k < 3; ++k) {
         rgb[3 * i + k] = v[k];
-        albedo[3 * i + k] = v[3 + k];
-        normal[3 * i + k] = v[6 + k];
+        if constexpr (AOV) {
+            albedo[3 * i + k] = v[3 + k];
+            normal[3 * i + k] = v[6 + k];
+        }
     }
-    denoise[i] = v[9];
+    if constexpr (AOV) denoise[i] = v[9];
 }
 
 __global__ void k_reset_counters(uint32_t *c) {
@@ -3591,14 +3640,14 @@ void launch_shade(const DevScene &s, const RenderConst &rc, const PathBuffers &p
     // media and delta surfaces without Disney, IBL or guiding (the volumetric
     // scenes): 199 VGPRs and no scratch against the full variant's spills
     const bool media_delta = (s.features & (SF_DISNEY | SF_IBL)) == 0;
-    if (lean && !rc.guide) hipLaunchKernelGGL(k_shade<0u>, dim3(grid_of(max_n, 256)), dim3(256), 0, st, s, rc, pb);
-    else if (lean) hipLaunchKernelGGL(k_shade<SF_GUIDE>, dim3(grid_of(max_n, 256)), dim3(256), 0, st, s, rc, pb);
+    if (lean && !rc.guide) hipLaunchKernelGGL(k_shade<0u>, dim3(grid_of(max_n, SHADE_BLOCK)), dim3(SHADE_BLOCK), 0, st, s, rc, pb);
+    else if (lean) hipLaunchKernelGGL(k_shade<SF_GUIDE>, dim3(grid_of(max_n, SHADE_BLOCK)), dim3(SHADE_BLOCK), 0, st, s, rc, pb);
     else if (media_delta && !rc.guide)
-        hipLaunchKernelGGL(k_shade<SF_MEDIA | SF_DELTA>, dim3(grid_of(max_n, 256)), dim3(256), 0, st, s, rc, pb);
+        hipLaunchKernelGGL(k_shade<SF_MEDIA | SF_DELTA>, dim3(grid_of(max_n, SHADE_BLOCK)), dim3(SHADE_BLOCK), 0, st, s, rc, pb);
     else if (media_delta)  // guided volumetric scenes
-        hipLaunchKernelGGL(k_shade<SF_MEDIA | SF_DELTA | SF_GUIDE>, dim3(grid_of(max_n, 256)), dim3(256), 0, st, s,
+        hipLaunchKernelGGL(k_shade<SF_MEDIA | SF_DELTA | SF_GUIDE>, dim3(grid_of(max_n, SHADE_BLOCK)), dim3(SHADE_BLOCK), 0, st, s,
                            rc, pb);
-    else hipLaunchKernelGGL(k_shade<SF_ALL>, dim3(grid_of(max_n, 256)), dim3(256), 0, st, s, rc, pb);
+    else hipLaunchKernelGGL(k_shade<SF_ALL>, dim3(grid_of(max_n, SHADE_BLOCK)), dim3(SHADE_BLOCK), 0, st, s, rc, pb);
 }
 
 uint32_t queue_compact_blocks(uint32_t max_n) { return (max_n + QC_SPAN - 1) / QC_SPAN + 1; }
@@ -3651,21 +3700,23 @@ void launch_reset_counters(uint32_t *c, hipStream_t st) {
 }
 void launch_film(const RenderConst &rc, const PathBuffers &pb, hipStream_t st) {
     const int64_t wh = int64_t(rc.W) * rc.H;
-    if (rc.splat) {
-        hipLaunchKernelGGL(k_film_splat, dim3(grid_of(uint64_t(wh), 256)), dim3(256), 0, st, rc, pb);
-        return;
-    }
-    const int64_t cover = rc.n_paths < wh ? int64_t(rc.n_paths) : wh;
+    const int64_t cover = rc.splat ? wh : (rc.n_paths < wh ? int64_t(rc.n_paths) : wh);
     if (cover <= 0) return;
-    hipLaunchKernelGGL(k_film, dim3(grid_of(uint64_t(cover), 256)), dim3(256), 0, st, rc, pb);
+    const dim3 grid(grid_of(uint64_t(cover), 256)), block(256);
+    if (rc.splat && rc.aov) hipLaunchKernelGGL(k_film_splat<true>, grid, block, 0, st, rc, pb);
+    else if (rc.splat) hipLaunchKernelGGL(k_film_splat<false>, grid, block, 0, st, rc, pb);
+    else if (rc.aov) hipLaunchKernelGGL(k_film<true>, grid, block, 0, st, rc, pb);
+    else hipLaunchKernelGGL(k_film<false>, grid, block, 0, st, rc, pb);
 }
-void launch_film_clear(const PathBuffers &pb, int64_t wh, hipStream_t st) {
-    hipLaunchKernelGGL(k_film_clear, dim3(grid_of(uint64_t(wh), 256)), dim3(256), 0, st, pb, wh);
+void launch_film_clear(const RenderConst &rc, const PathBuffers &pb, int64_t wh, hipStream_t st) {
+    hipLaunchKernelGGL(k_film_clear, dim3(grid_of(uint64_t(wh), 256)), dim3(256), 0, st, pb, wh,
+                       rc.aov ? FILM_CH<true> : FILM_CH<false>);
 }
-void launch_film_resolve(const PathBuffers &pb, int64_t wh, float *rgb, float *albedo, float *normal, float *denoise,
-                         hipStream_t st) {
-    hipLaunchKernelGGL(k_film_resolve, dim3(grid_of(uint64_t(wh), 256)), dim3(256), 0, st, pb, wh, rgb, albedo,
-                       normal, denoise);
+void launch_film_resolve(const RenderConst &rc, const PathBuffers &pb, int64_t wh, float *rgb, float *albedo,
+                         float *normal, float *denoise, hipStream_t st) {
+    const dim3 grid(grid_of(uint64_t(wh), 256)), block(256);
+    if (rc.aov) hipLaunchKernelGGL(k_film_resolve<true>, grid, block, 0, st, pb, wh, rgb, albedo, normal, denoise);
+    else hipLaunchKernelGGL(k_film_resolve<false>, grid, block, 0, st, pb, wh, rgb, albedo, normal, denoise);
 }
 void launch_capture_rays(const PathBuffers &pb, int which, float4 *o, float4 *d, uint32_t *count, uint32_t cap,
                          uint32_t max_n, hipStream_t st) {
