@@ -649,6 +649,7 @@ int agx_render(agx_ctx *c, const agx_render_params *p, const volatile int32_t *c
     st.prim_bytes = 48;
     st.info_bytes = 96;
     if (stats) HIP_TRY(hipMemsetAsync(c->dcnt, 0, 2 * sizeof(DevCounters), c->stream));
+    c->pb.eps = rc.eps;
     launch_film_clear(rc, c->pb, wh, c->stream);
     HIP_TRY(hipEventRecord(c->ev[0], c->stream));
     // Timing events: (start, end, kind) per launch group; read after the render.
@@ -1099,6 +1100,7 @@ int enqueue_render(agx_ctx *c, const agx_render_params *p, hipStream_t st, unsig
     const int spec = (c->ds.features & SF_DELTA) ? std::max(p->specular_depth, 0) : 0;
     const int max_bounces = p->max_depth + spec + 2;
     PathBuffers pb = c->pb;
+    pb.eps = rc.eps;
     launch_film_clear(rc, pb, wh, st);
     for (int64_t base = 0; base < total; base += per_pass) {
         rc.work_base = base;

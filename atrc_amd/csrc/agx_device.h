@@ -22,6 +22,11 @@ struct alignas(16) vec4 {
     float x, y, z, w;
 };
 
+// 12-byte POD (one dwordx3): path-state vectors without a fourth component
+struct vec3 {
+    float x, y, z;
+};
+
 constexpr uint32_t INTERIOR = 0xffffffffu;   // BLAS node: start == INTERIOR marks an interior node
 constexpr uint32_t TLAS_LEAF = 0x80000000u;  // TLAS node: left word has this bit for leaves
 constexpr int MAX_LIGHTS = 16;

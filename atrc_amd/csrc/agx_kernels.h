@@ -9,23 +9,24 @@ namespace agx {
 
 // Per-path state (structure of arrays, N = paths in flight).
 struct PathBuffers {
-    float4 *coef;        // [N] path throughput
+    vec3 *coef;          // [N] path throughput
     float4 *radiance;    // [N] accumulated radiance (unless PF_DARK)
     float4 *gb_albedo;   // [N] (albedo.xyz, denoise), with RenderConst::aov
     float4 *gb_normal;   // [N]
     unsigned long long *rng;     // [N] PCG32 state (the increment is derived from the path id)
     unsigned long long *rng_tr;  // [N] second stream: ratio-tracking transmittance draws
-    int4 *depth;         // [N] (depth, s_depth, medium scattering count, 0)
+    uint2 *depth;        // [N] depth, specular depth, medium scattering count, shadow mask: 16 bits each
     uint32_t *flags;     // [N] PF_* bits
     float4 *mis_a;       // [N] MIS-BSDF record: (coef.xyz, |cos|)
     float4 *mis_b;       // [N]                  (f.xyz, pdf)
     float4 *nee;         // [N*L] (coef * contribution.xyz, valid)
-    float4 *ray_o;       // [2N] (o.xyz, t_min); 2p = continuation, 2p+1 = MIS-BSDF ray
-    float4 *ray_d;       // [2N] (d.xyz, t_max)
+    vec3 *ray_o;         // [2N] origins; 2p = continuation, 2p+1 = MIS-BSDF ray; every ray's range is [0, inf]
+    vec3 *ray_d;         // [2N] directions
     float4 *hit;         // [2N] (t, u, v, entity bits), entity = -1 on miss
     int32_t *hit_prim;   // [2N] primitive slot (mesh: global BVH slot; quad: 0/1)
-    float4 *sh_o;        // [N*L] shadow rays (o.xyz, t_max)
-    float4 *sh_d;        // [N*L] (d.xyz, t_min)
+    vec3 *sh_o;          // [N*L] shadow rays: origins; every ray's range starts at eps
+    float4 *sh_d;        // [N*L] (d.xyz, t_max)
+    float eps;           // of the render (RenderConst::eps)
     uint8_t *occluded;   // [N*L]
     uint32_t *q_closest; // [2N] ray indices to trace (closest hit)
     uint32_t *q_shadow;  // [N*L] shadow ray indices

@@ -58,6 +58,8 @@ __device__ __forceinline__ V normalize(V a) { return a / length(a); }
 __device__ __forceinline__ bool black(V a) { return a.x == 0.0f && a.y == 0.0f && a.z == 0.0f; }
 __device__ __forceinline__ float cosv(V a, V b) { return dot(a, b) / (length(a) * length(b)); }
 __device__ __forceinline__ float4 f4(V a, float w) { return make_float4(a.x, a.y, a.z, w); }
+__device__ __forceinline__ V mk(const vec3 &a) { return V{a.x, a.y, a.z}; }
+__device__ __forceinline__ vec3 v3(V a) { return vec3{a.x, a.y, a.z}; }
 // std::min / std::max operand semantics (matter for NaN slab values)
 __device__ __forceinline__ float smin(float a, float b) { return b < a ? b : a; }
 __device__ __forceinline__ float smax(float a, float b) { return a < b ? b : a; }
@@ -141,6 +143,17 @@ __device__ Rng rng_seed(unsigned long long seed, unsigned long long seq) {
     r.next();
     return r;
 }
+
+// A path's depth record: (depth, specular depth, medium scattering count,
+// shadow mask), 16 bits each.  Depths and counts grow by at most one a bounce,
+// and no render has 65,535 bounces.
+__device__ __forceinline__ int4 unpack_depth(uint2 v) {
+    return make_int4(int(v.x & 0xffffu), int(v.x >> 16), int(v.y & 0xffffu), int(v.y >> 16));
+}
+__device__ __forceinline__ uint2 pack_depth(int4 d) {
+    return make_uint2((uint32_t(d.x) & 0xffffu) | (uint32_t(d.y) << 16), (uint32_t(d.z) & 0xffffu) | (uint32_t(d.w) << 16));
+}
+static_assert(MAX_LIGHTS <= 16, "the shadow mask of a path is 16 bits");
 
 // ---------------------------------------------------------------- queues
 // Appends one entry for every active lane with `pred` set: a single atomic per
@@ -1840,13 +1853,13 @@ __global__ void __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(TM == T
             // first, while the queue entry and then the ray arrive
             const B4Node root = b4_load(reinterpret_cast<const float4 *>(s.b4_nodes));
             const uint32_t ri = pb.q_closest[tid];
-            const float4 o4 = pb.ray_o[ri], d4 = pb.ray_d[ri];
+            const V o = mk(pb.ray_o[ri]), d = mk(pb.ray_d[ri]);
             constexpr int CAP = (TM == TM_B4_LARGE || TM == TM_B4W_LARGE) ? BVH4_STACK_LARGE : BVH4_STACK_SMALL;
             using Q = B4Closest<STATS, CAP, TM == TM_B4W_SMALL || TM == TM_B4W_LARGE, TB>;
             uint2 *ring = reinterpret_cast<uint2 *>(lds_col) + threadIdx.x;
             Q q;
             uint2 spill[Q::SPILL];
-            q.start(mk(o4), mk(d4), o4.w, d4.w);
+            q.start(o, d, 0.0f, INF_F);
             b4_run<false>(q, q.visit(root, c, ring, spill) ? false : q.pop_next(ring, spill), s, c, ring, spill);
             found = q.hit();
             pb.hit[ri] = make_float4(q.rec.t, q.rec.u, q.rec.v, __int_as_float(found ? q.rec.ent : -1));
@@ -1854,10 +1867,10 @@ __global__ void __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(TM == T
         }
     } else if (tid < n) {
         const uint32_t ri = pb.q_closest[tid];
-        const float4 o4 = pb.ray_o[ri], d4 = pb.ray_d[ri];
+        const V o = mk(pb.ray_o[ri]), d = mk(pb.ray_d[ri]);
         HitRec h;
         h.ent = -1; h.prim = -1; h.t = -1; h.u = 0; h.v = 0;
-        found = query_closest<STATS, TM, TB>(s, mk(o4), mk(d4), o4.w, d4.w, &h, c, lds_col);
+        found = query_closest<STATS, TM, TB>(s, o, d, 0.0f, INF_F, &h, c, lds_col);
         if (!found) h.ent = -1;
         pb.hit[ri] = make_float4(h.t, h.u, h.v, __int_as_float(h.ent));
         pb.hit_prim[ri] = h.prim;
@@ -1881,21 +1894,23 @@ __global__ void __launch_bounds__(TB) k_trace_shadow(DevScene s, PathBuffers pb,
             // root is visited from registers
             const B4Node root = b4_load(reinterpret_cast<const float4 *>(s.b4_nodes));
             const uint32_t ri = pb.q_shadow[tid];
-            const float4 o4 = pb.sh_o[ri], d4 = pb.sh_d[ri];
+            const V o = mk(pb.sh_o[ri]);
+            const float4 d4 = pb.sh_d[ri];
             constexpr int CAP = (TM == TM_B4_LARGE || TM == TM_B4W_LARGE) ? BVH4_STACK_LARGE : BVH4_STACK_SMALL;
             using Q = B4Any<STATS, CAP, TM == TM_B4W_SMALL || TM == TM_B4W_LARGE, TB>;
             uint32_t *ring = lds_col + threadIdx.x;
             Q q;
             uint32_t spill[Q::SPILL];
-            q.start(mk(o4), mk(d4), d4.w, o4.w);
+            q.start(o, mk(d4), pb.eps, d4.w);
             b4_run<false>(q, q.visit(root, c, ring, spill) ? false : q.pop_next(ring, spill), s, c, ring, spill);
             occ = q.occluded;
             pb.occluded[ri] = occ ? 1 : 0;
         }
     } else if (tid < n) {
         const uint32_t ri = pb.q_shadow[tid];
-        const float4 o4 = pb.sh_o[ri], d4 = pb.sh_d[ri];
-        occ = query_any<STATS, TM, TB>(s, mk(o4), mk(d4), d4.w, o4.w, c, lds_col);
+        const V o = mk(pb.sh_o[ri]);
+            const float4 d4 = pb.sh_d[ri];
+        occ = query_any<STATS, TM, TB>(s, o, mk(d4), pb.eps, d4.w, c, lds_col);
         pb.occluded[ri] = occ ? 1 : 0;
     }
     if (STATS) flush_counts(c, 0u, cnt);
@@ -1978,8 +1993,8 @@ __global__ void __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(6, 8)))
         next, last, s, c, reinterpret_cast<uint2 *>(lds_col) + threadIdx.x, spill,
         [&](uint32_t i, Q &q) {
             const uint32_t ri = pb.q_closest[i];
-            const float4 o4 = pb.ray_o[ri], d4 = pb.ray_d[ri];
-            q.start(mk(o4), mk(d4), o4.w, d4.w);
+            const V o = mk(pb.ray_o[ri]), d = mk(pb.ray_d[ri]);
+            q.start(o, d, 0.0f, INF_F);
             return ri;
         },
         [&](uint32_t ri, const Q &q) {
@@ -2004,8 +2019,9 @@ __global__ void __launch_bounds__(TB) k_trace_shadow_runs(DevScene s, PathBuffer
         next, last, s, c, lds_col + threadIdx.x, spill,
         [&](uint32_t i, Q &q) {
             const uint32_t ri = pb.q_shadow[i];
-            const float4 o4 = pb.sh_o[ri], d4 = pb.sh_d[ri];
-            q.start(mk(o4), mk(d4), d4.w, o4.w);
+            const V o = mk(pb.sh_o[ri]);
+            const float4 d4 = pb.sh_d[ri];
+            q.start(o, mk(d4), pb.eps, d4.w);
             return ri;
         },
         [&](uint32_t ri, const Q &q) { pb.occluded[ri] = q.occluded ? 1 : 0; });
@@ -2060,8 +2076,8 @@ __global__ void __launch_bounds__(256) k_raygen(DevScene s, RenderConst rc, Path
     }
     if (launch) {
         flags |= PF_CONT | PF_FRESH;
-        pb.ray_o[2 * p] = f4(o, 0.0f);
-        pb.ray_d[2 * p] = f4(d, INF_F);
+        pb.ray_o[2 * p] = v3(o);
+        pb.ray_d[2 * p] = v3(d);
     }
     if (rc.min_depth >= 1 && rc.max_depth >= 1) {
         // no roulette at depth 1 and a first segment to trace: every camera path is
@@ -2318,9 +2334,9 @@ __device__ V resolve_mis(const DevScene &s, const PathBuffers &pb, uint32_t p, u
 }
 
 // writes the shadow ray of slot p * L + l; k_shade queues the slots at its end
-__device__ __forceinline__ void put_shadow(const PathBuffers &pb, size_t slot, V o, V d, float tmin, float tmax) {
-    pb.sh_o[slot] = f4(o, tmax);
-    pb.sh_d[slot] = f4(d, tmin);
+__device__ __forceinline__ void put_shadow(const PathBuffers &pb, size_t slot, V o, V d, float tmax) {
+    pb.sh_o[slot] = v3(o);
+    pb.sh_d[slot] = f4(d, tmax);
 }
 
 // ---------------------------------------------------------------- path guiding
@@ -2666,7 +2682,7 @@ __global__ void __launch_bounds__(256) k_media(DevScene s, RenderConst rc, PathB
     const float4 h4 = pb.hit[2 * p];
     const int32_t ent = __float_as_int(h4.w);
     if ((flags & PF_CONT) && ent >= 0) {
-        const int4 dep = (flags & PF_FRESH) ? make_int4(1, 1, 0, 0) : pb.depth[p];
+        const int4 dep = (flags & PF_FRESH) ? make_int4(1, 1, 0, 0) : unpack_depth(pb.depth[p]);
         HitRec h;
         h.t = h4.x; h.u = h4.y; h.v = h4.z; h.ent = ent; h.prim = pb.hit_prim[2 * p];
         const V ro = mk(pb.ray_o[2 * p]), rd = mk(pb.ray_d[2 * p]);
@@ -2805,7 +2821,7 @@ __global__ void __launch_bounds__(SHADE_BLOCK) k_shade(DevScene s, RenderConst r
         dep = make_int4(1, 1, 0, 0);
     } else {
         coef = mk(pb.coef[p]);
-        dep = pb.depth[p];
+        dep = unpack_depth(pb.depth[p]);
     }
     const float4 h4 = pb.hit[2 * p];
     const int32_t hit_prim = pb.hit_prim[2 * p];  // loaded with the hit (a miss leaves it unused)
@@ -2867,7 +2883,7 @@ __global__ void __launch_bounds__(SHADE_BLOCK) k_shade(DevScene s, RenderConst r
                 pending = true;
                 // Scene::visible(light, point): from the light towards the point
                 const float dis = length(ls.pos - ms.pos);
-                put_shadow(pb, slot, ls.pos, normalize(ms.pos - ls.pos), eps, dis - eps);
+                put_shadow(pb, slot, ls.pos, normalize(ms.pos - ls.pos), dis - eps);
                 shadow_mask |= 1u << l;
             }
             if (!rc.nomis) {  // MIS-BSDF ray with the phase function (direct_illum.cpp:194-253)
@@ -2878,8 +2894,8 @@ __global__ void __launch_bounds__(SHADE_BLOCK) k_shade(DevScene s, RenderConst r
                 hg_sample(ms.g, ms.wr, u0, u1, &dir, &f);
                 if (f != 0.0f) {
                     dir = normalize(dir);
-                    pb.ray_o[2 * p + 1] = f4(ms.pos, 0.0f);
-                    pb.ray_d[2 * p + 1] = f4(dir, INF_F);
+                    pb.ray_o[2 * p + 1] = v3(ms.pos);
+                    pb.ray_d[2 * p + 1] = v3(dir);
                     pb.mis_a[p] = f4(coef, 1.0f);
                     pb.mis_b[p] = make_float4(f, f, f, f);
                     flags |= PF_MIS | (uint32_t(mi + 1) << PF_MIS_MED_SHIFT);
@@ -2905,8 +2921,8 @@ __global__ void __launch_bounds__(SHADE_BLOCK) k_shade(DevScene s, RenderConst r
                 }
                 const float pdf = a * guide_pdf(G, dir) + (1 - a) * fp;  // the phase function's pdf is its value
                 if (fp != 0.0f && !(pdf < eps) && isfinite(pdf)) {
-                    pb.ray_o[2 * p] = f4(ms.pos, 0.0f);
-                    pb.ray_d[2 * p] = f4(dir, INF_F);
+                    pb.ray_o[2 * p] = v3(ms.pos);
+                    pb.ray_d[2 * p] = v3(dir);
                     coef = coef * (fp / pdf);
                     dep.x += 1;
                     if (dep.x <= rc.max_depth) {
@@ -2927,8 +2943,8 @@ __global__ void __launch_bounds__(SHADE_BLOCK) k_shade(DevScene s, RenderConst r
                 float f;
                 hg_sample(ms.g, rc.nomis ? sp.wr : ms.wr, u0, u1, &dir, &f);
                 if (f != 0.0f && (rc.nomis || !(f < eps))) {
-                    pb.ray_o[2 * p] = f4(ms.pos, 0.0f);
-                    pb.ray_d[2 * p] = f4(rc.nomis ? dir : normalize(dir), INF_F);
+                    pb.ray_o[2 * p] = v3(ms.pos);
+                    pb.ray_d[2 * p] = v3(rc.nomis ? dir : normalize(dir));
                     coef = coef * (mk(f, f, f) / f);
                     dep.x += 1;
                     if (dep.x <= rc.max_depth) {
@@ -2998,7 +3014,7 @@ __global__ void __launch_bounds__(SHADE_BLOCK) k_shade(DevScene s, RenderConst r
             pb.nee[slot] = f4(contrib, valid ? 1.0f : 0.0f);
             if (valid) {
                 pending = true;
-                put_shadow(pb, slot, so, sd, eps, tmax);
+                put_shadow(pb, slot, so, sd, tmax);
                 shadow_mask |= 1u << l;
             }
         }
@@ -3008,8 +3024,8 @@ __global__ void __launch_bounds__(SHADE_BLOCK) k_shade(DevScene s, RenderConst r
             const BSmp bs = bsdf_sample<F>(b, wo, u0, u1, u2, eps);
             if (!black(bs.f)) {
                 const V dir = normalize(bs.dir);
-                pb.ray_o[2 * p + 1] = f4(eps_offset(sp, dir, eps), 0.0f);
-                pb.ray_d[2 * p + 1] = f4(dir, INF_F);
+                pb.ray_o[2 * p + 1] = v3(eps_offset(sp, dir, eps));
+                pb.ray_d[2 * p + 1] = v3(dir);
                 pb.mis_a[p] = f4(coef, fabsf(dot(sp.geo.z, dir)));
                 pb.mis_b[p] = f4(bs.f, bs.pdf);
                 const int32_t mm = (F & SF_MEDIA) ? medium_side(e, bs.dir, sp.geo.z) : -1;
@@ -3040,8 +3056,8 @@ __global__ void __launch_bounds__(SHADE_BLOCK) k_shade(DevScene s, RenderConst r
             if (!black(f) && !(pdf < eps) && isfinite(pdf)) {
                 const float abscos = fabsf(cosv(sp.geo.z, dir));
                 coef = coef * (f * abscos / pdf);
-                pb.ray_o[2 * p] = f4(eps_offset(sp, dir, eps), 0.0f);
-                pb.ray_d[2 * p] = f4(dir, INF_F);
+                pb.ray_o[2 * p] = v3(eps_offset(sp, dir, eps));
+                pb.ray_d[2 * p] = v3(dir);
                 dep.x += 1;
                 if (dep.x <= rc.max_depth) {
                     cont = true;
@@ -3060,8 +3076,8 @@ __global__ void __launch_bounds__(SHADE_BLOCK) k_shade(DevScene s, RenderConst r
             if (!black(bs.f) && (rc.nomis || !(bs.pdf < eps))) {
                 const float abscos = fabsf(cosv(sp.geo.z, bs.dir));
                 coef = coef * (bs.f * abscos / bs.pdf);
-                pb.ray_o[2 * p] = f4(eps_offset(sp, bs.dir, eps), 0.0f);
-                pb.ray_d[2 * p] = f4(rc.nomis ? bs.dir : normalize(bs.dir), INF_F);
+                pb.ray_o[2 * p] = v3(eps_offset(sp, bs.dir, eps));
+                pb.ray_d[2 * p] = v3(rc.nomis ? bs.dir : normalize(bs.dir));
                 if (bs.delta && dep.x >= 2 && dep.y <= rc.specular_depth) { dep.x -= 1; dep.y += 1; }
                 dep.x += 1;
                 if (dep.x <= rc.max_depth) {
@@ -3081,8 +3097,8 @@ __global__ void __launch_bounds__(SHADE_BLOCK) k_shade(DevScene s, RenderConst r
     // the lights in shadow_mask; k_queue_* build the queues from these after the launch
     (void)push_mis;
     dep.w = int32_t(shadow_mask);
-    pb.coef[p] = f4(coef, 0);
-    pb.depth[p] = dep;
+    pb.coef[p] = v3(coef);
+    pb.depth[p] = pack_depth(dep);
     pb.flags[p] = flags;
     pb.rng[p] = rng.state;
 }
@@ -3104,7 +3120,7 @@ __device__ __forceinline__ QPred queue_pred(const PathBuffers &pb, uint32_t p, u
     q.cont = (f & PF_CONT) ? 1u : 0u;
     q.mis = ((f & PF_MIS) && (f & PF_PENDING)) ? 1u : 0u;
     q.again = (f & (PF_CONT | PF_PENDING)) ? 1u : 0u;
-    q.mask = (f & PF_PENDING) ? uint32_t(pb.depth[p].w) & ((1u << L) - 1u) : 0u;  // L <= MAX_LIGHTS
+    q.mask = (f & PF_PENDING) ? (pb.depth[p].y >> 16) & ((1u << L) - 1u) : 0u;  // L <= MAX_LIGHTS
     return q;
 }
 // exclusive prefix sum over the wave's lanes; *total = the wave's sum
@@ -3527,14 +3543,12 @@ __global__ void __launch_bounds__(256) k_capture_rays(PathBuffers pb, int which,
     if (live && idx < cap) {
         if (which == 0) {
             const uint32_t ri = pb.q_closest[tid];
-            o[idx] = pb.ray_o[ri];
-            d[idx] = pb.ray_d[ri];
+            o[idx] = f4(mk(pb.ray_o[ri]), 0.0f);
+            d[idx] = f4(mk(pb.ray_d[ri]), INF_F);
         } else {
-            // shadow rays keep (o, t_max) (d, t_min); captured as (o, t_min) (d, t_max)
             const uint32_t ri = pb.q_shadow[tid];
-            const float4 so = pb.sh_o[ri], sd = pb.sh_d[ri];
-            o[idx] = make_float4(so.x, so.y, so.z, sd.w);
-            d[idx] = make_float4(sd.x, sd.y, sd.z, so.w);
+            o[idx] = f4(mk(pb.sh_o[ri]), pb.eps);
+            d[idx] = pb.sh_d[ri];
         }
     }
 }
