@@ -53,6 +53,11 @@ template <class T> hipError_t upload(T **p, const std::vector<T> &v, hipStream_t
 
 }  // namespace
 
+// agx_trace_rays: calls of up to RAYS_PINNED rays go through pinned memory, larger
+// ones through device buffers of at most RAYS_CHUNK rays
+constexpr uint32_t RAYS_PINNED = 1u << 15;
+constexpr uint32_t RAYS_CHUNK = 1u << 22;
+
 struct agx_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -107,6 +112,9 @@ struct agx_ctx {
     size_t media_cap = 0, media_nee_cap = 0;  // paths / NEE slots the media buffers hold
     std::vector<void *> media_allocs;
     std::vector<void *> guide_allocs, guide_wave_allocs;
+    float *rays_pin = nullptr;       // agx_trace_rays: pinned staging of small calls
+    float *rays_dev = nullptr;       // and the device staging of larger ones (at most RAYS_CHUNK rays, 218 MB)
+    uint32_t rays_dev_cap = 0;
     hipEvent_t ev[8]{};
     std::vector<hipEvent_t> pool;    // timing / readback events, reused across renders
     hipEvent_t event(size_t i) {
@@ -187,6 +195,26 @@ struct agx_ctx {
         HIP_TRY(galloc(media_allocs, &pb.nee_seg, nl));
         media_cap = n;
         media_nee_cap = nl;
+        return AGX_OK;
+    }
+    // staging of agx_trace_rays: pinned words of RAYS_PINNED rays and their waves' counts
+    int ensure_rays_pinned() {
+        if (rays_pin) return AGX_OK;
+        const size_t words = 13 * size_t(RAYS_PINNED) + 4 * size_t(RAYS_PINNED / 64 + 4);
+        if (hipHostMalloc(reinterpret_cast<void **>(&rays_pin), words * 4, hipHostMallocDefault) != hipSuccess) {
+            rays_pin = nullptr;
+            return fail(AGX_E_OUT_OF_MEMORY, "allocation of ray staging failed");
+        }
+        return AGX_OK;
+    }
+    // device words of n rays, kept for the next call
+    int ensure_rays_device(uint32_t n) {
+        if (n <= rays_dev_cap) return AGX_OK;
+        if (rays_dev) (void)hipFree(rays_dev);
+        rays_dev = nullptr;
+        rays_dev_cap = 0;
+        HIP_TRY(dalloc(&rays_dev, 13 * size_t(n)));
+        rays_dev_cap = n;
         return AGX_OK;
     }
     // network state; parameters initialised uniform in +-1/sqrt(fan-in) (weights)
@@ -458,6 +486,8 @@ void agx_destroy(agx_ctx *c) {
     if (c->h_counters) (void)hipHostFree(c->h_counters);
     if (c->d_resolve) (void)hipFree(c->d_resolve);
     if (c->h_resolve) (void)hipHostFree(c->h_resolve);
+    if (c->rays_pin) (void)hipHostFree(c->rays_pin);
+    if (c->rays_dev) (void)hipFree(c->rays_dev);
     for (auto &e : c->ev) if (e) (void)hipEventDestroy(e);
     for (auto &e : c->pool) if (e) (void)hipEventDestroy(e);
     if (c->stream) (void)hipStreamDestroy(c->stream);
@@ -858,49 +888,84 @@ int agx_trace_rays(agx_ctx *c, const float *o, const float *d, const float *tmin
     if (!c->has_scene) return fail(AGX_E_NO_SCENE, "no scene uploaded");
     if (!n) return AGX_OK;
     HIP_TRY(hipSetDevice(c->device));
-    std::vector<float4> ho(n), hd(n);
-    for (uint32_t i = 0; i < n; ++i) {
-        ho[i] = make_float4(o[3 * i], o[3 * i + 1], o[3 * i + 2], tmin[i]);
-        hd[i] = make_float4(d[3 * i], d[3 * i + 1], d[3 * i + 2], tmax[i]);
-    }
-    char *buf = nullptr;
-    const size_t bytes = size_t(n) * (16 + 16 + 4 * 5);
-    HIP_TRY(hipMalloc(reinterpret_cast<void **>(&buf), bytes));
-    float4 *dO = reinterpret_cast<float4 *>(buf);
-    float4 *dD = dO + n;
-    int32_t *dE = reinterpret_cast<int32_t *>(dD + n);
-    int32_t *dP = dE + n;
-    float *dT = reinterpret_cast<float *>(dP + n);
-    float *dU = dT + n;
-    float *dV = dU + n;
-    hipError_t e = hipMemcpyAsync(dO, ho.data(), n * sizeof(float4), hipMemcpyHostToDevice, c->stream);
-    if (e == hipSuccess) e = hipMemcpyAsync(dD, hd.data(), n * sizeof(float4), hipMemcpyHostToDevice, c->stream);
-    if (e == hipSuccess) e = hipMemsetAsync(c->dcnt, 0, 2 * sizeof(DevCounters), c->stream);
-    if (e == hipSuccess) e = hipEventRecord(c->ev[0], c->stream);
-    if (e == hipSuccess)
-        launch_trace_rays(c->ds, dO, dD, n, any_hit, dE, dP, dT, dU, dV, c->dcnt + (any_hit ? 1 : 0), c->stream);
-    if (e == hipSuccess) e = hipGetLastError();
-    if (e == hipSuccess) e = hipEventRecord(c->ev[1], c->stream);
-    std::vector<int32_t> he(n), hp(n);
-    std::vector<float> ht(n), hu(n), hv(n);
-    if (e == hipSuccess) e = hipMemcpyAsync(he.data(), dE, n * 4, hipMemcpyDeviceToHost, c->stream);
-    if (e == hipSuccess && !any_hit) {
-        e = hipMemcpyAsync(hp.data(), dP, n * 4, hipMemcpyDeviceToHost, c->stream);
-        if (e == hipSuccess) e = hipMemcpyAsync(ht.data(), dT, n * 4, hipMemcpyDeviceToHost, c->stream);
-        if (e == hipSuccess) e = hipMemcpyAsync(hu.data(), dU, n * 4, hipMemcpyDeviceToHost, c->stream);
-        if (e == hipSuccess) e = hipMemcpyAsync(hv.data(), dV, n * 4, hipMemcpyDeviceToHost, c->stream);
-    }
     DevCounters hc[2]{};
-    if (e == hipSuccess) e = hipMemcpyAsync(hc, c->dcnt, sizeof(hc), hipMemcpyDeviceToHost, c->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-    (void)hipFree(buf);
-    if (e != hipSuccess) return fail(AGX_E_HIP, std::string("trace_rays: ") + hipGetErrorString(e));
-    std::memcpy(entity_id, he.data(), n * 4);
-    if (!any_hit) {
-        if (prim_id) std::memcpy(prim_id, hp.data(), n * 4);
-        if (t) std::memcpy(t, ht.data(), n * 4);
-        if (u) std::memcpy(u, hu.data(), n * 4);
-        if (v) std::memcpy(v, hv.data(), n * 4);
+    double ms = 0;
+    // Small calls: one pinned buffer that the kernel reads the rays from and writes the hits
+    // to over the link, so that a call is two host copies, one launch and one wait (1001 rays:
+    // 245 -> 106 us).  Larger ones: the callers' arrays to and from device
+    // buffers that the context keeps, at most RAYS_CHUNK rays at a time
+    // (2,000,003 rays: 12.5 -> 6.5 ms).
+    if (n <= RAYS_PINNED) {
+        if (int r = c->ensure_rays_pinned(); r != AGX_OK) return r;
+        float *w = c->rays_pin;  // in words: o 3n, d 3n, tmin n, tmax n, then entity, primitive, t, u, v
+        const size_t N = n;
+        std::memcpy(w, o, 12 * N);
+        std::memcpy(w + 3 * N, d, 12 * N);
+        std::memcpy(w + 6 * N, tmin, 4 * N);
+        std::memcpy(w + 7 * N, tmax, 4 * N);
+        float *res = w + 8 * N;
+        uint4 *counts = reinterpret_cast<uint4 *>(c->rays_pin + 13 * size_t(RAYS_PINNED));
+        const uint32_t waves = (n + 255) / 256 * 4;  // every wave of the launch writes its counts
+        HIP_TRY(hipEventRecord(c->ev[0], c->stream));
+        launch_trace_rays(c->ds, RayArrays{w, w + 3 * N, w + 6 * N, w + 7 * N, 3, 1}, n, any_hit,
+                          reinterpret_cast<int32_t *>(res), reinterpret_cast<int32_t *>(res + N), res + 2 * N,
+                          res + 3 * N, res + 4 * N, nullptr, counts, c->stream);
+        HIP_TRY(hipGetLastError());
+        HIP_TRY(hipEventRecord(c->ev[1], c->stream));
+        HIP_TRY(hipStreamSynchronize(c->stream));
+        std::memcpy(entity_id, res, 4 * N);
+        if (!any_hit) {
+            if (prim_id) std::memcpy(prim_id, res + N, 4 * N);
+            if (t) std::memcpy(t, res + 2 * N, 4 * N);
+            if (u) std::memcpy(u, res + 3 * N, 4 * N);
+            if (v) std::memcpy(v, res + 4 * N, 4 * N);
+        }
+        DevCounters &k = hc[any_hit ? 1 : 0];
+        for (uint32_t i = 0; i < waves; ++i) {
+            k.node_visits += counts[i].x;
+            k.tri_tests += counts[i].y;
+            k.hits += counts[i].z;
+        }
+        ms = elapsed(c->ev[0], c->ev[1]);
+    } else {
+        if (int r = c->ensure_rays_device(std::min(n, RAYS_CHUNK)); r != AGX_OK) return r;
+        float *w = c->rays_dev;
+        HIP_TRY(hipMemsetAsync(c->dcnt, 0, 2 * sizeof(DevCounters), c->stream));
+        for (uint32_t first = 0; first < n; first += RAYS_CHUNK) {
+            const size_t N = std::min(n - first, RAYS_CHUNK), f = first;
+            float *res = w + 8 * N;
+            hipError_t e = hipSuccess;
+            auto put = [&](float *dst, const float *src, size_t words) {
+                if (e == hipSuccess) e = hipMemcpyAsync(dst, src, words * 4, hipMemcpyHostToDevice, c->stream);
+            };
+            auto get = [&](void *dst, const float *src) {
+                if (e == hipSuccess && dst) e = hipMemcpyAsync(dst, src, N * 4, hipMemcpyDeviceToHost, c->stream);
+            };
+            put(w, o + 3 * f, 3 * N);
+            put(w + 3 * N, d + 3 * f, 3 * N);
+            put(w + 6 * N, tmin + f, N);
+            put(w + 7 * N, tmax + f, N);
+            if (e == hipSuccess) e = hipEventRecord(c->ev[0], c->stream);
+            if (e == hipSuccess) {
+                launch_trace_rays(c->ds, RayArrays{w, w + 3 * N, w + 6 * N, w + 7 * N, 3, 1}, uint32_t(N), any_hit,
+                                  reinterpret_cast<int32_t *>(res), reinterpret_cast<int32_t *>(res + N), res + 2 * N,
+                                  res + 3 * N, res + 4 * N, c->dcnt + (any_hit ? 1 : 0), nullptr, c->stream);
+                e = hipGetLastError();
+            }
+            if (e == hipSuccess) e = hipEventRecord(c->ev[1], c->stream);
+            get(entity_id + f, res);
+            if (!any_hit) {
+                get(prim_id ? prim_id + f : nullptr, res + N);
+                get(t ? t + f : nullptr, res + 2 * N);
+                get(u ? u + f : nullptr, res + 3 * N);
+                get(v ? v + f : nullptr, res + 4 * N);
+            }
+            const hipError_t done = hipStreamSynchronize(c->stream);  // also after an error: copies may be in flight
+            if (e == hipSuccess) e = done;
+            if (e != hipSuccess) return fail(AGX_E_HIP, std::string("trace_rays: ") + hipGetErrorString(e));
+            ms += elapsed(c->ev[0], c->ev[1]);
+        }
+        HIP_TRY(hipMemcpy(hc, c->dcnt, sizeof(hc), hipMemcpyDeviceToHost));
     }
     agx_stats_t st{};
     st.node_bytes = c->accel != AGX_ACCEL_ATRC ? 16 * BVH4_NODE_VEC4 : 32;
@@ -908,9 +973,10 @@ int agx_trace_rays(agx_ctx *c, const float *o, const float *d, const float *tmin
     st.info_bytes = 96;
     if (any_hit) st.shadow_rays = n; else st.closest_rays = n;
     fill_traversal_stats(hc, &st);
-    st.total_ms = elapsed(c->ev[0], c->ev[1]);
-    if (any_hit) { st.trace_shadow_ms = st.total_ms; st.trace_shadow_launches = 1; }
-    else { st.trace_closest_ms = st.total_ms; st.trace_closest_launches = 1; }
+    st.total_ms = ms;
+    const uint64_t launches = n <= RAYS_PINNED ? 1 : (n - 1) / RAYS_CHUNK + 1;
+    if (any_hit) { st.trace_shadow_ms = ms; st.trace_shadow_launches = launches; }
+    else { st.trace_closest_ms = ms; st.trace_closest_launches = launches; }
     c->stats = st;
     return AGX_OK;
 }
@@ -1670,8 +1736,10 @@ int agx_debug_replay_rays(agx_ctx *c, const agx_render_params *p, uint32_t max_r
         double ms = 0;
         for (int k = 0; k <= reps; ++k) {
             HIP_TRY(hipEventRecord(c->ev[0], c->stream));
-            launch_trace_rays(c->ds, base + 2 * size_t(which) * max_rays, base + (2 * size_t(which) + 1) * max_rays,
-                              n[which], which, ent, prim, t, u, v, nullptr, c->stream);
+            const float *ro = reinterpret_cast<const float *>(base + 2 * size_t(which) * max_rays);
+            const float *rd = reinterpret_cast<const float *>(base + (2 * size_t(which) + 1) * max_rays);
+            launch_trace_rays(c->ds, RayArrays{ro, rd, ro + 3, rd + 3, 4, 4}, n[which], which, ent, prim, t, u, v,
+                              nullptr, nullptr, c->stream);
             HIP_TRY(hipGetLastError());
             HIP_TRY(hipEventRecord(c->ev[1], c->stream));
             HIP_TRY(hipEventSynchronize(c->ev[1]));

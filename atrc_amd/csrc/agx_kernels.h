@@ -167,11 +167,20 @@ constexpr uint32_t NOALLOC_MAX_RAYS = 1u << 17;
 constexpr size_t NOALLOC_BYTES_PER_RAY = 84;
 hipError_t noalloc_scratch_init(int device);
 void *noalloc_scratch(int device);
-// trace_rays over raw host-layout inputs staged in the scratch: packs
-// (o, tmin) / (d, tmax), clears cnt with a kernel, then traces
+// trace_rays over raw host-layout inputs staged in the scratch: clears cnt with a
+// kernel, then traces
 void launch_trace_rays_staged(const DevScene &s, void *scratch, uint32_t n, int any_hit, DevCounters *cnt,
                               hipStream_t st);
-void launch_trace_rays(const DevScene &s, const float4 *o, const float4 *d, uint32_t n, int any_hit, int32_t *ent,
-                       int32_t *prim, float *t, float *u, float *v, DevCounters *cnt, hipStream_t st);
+// Rays of a query: component k of ray i's origin at o[i * vstride + k], its range
+// at tmin[i * tstride], tmax[i * tstride] (separate arrays: strides 3 and 1; packed
+// (o, tmin) (d, tmax) rows: 4 and 4)
+struct RayArrays {
+    const float *o, *d, *tmin, *tmax;
+    int32_t vstride, tstride;
+};
+// cnt: totals are added to it; or wave_counts: (visits, tests, hits, 0) of each of
+// the ceil(n / 64) waves; both null: nothing is counted
+void launch_trace_rays(const DevScene &s, const RayArrays &in, uint32_t n, int any_hit, int32_t *ent, int32_t *prim,
+                       float *t, float *u, float *v, DevCounters *cnt, uint4 *wave_counts, hipStream_t st);
 
 }  // namespace agx

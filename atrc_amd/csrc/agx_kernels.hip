@@ -1804,14 +1804,17 @@ __device__ BSmp bsdf_sample(const Bsdf &b, const WoTerms &o, float su, float sv,
 }
 
 // ---------------------------------------------------------------- wave-level counter reduction
-__device__ __forceinline__ void flush_counts(const Counts &c, uint32_t hits, DevCounters *cnt) {
+__device__ __forceinline__ void flush_counts(const Counts &c, uint32_t hits, DevCounters *cnt,
+                                             uint4 *wave_counts = nullptr) {
     uint32_t v = c.visits, t = c.tests, h = hits;
     for (int off = 32; off > 0; off >>= 1) {
         v += __shfl_xor(v, off);
         t += __shfl_xor(t, off);
         h += __shfl_xor(h, off);
     }
-    if ((threadIdx.x & 63) == 0) {
+    if ((threadIdx.x & 63) == 0 && wave_counts) {
+        *wave_counts = make_uint4(v, t, h, 0);
+    } else if ((threadIdx.x & 63) == 0) {
         atomicAdd(&cnt->node_visits, (unsigned long long)v);
         atomicAdd(&cnt->tri_tests, (unsigned long long)t);
         atomicAdd(&cnt->hits, (unsigned long long)h);
@@ -3500,24 +3503,29 @@ __global__ void k_reset_counters(uint32_t *c) {
     if (threadIdx.x < 4) c[threadIdx.x] = 0;
 }
 
+// Ray queries: rays and results may lie in device or in pinned host memory.
+// wave_counts (may be null): (visits, tests, hits, 0) of every wave, for a host
+// that sums them itself; otherwise the totals are added to cnt.
 template <bool STATS, int TM, int TB>
-__global__ void __launch_bounds__(TB) k_trace_rays(DevScene s, const float4 *o, const float4 *d, uint32_t n,
-                                                    int any_hit, int32_t *ent, int32_t *prim, float *t, float *u,
-                                                    float *v, DevCounters *cnt) {
+__global__ void __launch_bounds__(TB) k_trace_rays(DevScene s, RayArrays in, uint32_t n, int any_hit, int32_t *ent,
+                                                    int32_t *prim, float *t, float *u, float *v, DevCounters *cnt,
+                                                    uint4 *wave_counts) {
     AGX_LDS_COLUMN(TM, TB);
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     Counts c;
     bool found = false;
     if (i < n) {
-        const float4 o4 = o[i], d4 = d[i];
+        const float *po = in.o + size_t(i) * in.vstride, *pd = in.d + size_t(i) * in.vstride;
+        const V o = mk(po[0], po[1], po[2]), d = mk(pd[0], pd[1], pd[2]);
+        const float tmin = in.tmin[size_t(i) * in.tstride], tmax = in.tmax[size_t(i) * in.tstride];
         if (any_hit) {
-            found = query_any<STATS, TM, TB>(s, mk(o4), mk(d4), o4.w, d4.w, c, lds_col);
+            found = query_any<STATS, TM, TB>(s, o, d, tmin, tmax, c, lds_col);
             ent[i] = found ? 1 : -1;
             found = false;
         } else {
             HitRec h;
             h.ent = -1; h.prim = -1; h.t = -1; h.u = 0; h.v = 0;
-            found = query_closest<STATS, TM, TB>(s, mk(o4), mk(d4), o4.w, d4.w, &h, c, lds_col);
+            found = query_closest<STATS, TM, TB>(s, o, d, tmin, tmax, &h, c, lds_col);
             if (found) {
                 const DevEntity &e = s.ents[h.ent];
                 int32_t pid = h.prim;
@@ -3528,7 +3536,7 @@ __global__ void __launch_bounds__(TB) k_trace_rays(DevScene s, const float4 *o, 
             }
         }
     }
-    if (STATS) flush_counts(c, found ? 1u : 0u, cnt);
+    if (STATS) flush_counts(c, found ? 1u : 0u, cnt, wave_counts ? wave_counts + (i >> 6) : nullptr);
 }
 
 // Copies the rays of the current closest-hit (which = 0) or any-hit (1) queue,
@@ -3740,7 +3748,7 @@ void launch_capture_rays(const PathBuffers &pb, int which, float4 *o, float4 *d,
 // ---------------------------------------------------------------- staging without allocation
 // The staging buffer of agx_trace_rays_noalloc.  Layout for n rays (n <=
 // NOALLOC_MAX_RAYS), offsets in units of NOALLOC_MAX_RAYS 4-byte words:
-//   [0, 4) packed (o, tmin) float4   [4, 8) packed (d, tmax) float4
+//   [0, 8) unused
 //   [8, 11) o (3 floats per ray)     [11, 14) d   [14] tmin   [15] tmax
 //   [16] entity  [17] primitive  [18] t  [19] u  [20] v
 // Every GPU holds its own copy until the process ends; host code uses the
@@ -3752,17 +3760,6 @@ namespace {
 constexpr int NOALLOC_MAX_DEVICES = 64;
 std::mutex g_scratch_mu;
 void *g_scratch_ptr[NOALLOC_MAX_DEVICES] = {};
-
-__global__ void __launch_bounds__(256) k_pack_rays(uint32_t *base, uint32_t n) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const size_t M = NOALLOC_MAX_RAYS;
-    const float *o = reinterpret_cast<const float *>(base + 8 * M), *d = reinterpret_cast<const float *>(base + 11 * M);
-    const float *tmin = reinterpret_cast<const float *>(base + 14 * M), *tmax = reinterpret_cast<const float *>(base + 15 * M);
-    float4 *po = reinterpret_cast<float4 *>(base), *pd = reinterpret_cast<float4 *>(base + 4 * M);
-    po[i] = make_float4(o[3 * i], o[3 * i + 1], o[3 * i + 2], tmin[i]);
-    pd[i] = make_float4(d[3 * i], d[3 * i + 1], d[3 * i + 2], tmax[i]);
-}
 
 __global__ void k_zero_counters(DevCounters *c) {
     if (threadIdx.x < 2) c[threadIdx.x] = DevCounters{0, 0, 0, 0};
@@ -3792,18 +3789,18 @@ void launch_trace_rays_staged(const DevScene &s, void *scratch_ptr, uint32_t n, 
     uint32_t *base = static_cast<uint32_t *>(scratch_ptr);
     const size_t M = NOALLOC_MAX_RAYS;
     hipLaunchKernelGGL(k_zero_counters, dim3(1), dim3(64), 0, st, cnt);
-    hipLaunchKernelGGL(k_pack_rays, dim3(grid_of(n, 256)), dim3(256), 0, st, base, n);
-    launch_trace_rays(s, reinterpret_cast<const float4 *>(base), reinterpret_cast<const float4 *>(base + 4 * M), n,
-                      any_hit, reinterpret_cast<int32_t *>(base + 16 * M), reinterpret_cast<int32_t *>(base + 17 * M),
-                      reinterpret_cast<float *>(base + 18 * M), reinterpret_cast<float *>(base + 19 * M),
-                      reinterpret_cast<float *>(base + 20 * M), cnt + (any_hit ? 1 : 0), st);
+    auto floats = [&](size_t word) { return reinterpret_cast<float *>(base + word * M); };
+    launch_trace_rays(s, RayArrays{floats(8), floats(11), floats(14), floats(15), 3, 1}, n, any_hit,
+                      reinterpret_cast<int32_t *>(base + 16 * M), reinterpret_cast<int32_t *>(base + 17 * M),
+                      floats(18), floats(19), floats(20), cnt + (any_hit ? 1 : 0), nullptr, st);
 }
 
-void launch_trace_rays(const DevScene &s, const float4 *o, const float4 *d, uint32_t n, int any_hit, int32_t *ent,
-                       int32_t *prim, float *t, float *u, float *v, DevCounters *cnt, hipStream_t st) {
+void launch_trace_rays(const DevScene &s, const RayArrays &in, uint32_t n, int any_hit, int32_t *ent, int32_t *prim,
+                       float *t, float *u, float *v, DevCounters *cnt, uint4 *wave_counts, hipStream_t st) {
     if (!n) return;
-    const bool stats = cnt != nullptr;
-    AGX_LAUNCH_STACKED(k_trace_rays, TRACE_BLOCK, dim3(grid_of(n, TRACE_BLOCK)), st, s, o, d, n, any_hit, ent, prim, t, u, v, cnt);
+    const bool stats = cnt != nullptr || wave_counts != nullptr;
+    AGX_LAUNCH_STACKED(k_trace_rays, TRACE_BLOCK, dim3(grid_of(n, TRACE_BLOCK)), st, s, in, n, any_hit, ent, prim, t, u,
+                       v, cnt, wave_counts);
 }
 
 }  // namespace agx

@@ -1,0 +1,53 @@
+"""agx_trace_rays over its staging paths: one ray, sizes around a wave, a block
+and the limit between the pinned and the device staging, a smaller call after a
+larger one, and outputs left out; against the staging without allocation.
+"""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from atrc_amd import capi, scenes
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("accel", [capi.ACCEL_ATRC, capi.ACCEL_BVH4, capi.ACCEL_BVH4_WATERTIGHT])
+def test_ray_counts(accel):
+    s, _, _ = scenes.procedural_spheres(n_spheres=8, subdiv=2, seed=3, extent=12.0)
+    s.accel = accel
+    desc, keep = s.to_desc()
+    with capi.Context(0) as ctx:
+        ctx.upload_scene(desc)
+        for n in (1, 63, 64, 65, 257, 32767, 32768, 32769, 5, 100_001):
+            o, d = scenes.random_rays(((-2, -2, -2), (14, 14, 14)), n, seed=n)
+            tmin, tmax = np.full(n, 0.01, np.float32), np.full(n, 40.0, np.float32)
+            print(f"[ray sizes] accel {accel}, {n} rays", flush=True)
+            for any_hit in (False, True):
+                a = ctx.trace_rays(o, d, tmin, tmax, any_hit=any_hit)
+                sa = ctx.stats()
+                b = ctx.trace_rays(o, d, tmin, tmax, any_hit=any_hit, noalloc=True)
+                sb = ctx.stats()
+                for k in ("entity",) if any_hit else ("entity", "prim", "t", "u", "v"):
+                    np.testing.assert_array_equal(a[k].view(np.uint32), b[k].view(np.uint32))
+                for k in ("closest_rays", "shadow_rays", "closest_node_visits", "closest_tri_tests", "closest_hits",
+                          "shadow_node_visits", "shadow_tri_tests"):
+                    assert sa[k] == sb[k], (n, k)
+                assert sa["total_ms"] > 0
+
+
+@pytest.mark.parametrize("n", [100, 40_000])
+def test_outputs_may_be_left_out(gpu_ctx, n):
+    s, _, _ = scenes.cornell_box()
+    s.accel = capi.ACCEL_BVH4
+    desc, keep = s.to_desc()
+    gpu_ctx.upload_scene(desc)
+    o, d = scenes.random_rays(((0.1, 0.1, 0.1), (5, 5, 5)), n, seed=1)
+    tmin, tmax = np.zeros(n, np.float32), np.full(n, np.inf, np.float32)
+    full = gpu_ctx.trace_rays(o, d, tmin, tmax)
+    ent, t = np.zeros(n, np.int32), np.zeros(n, np.float32)
+    f = capi.fptr
+    assert gpu_ctx.lib.agx_trace_rays(gpu_ctx.h, f(o), f(d), f(tmin), f(tmax), n, 0, capi.iptr(ent), None, f(t), None,
+                                      None) == 0
+    np.testing.assert_array_equal(ent, full["entity"])
+    np.testing.assert_array_equal(t.view(np.uint32), full["t"].view(np.uint32))
