@@ -112,6 +112,9 @@ struct agx_ctx {
     size_t media_cap = 0, media_nee_cap = 0;  // paths / NEE slots the media buffers hold
     std::vector<void *> media_allocs;
     std::vector<void *> guide_allocs, guide_wave_allocs;
+    unsigned long long *h_stamps = nullptr;  // pinned: start times of a pass's kernels, 3 per bounce
+    double clock_khz = 100000;       // rate of those times
+    uint32_t seq = 0;                // of the queue sizes in h_counters
     float *rays_pin = nullptr;       // agx_trace_rays: pinned staging of small calls
     float *rays_dev = nullptr;       // and the device staging of larger ones (at most RAYS_CHUNK rays, 218 MB)
     uint32_t rays_dev_cap = 0;
@@ -195,6 +198,21 @@ struct agx_ctx {
         HIP_TRY(galloc(media_allocs, &pb.nee_seg, nl));
         media_cap = n;
         media_nee_cap = nl;
+        return AGX_OK;
+    }
+    // waits until slot k of the pinned ring holds the queue sizes marked seq.  The kernel
+    // that writes them is on the stream, so the wait ends with it at the latest.
+    int wait_counts(int k, uint32_t want) {
+        const uint32_t *mark = h_counters + 4 * k + 3;
+        for (uint32_t spin = 0; __atomic_load_n(mark, __ATOMIC_ACQUIRE) != want; ++spin) {
+            __builtin_ia32_pause();
+            if (spin % 4096 != 4095) continue;
+            const hipError_t e = hipStreamQuery(stream);
+            if (e == hipErrorNotReady) continue;
+            if (e != hipSuccess) return fail(AGX_E_HIP, std::string("render: ") + hipGetErrorString(e));
+            if (__atomic_load_n(mark, __ATOMIC_ACQUIRE) == want) break;
+            return fail(AGX_E_HIP, "render: queue sizes missing");
+        }
         return AGX_OK;
     }
     // staging of agx_trace_rays: pinned words of RAYS_PINNED rays and their waves' counts
@@ -452,8 +470,9 @@ int agx_create(int device_ordinal, agx_ctx **out) {
     }
     if (hipMalloc(reinterpret_cast<void **>(&c->dcnt), 2 * sizeof(DevCounters)) != hipSuccess ||
         hipHostMalloc(reinterpret_cast<void **>(&c->h_counters), agx_ctx::RING * 4 * sizeof(uint32_t),
-                      hipHostMallocDefault) !=
-            hipSuccess) {
+                      hipHostMallocDefault) != hipSuccess ||
+        hipHostMalloc(reinterpret_cast<void **>(&c->h_stamps), (agx_ctx::RING + 1) * 3 * sizeof(unsigned long long),
+                      hipHostMallocDefault) != hipSuccess) {
         agx_destroy(c);
         return fail(AGX_E_OUT_OF_MEMORY, "allocation of counters failed");
     }
@@ -462,6 +481,9 @@ int agx_create(int device_ordinal, agx_ctx **out) {
             agx_destroy(c);
             return fail(AGX_E_HIP, "hipEventCreate failed");
         }
+    int khz = 0;
+    if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, device_ordinal) == hipSuccess && khz > 0)
+        c->clock_khz = khz;
     // the staging array of agx_trace_rays_noalloc, resolved once per device
     if (const hipError_t e = noalloc_scratch_init(device_ordinal); e != hipSuccess) {
         agx_destroy(c);
@@ -484,6 +506,7 @@ void agx_destroy(agx_ctx *c) {
     c->free_guide();
     if (c->dcnt) (void)hipFree(c->dcnt);
     if (c->h_counters) (void)hipHostFree(c->h_counters);
+    if (c->h_stamps) (void)hipHostFree(c->h_stamps);
     if (c->d_resolve) (void)hipFree(c->d_resolve);
     if (c->h_resolve) (void)hipHostFree(c->h_resolve);
     if (c->rays_pin) (void)hipHostFree(c->rays_pin);
@@ -693,8 +716,6 @@ int agx_render(agx_ctx *c, const agx_render_params *p, const volatile int32_t *c
         HIP_TRY(hipEventRecord(e, c->stream));
         return AGX_OK;
     };
-    // Every bounce's queue sizes are written into a slot of a pinned ring by the kernel that
-    // makes the queues; the host reads a slot after the event that follows it.
     const int max_bounces = p->max_depth + std::max(p->specular_depth, 0) + 2;
     if (max_bounces + 1 > agx_ctx::RING)
         return fail(AGX_E_UNSUPPORTED, "max_depth + specular_depth too large (at most " +
@@ -706,27 +727,40 @@ int agx_render(agx_ctx *c, const agx_render_params *p, const volatile int32_t *c
         rc.n_paths = int32_t(std::min<int64_t>(per_pass, total - base));
         rc.guide_rec_rot = uint32_t(uint64_t(base / per_pass) * 2654435761ull) & ((1u << rc.guide_rec_shift) - 1u);
         uint32_t *cin = c->counters, *cout = c->counters + 4;
-        size_t a, b;
-        if ((r = mark(&a))) return r;
+        size_t a = 0, b = 0;
+        // a plain render's kernels note their start times; with guiding, whose inference
+        // is timed apart, events do
+        const bool stamps = !guide;
+        auto stamp = [&](int k) { return stamps ? c->h_stamps + k : nullptr; };
+        if (!stamps && (r = mark(&a))) return r;
         launch_reset_counters(cout, c->stream);
         c->pb.cnt_out = cout;
+        c->pb.stamp = stamp(0);
         launch_raygen(c->ds, rc, c->pb, c->stream);
-        // raygen queues every camera path, or (roulette at depth 1) those it counts
-        const bool all_queued = rc.min_depth >= 1 && rc.max_depth >= 1;
-        if (!all_queued) {
-            HIP_TRY(hipMemcpyAsync(c->h_counters, cout, 4 * sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream));
-        } else {
+        c->pb.stamp = nullptr;
+        // Slot k of the pinned ring: the queue sizes that bounce k consumes, complete once its
+        // fourth word is base_seq + k.  Raygen queues every camera path, or (roulette at
+        // depth 1) those it counts.
+        const uint32_t base_seq = c->seq + 1;
+        c->seq += uint32_t(max_bounces) + 2;
+        if (rc.min_depth >= 1 && rc.max_depth >= 1) {
             c->h_counters[0] = c->h_counters[2] = uint32_t(rc.n_paths);
-            c->h_counters[1] = c->h_counters[3] = 0;
+            c->h_counters[1] = 0;
+        } else {
+            HIP_TRY(hipMemcpyAsync(c->h_counters, cout, 4 * sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream));
+            HIP_TRY(hipStreamSynchronize(c->stream));
         }
-        if ((r = mark(&b))) return r;
-        timed.push_back({a, b, 2});
+        c->h_counters[3] = base_seq;
+        for (int k = 1; k <= max_bounces; ++k) c->h_counters[4 * k + 3] = base_seq - 1;
+        if (!stamps) {
+            if ((r = mark(&b))) return r;
+            timed.push_back({a, b, 2});
+        }
         st.paths += uint64_t(rc.n_paths);
-        // done[k] = the event after which slot k of the pinned ring holds the queue
-        // sizes that bounce k consumes (and the start of bounce k)
-        std::vector<size_t> done(1, b);
         uint32_t alive = uint32_t(rc.n_paths);  // at least the paths that the coming bounce shades
         int bounces = 0;
+        size_t e_last = b;  // guided: the event that starts the coming bounce
+        std::vector<char> had_shadow;
         std::swap(cin, cout);
         std::swap(c->pb.q_in, c->pb.q_out);
         for (int bounce = 0; bounce < max_bounces; ++bounce) {
@@ -737,25 +771,36 @@ int agx_render(agx_ctx *c, const agx_render_params *p, const volatile int32_t *c
             // 33 million paths.  Camera paths have no MIS or shadow rays yet.
             const uint32_t n_closest = bounce == 0 ? alive : 2 * alive;
             const uint32_t n_shadow = bounce == 0 ? 0 : alive * uint32_t(std::max(rc.L, 0));
-            size_t e0 = done.back(), e1, e2, e3;
+            size_t e1 = 0, e2 = 0, e3 = 0;
+            c->pb.stamp = stamp(3 * bounce + 1);
             launch_trace_closest(c->ds, c->pb, n_closest, stats, c->dcnt, c->stream);
-            if ((r = mark(&e1))) return r;
+            c->pb.stamp = nullptr;
+            if (!stamps && (r = mark(&e1))) return r;
             if (c->capture_count) {
                 launch_capture_rays(c->pb, 0, c->capture_o[0], c->capture_d[0], c->capture_count, c->capture_cap,
                                     n_closest, c->stream);
                 launch_capture_rays(c->pb, 1, c->capture_o[1], c->capture_d[1], c->capture_count + 1,
                                     c->capture_cap, n_shadow, c->stream);
             }
-            timed.push_back({e0, e1, 0});
+            if (!stamps) timed.push_back({e_last, e1, 0});
             e2 = e1;
             st.trace_closest_launches += 1;
+            had_shadow.push_back(n_shadow ? 1 : 0);
             if (n_shadow) {
+                c->pb.stamp = stamp(3 * bounce + 2);
                 launch_trace_shadow(c->ds, c->pb, n_shadow, stats, c->dcnt + 1, c->stream);
-                if ((r = mark(&e2))) return r;
-                timed.push_back({e1, e2, 1});
+                c->pb.stamp = nullptr;
+                if (!stamps) {
+                    if ((r = mark(&e2))) return r;
+                    timed.push_back({e1, e2, 1});
+                }
                 st.trace_shadow_launches += 1;
             }
-            if (media) launch_media(c->ds, rc, c->pb, alive, c->stream);
+            c->pb.stamp = stamp(3 * bounce + 3);
+            if (media) {
+                launch_media(c->ds, rc, c->pb, alive, c->stream);
+                c->pb.stamp = nullptr;
+            }
             if (guide) {
                 // the network's mixture for every vertex about to be shaded (in media,
                 // at the scattering point the vertex's medium sample reaches)
@@ -769,23 +814,29 @@ int agx_render(agx_ctx *c, const agx_render_params *p, const volatile int32_t *c
                 e2 = eg;
             }
             launch_shade(c->ds, rc, c->pb, alive, c->stream);
-            launch_queue_compact(c->pb, alive, rc.L, c->qc_blk, c->h_counters + 4 * (bounce + 1), c->stream);
-            if ((r = mark(&e3))) return r;
-            timed.push_back({e2, e3, 2});
-            done.push_back(e3);
+            c->pb.stamp = nullptr;
+            launch_queue_compact(c->pb, alive, rc.L, c->qc_blk, c->h_counters + 4 * (bounce + 1),
+                                 base_seq + uint32_t(bounce) + 1, c->stream);
+            if (!stamps) {
+                if ((r = mark(&e3))) return r;
+                timed.push_back({e2, e3, 2});
+                e_last = e3;
+            }
             bounces = bounce + 1;
             std::swap(cin, cout);
             std::swap(c->pb.q_in, c->pb.q_out);
             // what this bounce consumes is known by now (the bounce before it wrote it), so
             // the GPU, busy with this bounce, does not wait for the host
-            HIP_TRY(hipEventSynchronize(c->pool[done[size_t(bounce)]]));
+            if ((r = c->wait_counts(bounce, base_seq + uint32_t(bounce))) != AGX_OK) return r;
             alive = std::min(alive, c->h_counters[4 * bounce + 2]);
             if (alive == 0) break;  // this bounce was a no-op, and so would be the rest
             if (cancel_flag && *cancel_flag) { cancelled = true; break; }
         }
         if (cancelled) break;
         if ((r = mark(&a))) return r;
+        c->pb.stamp = stamp(3 * bounces + 1);
         launch_film(rc, c->pb, c->stream);
+        c->pb.stamp = nullptr;
         if ((r = mark(&b))) return r;
         timed.push_back({a, b, 2});
         if (guide_train) {
@@ -819,7 +870,17 @@ int agx_render(agx_ctx *c, const agx_render_params *p, const volatile int32_t *c
             st.guide_samples += std::min<uint32_t>(guide_samples_h, guide_batch);
             st.guide_trained += uint64_t(guide_valid_h) * uint64_t(guide_steps);
         }
-        // sum the ray queue sizes of this pass
+        if (stamps) {
+            auto ms = [&](int from, int to) { return double(c->h_stamps[to] - c->h_stamps[from]) / c->clock_khz; };
+            st.shade_ms += ms(0, 1);
+            for (int k = 0; k < bounces; ++k) {
+                const int shade = 3 * k + 3, shadow = had_shadow[size_t(k)] ? 3 * k + 2 : shade;
+                st.trace_closest_ms += ms(3 * k + 1, shadow);
+                st.trace_shadow_ms += ms(shadow, shade);
+                st.shade_ms += ms(shade, 3 * k + 4);
+            }
+        }
+        // sum the ray queue sizes of this pass (the last bounce's are complete: the pass has ended)
         for (int k = 0; k <= bounces; ++k) {
             const uint32_t *q = c->h_counters + 4 * k;
             st.closest_rays += q[0];
@@ -1167,6 +1228,7 @@ int enqueue_render(agx_ctx *c, const agx_render_params *p, hipStream_t st, unsig
     const int max_bounces = p->max_depth + spec + 2;
     PathBuffers pb = c->pb;
     pb.eps = rc.eps;
+    pb.stamp = nullptr;
     launch_film_clear(rc, pb, wh, st);
     for (int64_t base = 0; base < total; base += per_pass) {
         rc.work_base = base;
@@ -1185,7 +1247,7 @@ int enqueue_render(agx_ctx *c, const agx_render_params *p, hipStream_t st, unsig
             if (bounce > 0) launch_trace_shadow(c->ds, pb, n_shadow_max, false, c->dcnt + 1, st);
             if (c->ds.features & SF_MEDIA) launch_media(c->ds, rc, pb, uint32_t(rc.n_paths), st);
             launch_shade(c->ds, rc, pb, uint32_t(rc.n_paths), st);
-            launch_queue_compact(pb, uint32_t(rc.n_paths), rc.L, c->qc_blk, nullptr, st);
+            launch_queue_compact(pb, uint32_t(rc.n_paths), rc.L, c->qc_blk, nullptr, 0, st);
             std::swap(cin, cout);
             std::swap(pb.q_in, pb.q_out);
         }

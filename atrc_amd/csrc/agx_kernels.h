@@ -26,6 +26,7 @@ struct PathBuffers {
     int32_t *hit_prim;   // [2N] primitive slot (mesh: global BVH slot; quad: 0/1)
     vec3 *sh_o;          // [N*L] shadow rays: origins; every ray's range starts at eps
     float4 *sh_d;        // [N*L] (d.xyz, t_max)
+    unsigned long long *stamp;  // start time of the next launch (wall_clock64), or null
     float eps;           // of the render (RenderConst::eps)
     uint8_t *occluded;   // [N*L]
     uint32_t *q_closest; // [2N] ray indices to trace (closest hit)
@@ -129,12 +130,12 @@ void launch_trace_shadow(const DevScene &s, const PathBuffers &pb, uint32_t max_
 void launch_shade(const DevScene &s, const RenderConst &rc, const PathBuffers &pb, uint32_t max_n, hipStream_t st);
 // queues of the next bounce from the paths k_shade shaded (at most max_n of them);
 // blk holds queue_compact_blocks(max_n) entries; the three queue sizes also go to
-// host_counts (pinned memory; may be null)
+// host_counts (pinned memory; may be null), and seq into its fourth word after them
 uint32_t queue_compact_blocks(uint32_t max_n);
 // *acc += cin[0] + cin[1] (rays of the coming bounce), on the stream
 void launch_count_rays(const uint32_t *cin, unsigned long long *acc, hipStream_t st);
 void launch_queue_compact(const PathBuffers &pb, uint32_t max_n, int L, uint4 *blk, uint32_t *host_counts,
-                          hipStream_t st);
+                          uint32_t seq, hipStream_t st);
 // network inputs of the vertices about to be shaded (q_in order)
 void launch_guide_features(const DevScene &s, const RenderConst &rc, const PathBuffers &pb, uint32_t max_n,
                            hipStream_t st);

@@ -1822,6 +1822,13 @@ __device__ __forceinline__ void flush_counts(const Counts &c, uint32_t hits, Dev
 }
 
 // ---------------------------------------------------------------- kernels
+// The kernels of a plain render's bounce note when they start (pb.stamp, pinned
+// memory): on one stream that is when the kernel before has ended, and costs nothing,
+// where an event between two kernels kept the GPU idle for 6 us.
+__device__ __forceinline__ void stamp_start(const PathBuffers &pb) {
+    if (pb.stamp && blockIdx.x == 0 && threadIdx.x == 0) *pb.stamp = wall_clock64();
+}
+
 // The dispatcher deals blocks to the eight XCDs round-robin by block index.
 // The traversal kernels map them so that XCD x takes the x-th contiguous
 // eighth of the queue: queues are in path (pixel) order, so an XCD's rays come
@@ -1843,6 +1850,7 @@ __device__ __forceinline__ int32_t xcd_block(uint32_t n) {
 // room for seven; eight fit in 64 without spilling.
 template <bool STATS, int TM, int TB>
 __global__ void __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(TM == TM_ATRC ? 5 : 8, 8))) k_trace_closest(DevScene s, PathBuffers pb, DevCounters *cnt) {
+    stamp_start(pb);
     const uint32_t n = pb.cnt_in[0];
     const int32_t lb = xcd_block<TB>(n);
     if (lb < 0) return;  // whole block past the queue
@@ -1883,6 +1891,7 @@ __global__ void __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(TM == T
 
 template <bool STATS, int TM, int TB>
 __global__ void __launch_bounds__(TB) k_trace_shadow(DevScene s, PathBuffers pb, DevCounters *cnt) {
+    stamp_start(pb);
     const uint32_t n = pb.cnt_in[1];
     const int32_t lb = xcd_block<TB>(n);
     if (lb < 0) return;
@@ -1983,6 +1992,7 @@ __device__ __forceinline__ void refill_traverse(uint32_t next, uint32_t last, co
 
 template <bool STATS, int TM, int TB>
 __global__ void __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(6, 8))) k_trace_closest_runs(DevScene s, PathBuffers pb, DevCounters *cnt) {
+    stamp_start(pb);
     uint32_t next, last;
     refill_range(pb.cnt_in[0], &next, &last);
     if (next >= last) return;
@@ -2010,6 +2020,7 @@ __global__ void __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(6, 8)))
 
 template <bool STATS, int TM, int TB>
 __global__ void __launch_bounds__(TB) k_trace_shadow_runs(DevScene s, PathBuffers pb, DevCounters *cnt) {
+    stamp_start(pb);
     uint32_t next, last;
     refill_range(pb.cnt_in[1], &next, &last);
     if (next >= last) return;
@@ -2032,6 +2043,7 @@ __global__ void __launch_bounds__(TB) k_trace_shadow_runs(DevScene s, PathBuffer
 }
 
 __global__ void __launch_bounds__(256) k_raygen(DevScene s, RenderConst rc, PathBuffers pb) {
+    stamp_start(pb);
     const int32_t p = int32_t(blockIdx.x * blockDim.x + threadIdx.x);
     if (p >= rc.n_paths) return;
     // work item = layer * (sampled pixels) + pixel; the sampled grid is the image,
@@ -2639,6 +2651,7 @@ __device__ __forceinline__ MScat medium_sample(const DevScene &s, int32_t mi, V 
 // The door-gap room with a 256^3 grid, 1024x1024 at 4 samples: 168.0 -> 56.0 ms,
 // of which this kernel 9.0 ms and k_shade 12.1 ms (130 ms with the tracking inside it).
 __global__ void __launch_bounds__(256) k_media(DevScene s, RenderConst rc, PathBuffers pb) {
+    stamp_start(pb);
     const uint32_t n = pb.cnt_in[2];
     const uint32_t tid = blockIdx.x * blockDim.x + threadIdx.x;
     if (tid >= n) return;
@@ -2756,6 +2769,7 @@ __device__ __forceinline__ uint32_t put_radiance(const PathBuffers &pb, uint32_t
 
 template <uint32_t F>
 __global__ void __launch_bounds__(SHADE_BLOCK) k_shade(DevScene s, RenderConst rc, PathBuffers pb) {
+    stamp_start(pb);
     const uint32_t n = pb.cnt_in[2];
     const uint32_t tid = blockIdx.x * blockDim.x + threadIdx.x;
     if (tid >= n) return;
@@ -3170,8 +3184,8 @@ __global__ void __launch_bounds__(QC_THREADS) k_queue_count(PathBuffers pb, uint
 }
 
 // one block: blk[b] <- exclusive prefix of the block counts; cnt_out[0..2] <- totals, and
-// the same into host (pinned memory, may be null)
-__global__ void __launch_bounds__(1024) k_queue_scan(PathBuffers pb, uint4 *blk, uint32_t *host) {
+// the same into host[0..2] (pinned memory, may be null), then seq into host[3]
+__global__ void __launch_bounds__(1024) k_queue_scan(PathBuffers pb, uint4 *blk, uint32_t *host, uint32_t seq) {
     const uint32_t n = pb.cnt_in[2];
     const uint32_t nb = (n + QC_SPAN - 1) / QC_SPAN;
     __shared__ uint32_t wsum[3][16];
@@ -3202,6 +3216,8 @@ __global__ void __launch_bounds__(1024) k_queue_scan(PathBuffers pb, uint4 *blk,
             host[0] = carry[0];
             host[1] = carry[1];
             host[2] = carry[2];
+            __threadfence_system();
+            __hip_atomic_store(host + 3, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
         }
     }
 }
@@ -3362,6 +3378,7 @@ __device__ __forceinline__ bool finite3(V v) { return isfinite(v.x) && isfinite(
 // written back once (the same operations in the same order as updates in memory).
 template <bool AOV>
 __global__ void __launch_bounds__(256) k_film(RenderConst rc, PathBuffers pb) {
+    stamp_start(pb);
     constexpr int CH = FILM_CH<AOV>;
     const int64_t wh = int64_t(rc.W) * rc.H;
     const int64_t cover = rc.n_paths < wh ? int64_t(rc.n_paths) : wh;
@@ -3423,6 +3440,7 @@ __device__ __forceinline__ float atrc_filter_rel(int32_t x, int32_t lo, int32_t 
 
 template <bool AOV>
 __global__ void __launch_bounds__(256) k_film_splat(RenderConst rc, PathBuffers pb) {
+    stamp_start(pb);
     constexpr int CH = FILM_CH<AOV>;
     const int64_t wh = int64_t(rc.W) * rc.H;
     const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -3675,11 +3693,11 @@ void launch_shade(const DevScene &s, const RenderConst &rc, const PathBuffers &p
 uint32_t queue_compact_blocks(uint32_t max_n) { return (max_n + QC_SPAN - 1) / QC_SPAN + 1; }
 
 void launch_queue_compact(const PathBuffers &pb, uint32_t max_n, int L, uint4 *blk, uint32_t *host_counts,
-                          hipStream_t st) {
+                          uint32_t seq, hipStream_t st) {
     const uint32_t nb = (max_n + QC_SPAN - 1) / QC_SPAN;
     const uint32_t nl = uint32_t(L > 0 ? L : 0);
     if (nb) hipLaunchKernelGGL(k_queue_count, dim3(nb), dim3(QC_THREADS), 0, st, pb, nl, blk);
-    hipLaunchKernelGGL(k_queue_scan, dim3(1), dim3(1024), 0, st, pb, blk, host_counts);
+    hipLaunchKernelGGL(k_queue_scan, dim3(1), dim3(1024), 0, st, pb, blk, host_counts, seq);
     if (nb) hipLaunchKernelGGL(k_queue_scatter, dim3(nb), dim3(QC_THREADS), 0, st, pb, nl, blk);
 }
 
