@@ -14,7 +14,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("accel", [capi.ACCEL_ATRC, capi.ACCEL_BVH4, capi.ACCEL_BVH4_WATERTIGHT])
-@pytest.mark.parametrize("W,H", [(1, 1), (13, 5), (65, 63)])
+@pytest.mark.parametrize("W,H", [(1, 1), (13, 5), (65, 63), (64, 64), (241, 17)])  # 4096: the one-block queues
 @pytest.mark.parametrize("min_depth", [0, 2])
 def test_small_images_path_parity(gpu_ctx, W, H, min_depth, accel):
     s, cam, tr = scenes.cornell_box()
