@@ -1,8 +1,9 @@
 // gfx950 kernels of the wavefront path tracer that reproduces Atrc's `pt`.
 //
-// Pipeline per bounce (one HIP stream, queues compacted with wave-aggregated
-// atomics):
+// Pipeline per bounce (one HIP stream; queues are built by count, scan and
+// scatter, without atomics):
 //   raygen  -> trace_closest (continuation + MIS-BSDF rays) -> trace_shadow (NEE rays)
+//           -> media (scenes with media: transmittances, medium samples)
 //           -> shade (resolve NEE/MIS of the previous vertex, shade the new vertex,
 //              emit next rays, Russian roulette) -> ... -> film
 // Each path owns fixed slots in the ray/hit/NEE arrays, so queue order never
