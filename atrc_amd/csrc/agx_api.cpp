@@ -20,6 +20,7 @@
 #include "agx_guide.h"
 #include "agx_guide_kernels.h"
 #include "agx_build.h"
+#include "agx_chunks.h"
 #include "agx_kernels.h"
 
 using namespace agx;
@@ -992,8 +993,8 @@ int agx_trace_rays(agx_ctx *c, const float *o, const float *d, const float *tmin
         if (int r = c->ensure_rays_device(std::min(n, RAYS_CHUNK)); r != AGX_OK) return r;
         float *w = c->rays_dev;
         HIP_TRY(hipMemsetAsync(c->dcnt, 0, 2 * sizeof(DevCounters), c->stream));
-        for (uint32_t first = 0; first < n; first += RAYS_CHUNK) {
-            const size_t N = std::min(n - first, RAYS_CHUNK), f = first;
+        const int r = for_each_chunk(n, RAYS_CHUNK, [&](size_t f, uint32_t count) {
+            const size_t N = count;
             float *res = w + 8 * N;
             hipError_t e = hipSuccess;
             auto put = [&](float *dst, const float *src, size_t words) {
@@ -1008,7 +1009,7 @@ int agx_trace_rays(agx_ctx *c, const float *o, const float *d, const float *tmin
             put(w + 7 * N, tmax + f, N);
             if (e == hipSuccess) e = hipEventRecord(c->ev[0], c->stream);
             if (e == hipSuccess) {
-                launch_trace_rays(c->ds, RayArrays{w, w + 3 * N, w + 6 * N, w + 7 * N, 3, 1}, uint32_t(N), any_hit,
+                launch_trace_rays(c->ds, RayArrays{w, w + 3 * N, w + 6 * N, w + 7 * N, 3, 1}, count, any_hit,
                                   reinterpret_cast<int32_t *>(res), reinterpret_cast<int32_t *>(res + N), res + 2 * N,
                                   res + 3 * N, res + 4 * N, c->dcnt + (any_hit ? 1 : 0), nullptr, c->stream);
                 e = hipGetLastError();
@@ -1025,7 +1026,9 @@ int agx_trace_rays(agx_ctx *c, const float *o, const float *d, const float *tmin
             if (e == hipSuccess) e = done;
             if (e != hipSuccess) return fail(AGX_E_HIP, std::string("trace_rays: ") + hipGetErrorString(e));
             ms += elapsed(c->ev[0], c->ev[1]);
-        }
+            return int(AGX_OK);
+        });
+        if (r != AGX_OK) return r;
         HIP_TRY(hipMemcpy(hc, c->dcnt, sizeof(hc), hipMemcpyDeviceToHost));
     }
     agx_stats_t st{};

@@ -51,3 +51,28 @@ def test_outputs_may_be_left_out(gpu_ctx, n):
                                       None) == 0
     np.testing.assert_array_equal(ent, full["entity"])
     np.testing.assert_array_equal(t.view(np.uint32), full["t"].view(np.uint32))
+
+
+@pytest.mark.parametrize("any_hit", [False, True])
+def test_calls_of_several_parts(gpu_ctx, any_hit):
+    """A call of more rays than the device staging holds is traced in parts of 2^22:
+    the same as the parts asked for one by one."""
+    part = 1 << 22
+    n = part + 77
+    s, _, _ = scenes.cornell_box()
+    s.accel = capi.ACCEL_BVH4
+    desc, keep = s.to_desc()
+    gpu_ctx.upload_scene(desc)
+    o, d = scenes.random_rays(((0.1, 0.1, 0.1), (5, 5, 5)), n, seed=2)
+    tmin, tmax = np.zeros(n, np.float32), np.full(n, 9.0, np.float32)
+    print(f"[ray parts] {n} rays, any_hit {any_hit}", flush=True)
+    full = gpu_ctx.trace_rays(o, d, tmin, tmax, any_hit=any_hit)
+    st = gpu_ctx.stats()
+    assert st["trace_shadow_launches" if any_hit else "trace_closest_launches"] == 2
+    tests = 0
+    for a, b in ((0, part), (part, n)):
+        g = gpu_ctx.trace_rays(o[a:b], d[a:b], tmin[a:b], tmax[a:b], any_hit=any_hit)
+        tests += gpu_ctx.stats()["shadow_tri_tests" if any_hit else "closest_tri_tests"]
+        for k in ("entity",) if any_hit else ("entity", "prim", "t", "u", "v"):
+            np.testing.assert_array_equal(full[k][a:b].view(np.uint32), g[k].view(np.uint32))
+    assert tests == st["shadow_tri_tests" if any_hit else "closest_tri_tests"]
