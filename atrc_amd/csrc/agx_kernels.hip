@@ -598,17 +598,28 @@ __device__ __forceinline__ bool wt_test(const WtRay &r, V A, V B, V C, float tmi
 
 // ---------------------------------------------------------------- BVH4 (production mode)
 // A ray as the box tests see it: the reciprocal direction with its magnitude
-// held to 2^80 (so that the products below stay finite for a component that is
-// zero: a plane is then met at +-2^80 times its distance, outside any scene),
+// held to M (so that the products below stay finite for a component that is
+// zero: a plane is then met at +-M times its distance, outside any scene),
 // and which bound of an axis it meets first.
 struct B4Ray {
     V o, inv;
     bool nx, ny, nz;  // the ray runs towards smaller x / y / z: the high bound comes first
 };
-__device__ __forceinline__ B4Ray b4_ray(V o, V d) {
+// M of a direction of unit length, as the wavefront's are
+constexpr float B4_HOLD = 0x1p80f;
+// M of a caller's direction: 2^80 times the smallest |1/d|, at least 2^80.  (With
+// 2^80 for all, the components of a direction of 1e-25 are held to one value, and it
+// loses its hits.)  Directions shorter than 2^-40 are not held: an axis whose
+// products overflow gives NaNs, which cull nothing, so that hits stay right and only axis-parallel
+// rays of that length visit more nodes.  A direction of zeros hits nothing and is
+// held, so that it culls.
+__device__ __forceinline__ float b4_hold(V d) {
+    const float m = fminf(fminf(fabsf(1 / d.x), fabsf(1 / d.y)), fabsf(1 / d.z));
+    return m <= 0x1p40f ? B4_HOLD * fmaxf(m, 1.0f) : (m < INF_F ? INF_F : B4_HOLD);
+}
+__device__ __forceinline__ B4Ray b4_ray(V o, V d, float M) {
     B4Ray r;
     r.o = o;
-    constexpr float M = 0x1p80f;
     r.inv = mk(fminf(fmaxf(1 / d.x, -M), M), fminf(fmaxf(1 / d.y, -M), M), fminf(fmaxf(1 / d.z, -M), M));
     r.nx = r.inv.x < 0; r.ny = r.inv.y < 0; r.nz = r.inv.z < 0;
     return r;
@@ -708,9 +719,9 @@ struct B4Closest {
     int32_t best_rank;  // tie rank of the entity of the current hit, -1 = no hit yet
     HitRec rec;
 
-    __device__ __forceinline__ void start(V o_, V d_, float tmin_, float tmax_) {
+    __device__ __forceinline__ void start(V o_, V d_, float tmin_, float tmax_, float hold = B4_HOLD) {
         d = d_; tmin = tmin_; tmax = tmax_;
-        r = b4_ray(o_, d_);
+        r = b4_ray(o_, d_, hold);
         if (WT) wr = wt_ray(o_, d_);
         code = 0; sp = 0; best_rank = -1;
         rec.ent = -1; rec.prim = -1; rec.t = -1; rec.u = 0; rec.v = 0;
@@ -840,7 +851,7 @@ __device__ bool b4_closest(const DevScene &s, V o, V d, float tmin, float tmax, 
                            uint2 *ring) {
     B4Closest<STATS, CAP, WT, TB> q;
     uint2 spill[B4Closest<STATS, CAP, WT, TB>::SPILL];
-    q.start(o, d, tmin, tmax);
+    q.start(o, d, tmin, tmax, b4_hold(d));
     q.rec = *h;
     b4_run<false>(q, false, s, c, ring, spill);
     *h = q.rec;
@@ -860,9 +871,9 @@ struct B4Any {
     int sp;
     bool occluded;
 
-    __device__ __forceinline__ void start(V o_, V d_, float tmin_, float tmax_) {
+    __device__ __forceinline__ void start(V o_, V d_, float tmin_, float tmax_, float hold = B4_HOLD) {
         d = d_; tmin = tmin_; tmax = tmax_;
-        r = b4_ray(o_, d_);
+        r = b4_ray(o_, d_, hold);
         if (WT) wr = wt_ray(o_, d_);
         code = 0; sp = 0; occluded = false;
     }
@@ -936,7 +947,7 @@ template <bool STATS, int CAP, bool WT, int TB>
 __device__ bool b4_any(const DevScene &s, V o, V d, float tmin, float tmax, Counts &c, uint32_t *ring) {
     B4Any<STATS, CAP, WT, TB> q;
     uint32_t spill[B4Any<STATS, CAP, WT, TB>::SPILL];
-    q.start(o, d, tmin, tmax);
+    q.start(o, d, tmin, tmax, b4_hold(d));
     b4_run<false>(q, false, s, c, ring, spill);
     return q.occluded;
 }

@@ -73,3 +73,50 @@ def test_box_test_is_conservative(gpu_ctx, kind, accel):
     np.testing.assert_array_equal(g["t"][inside].view(np.uint32), t[inside].view(np.uint32))
     a = gpu_ctx.trace_rays(o, d, tmin, tmax, any_hit=True)
     assert (a["entity"][inside] == 1).all()
+
+
+@pytest.mark.parametrize("accel", [capi.ACCEL_BVH4, capi.ACCEL_BVH4_WATERTIGHT])
+@pytest.mark.parametrize("kind", ["any", "plane", "axis"])
+@pytest.mark.parametrize("scale", [1e-33, 1e-25, 1e-20, 1e-12, 1e-9, 1e20, 1e30])
+def test_length_of_the_direction(gpu_ctx, kind, scale, accel):
+    """Rays whose whole direction is short or long, with and without zero
+    components: the same hits as by brute force (distances are in units of it)."""
+    meshes = _soup()
+    s = scenes.Scene(aggregate=capi.AGGREGATE_BVH, accel=accel)
+    m = s.add_material(scenes.Material(color=(0.5, 0.5, 0.5)))
+    for t in meshes:
+        s.add(scenes.Entity(capi.GEOM_TRIANGLE_BVH, m, tris=t))
+    desc, keep = s.to_desc()
+    gpu_ctx.upload_scene(desc)
+    tris = np.concatenate([t[:, :3].reshape(-1, 3, 3) for t in meshes])
+    o, d = _rays(kind, tris, 3000)
+    d = (d.astype(np.float64) * scale).astype(np.float32)
+    n = len(o)
+    tmin, tmax = np.full(n, 1e-3 / scale, np.float32), np.full(n, np.inf, np.float32)
+    print(f"[box test] {kind}, length {scale}, accel {accel}", flush=True)
+    prim, t, u, v = po.triangle_soup_closest(tris, o, d, tmin, tmax, watertight=accel == capi.ACCEL_BVH4_WATERTIGHT)
+    inside = (prim >= 0) & (u > 0.02) & (v > 0.02) & (u + v < 0.98)
+    assert inside.mean() > 0.5
+    g = gpu_ctx.trace_rays(o, d, tmin, tmax)
+    np.testing.assert_array_equal(g["t"][inside].view(np.uint32), t[inside].view(np.uint32))
+    a = gpu_ctx.trace_rays(o, d, tmin, tmax, any_hit=True)
+    assert (a["entity"][inside] == 1).all()
+
+
+@pytest.mark.parametrize("accel", [capi.ACCEL_BVH4, capi.ACCEL_BVH4_WATERTIGHT])
+def test_directions_without_length(gpu_ctx, accel):
+    """Zero and NaN directions hit nothing."""
+    s = scenes.Scene(aggregate=capi.AGGREGATE_BVH, accel=accel)
+    m = s.add_material(scenes.Material(color=(0.5, 0.5, 0.5)))
+    for t in _soup():
+        s.add(scenes.Entity(capi.GEOM_TRIANGLE_BVH, m, tris=t))
+    desc, keep = s.to_desc()
+    gpu_ctx.upload_scene(desc)
+    o = np.random.default_rng(3).uniform(-1, 2, (300, 3)).astype(np.float32)
+    d = np.zeros_like(o)
+    d[100:] = np.nan
+    d[200:, 0] = 1.0
+    tmin, tmax = np.zeros(300, np.float32), np.full(300, np.inf, np.float32)
+    print(f"[box test] zero and NaN directions, accel {accel}", flush=True)
+    assert (gpu_ctx.trace_rays(o, d, tmin, tmax)["entity"] == -1).all()
+    assert (gpu_ctx.trace_rays(o, d, tmin, tmax, any_hit=True)["entity"] == -1).all()
