@@ -1022,6 +1022,7 @@ int agx_trace_rays(agx_ctx *c, const float *o, const float *d, const float *tmin
                 get(u ? u + f : nullptr, res + 3 * N);
                 get(v ? v + f : nullptr, res + 4 * N);
             }
+            if (e == hipSuccess) e = hipMemcpyAsync(hc, c->dcnt, sizeof(hc), hipMemcpyDeviceToHost, c->stream);
             const hipError_t done = hipStreamSynchronize(c->stream);  // also after an error: copies may be in flight
             if (e == hipSuccess) e = done;
             if (e != hipSuccess) return fail(AGX_E_HIP, std::string("trace_rays: ") + hipGetErrorString(e));
@@ -1029,7 +1030,6 @@ int agx_trace_rays(agx_ctx *c, const float *o, const float *d, const float *tmin
             return int(AGX_OK);
         });
         if (r != AGX_OK) return r;
-        HIP_TRY(hipMemcpy(hc, c->dcnt, sizeof(hc), hipMemcpyDeviceToHost));
     }
     agx_stats_t st{};
     st.node_bytes = c->accel != AGX_ACCEL_ATRC ? 16 * BVH4_NODE_VEC4 : 32;
