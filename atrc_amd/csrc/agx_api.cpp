@@ -54,9 +54,11 @@ template <class T> hipError_t upload(T **p, const std::vector<T> &v, hipStream_t
 
 }  // namespace
 
-// agx_trace_rays: calls of up to RAYS_PINNED rays go through pinned memory, larger
-// ones through device buffers of at most RAYS_CHUNK rays
+// agx_trace_rays: calls of up to RAYS_PINNED rays go through pinned memory (those of
+// more than RAYS_PINNED_FIRST once a context has had several), larger ones through device
+// buffers of at most RAYS_CHUNK rays
 constexpr uint32_t RAYS_PINNED = 1u << 15;
+constexpr uint32_t RAYS_PINNED_FIRST = 1u << 12;
 constexpr uint32_t RAYS_CHUNK = 1u << 22;
 
 struct agx_ctx {
@@ -117,6 +119,8 @@ struct agx_ctx {
     double clock_khz = 100000;       // rate of those times
     uint32_t seq = 0;                // of the queue sizes in h_counters
     float *rays_pin = nullptr;       // agx_trace_rays: pinned staging of small calls
+    uint32_t rays_pin_cap = 0;       // rays it holds
+    uint64_t rays_seen = 0;          // rays of calls that it was too small for
     float *rays_dev = nullptr;       // and the device staging of larger ones (at most RAYS_CHUNK rays, 218 MB)
     uint32_t rays_dev_cap = 0;
     hipEvent_t ev[8]{};
@@ -216,14 +220,31 @@ struct agx_ctx {
         }
         return AGX_OK;
     }
-    // staging of agx_trace_rays: pinned words of RAYS_PINNED rays and their waves' counts
-    int ensure_rays_pinned() {
-        if (rays_pin) return AGX_OK;
-        const size_t words = 13 * size_t(RAYS_PINNED) + 4 * size_t(RAYS_PINNED / 64 + 4);
+    // Pinned staging of agx_trace_rays for a call of n rays (13 words a ray, then a
+    // count of each wave): *use is whether the call goes through it.  Its pages cost
+    // 0.1 ms + 0.65 ms per 32,768 rays when they are made and first touched, and a call of
+    // 8,192 to 32,768 rays gains 0.15 ms by it, so it is as large as the calls need, and a call of
+    // more than RAYS_PINNED_FIRST rays grows it only once earlier ones had 4 n rays
+    // (a context's first call of 32,768 rays: 1.17 ms with the whole buffer made at once, 0.45 without).
+    int ensure_rays_pinned(uint32_t n, bool *use) {
+        *use = n <= rays_pin_cap;
+        if (*use || n > RAYS_PINNED) return AGX_OK;
+        if (n > RAYS_PINNED_FIRST && rays_seen < 4ull * n) {
+            rays_seen += n;
+            return AGX_OK;
+        }
+        uint32_t cap = 1024;
+        while (cap < n) cap *= 2;
+        if (rays_pin) (void)hipHostFree(rays_pin);
+        rays_pin = nullptr;
+        rays_pin_cap = 0;
+        const size_t words = 13 * size_t(cap) + 4 * size_t(cap / 64 + 4);
         if (hipHostMalloc(reinterpret_cast<void **>(&rays_pin), words * 4, hipHostMallocDefault) != hipSuccess) {
             rays_pin = nullptr;
             return fail(AGX_E_OUT_OF_MEMORY, "allocation of ray staging failed");
         }
+        rays_pin_cap = cap;
+        *use = true;
         return AGX_OK;
     }
     // device words of n rays, kept for the next call
@@ -957,8 +978,9 @@ int agx_trace_rays(agx_ctx *c, const float *o, const float *d, const float *tmin
     // 245 -> 106 us).  Larger ones: the callers' arrays to and from device
     // buffers that the context keeps, at most RAYS_CHUNK rays at a time
     // (2,000,003 rays: 12.5 -> 6.5 ms).
-    if (n <= RAYS_PINNED) {
-        if (int r = c->ensure_rays_pinned(); r != AGX_OK) return r;
+    bool pinned = false;
+    if (int r = c->ensure_rays_pinned(n, &pinned); r != AGX_OK) return r;
+    if (pinned) {
         float *w = c->rays_pin;  // in words: o 3n, d 3n, tmin n, tmax n, then entity, primitive, t, u, v
         const size_t N = n;
         std::memcpy(w, o, 12 * N);
@@ -966,7 +988,7 @@ int agx_trace_rays(agx_ctx *c, const float *o, const float *d, const float *tmin
         std::memcpy(w + 6 * N, tmin, 4 * N);
         std::memcpy(w + 7 * N, tmax, 4 * N);
         float *res = w + 8 * N;
-        uint4 *counts = reinterpret_cast<uint4 *>(c->rays_pin + 13 * size_t(RAYS_PINNED));
+        uint4 *counts = reinterpret_cast<uint4 *>(c->rays_pin + 13 * size_t(c->rays_pin_cap));
         const uint32_t waves = (n + 255) / 256 * 4;  // every wave of the launch writes its counts
         HIP_TRY(hipEventRecord(c->ev[0], c->stream));
         launch_trace_rays(c->ds, RayArrays{w, w + 3 * N, w + 6 * N, w + 7 * N, 3, 1}, n, any_hit,
@@ -1038,7 +1060,7 @@ int agx_trace_rays(agx_ctx *c, const float *o, const float *d, const float *tmin
     if (any_hit) st.shadow_rays = n; else st.closest_rays = n;
     fill_traversal_stats(hc, &st);
     st.total_ms = ms;
-    const uint64_t launches = n <= RAYS_PINNED ? 1 : (n - 1) / RAYS_CHUNK + 1;
+    const uint64_t launches = (n - 1) / RAYS_CHUNK + 1;
     if (any_hit) { st.trace_shadow_ms = ms; st.trace_shadow_launches = launches; }
     else { st.trace_closest_ms = ms; st.trace_closest_launches = launches; }
     c->stats = st;
