@@ -794,16 +794,18 @@ int agx_render(agx_ctx *c, const agx_render_params *p, const volatile int32_t *c
             const uint32_t n_closest = bounce == 0 ? alive : 2 * alive;
             const uint32_t n_shadow = bounce == 0 ? 0 : alive * uint32_t(std::max(rc.L, 0));
             size_t e1 = 0, e2 = 0, e3 = 0;
-            c->pb.stamp = stamp(3 * bounce + 1);
-            launch_trace_closest(c->ds, c->pb, n_closest, stats, c->dcnt, c->stream);
-            c->pb.stamp = nullptr;
-            if (!stamps && (r = mark(&e1))) return r;
             if (c->capture_count) {
+                // ahead of the traversals, whose times are the render's own: the queues are complete
                 launch_capture_rays(c->pb, 0, c->capture_o[0], c->capture_d[0], c->capture_count, c->capture_cap,
                                     n_closest, c->stream);
                 launch_capture_rays(c->pb, 1, c->capture_o[1], c->capture_d[1], c->capture_count + 1,
                                     c->capture_cap, n_shadow, c->stream);
+                if (!stamps && (r = mark(&e_last))) return r;
             }
+            c->pb.stamp = stamp(3 * bounce + 1);
+            launch_trace_closest(c->ds, c->pb, n_closest, stats, c->dcnt, c->stream);
+            c->pb.stamp = nullptr;
+            if (!stamps && (r = mark(&e1))) return r;
             if (!stamps) timed.push_back({e_last, e1, 0});
             e2 = e1;
             st.trace_closest_launches += 1;

@@ -126,3 +126,24 @@ def test_ray_replay_captures_every_query(gpu_ctx):
     log(f"[replay] cornell 64x64 2 spp: {rr}")
     assert rr["closest_rays"] == st["closest_rays"] and rr["shadow_rays"] == st["shadow_rays"]
     assert rr["replay_closest_ms"] > 0 and rr["replay_shadow_ms"] > 0
+
+
+def test_ray_replay_times_are_the_renders_own(gpu_ctx):
+    """The closest-hit and any-hit times that a replay reports of its render do
+    not hold the capturing."""
+    s, cam, tr = scenes.procedural_spheres(n_spheres=24, subdiv=3, seed=3, extent=20.0, sun=True)
+    cam = {"pos": (-12.0, -16.0, 24.0), "dst": (10.0, 10.0, 8.0), "fov": 40.0}
+    s.accel = capi.ACCEL_BVH4
+    desc, keep = s.to_desc()
+    gpu_ctx.upload_scene(desc)
+    p = scenes.render_params(1024, 768, 2, cam, seed=5, **tr)
+    plain, replay = [], []
+    for _ in range(4):  # the first of each warms up; the fastest counts
+        gpu_ctx.render(p, aovs=False)
+        st = gpu_ctx.stats()
+        plain.append((st["trace_closest_ms"], st["trace_shadow_ms"]))
+        rr = gpu_ctx.replay_rays(p, max_rays=1 << 24, reps=1)
+        replay.append((rr["render_closest_ms"], rr["render_shadow_ms"]))
+    a, b = np.min(plain, axis=0), np.min(replay, axis=0)
+    log(f"[replay] closest / any hit {a} ms in a render, {b} ms in a replay's")
+    assert (b < 1.4 * a + 0.05).all()
