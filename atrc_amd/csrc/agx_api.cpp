@@ -856,7 +856,27 @@ int agx_render(agx_ctx *c, const agx_render_params *p, const volatile int32_t *c
             if (alive == 0) break;  // this bounce was a no-op, and so would be the rest
             if (cancel_flag && *cancel_flag) { cancelled = true; break; }
         }
-        if (cancelled) break;
+        // device times of the pass from the kernels' notes; one follows the last bounce's
+        auto add_stamps = [&]() {
+            auto ms = [&](int from, int to) { return double(c->h_stamps[to] - c->h_stamps[from]) / c->clock_khz; };
+            st.shade_ms += ms(0, 1);
+            for (int k = 0; k < bounces; ++k) {
+                const int shade = 3 * k + 3, shadow = had_shadow[size_t(k)] ? 3 * k + 2 : shade;
+                st.trace_closest_ms += ms(3 * k + 1, shadow);
+                st.trace_shadow_ms += ms(shadow, shade);
+                st.shade_ms += ms(shade, 3 * k + 4);
+            }
+        };
+        if (cancelled) {
+            if (stamps) {
+                c->pb.stamp = stamp(3 * bounces + 1);
+                launch_stamp(c->pb, c->stream);
+                c->pb.stamp = nullptr;
+                HIP_TRY(hipStreamSynchronize(c->stream));
+                add_stamps();
+            }
+            break;
+        }
         if ((r = mark(&a))) return r;
         c->pb.stamp = stamp(3 * bounces + 1);
         launch_film(rc, c->pb, c->stream);
@@ -894,16 +914,7 @@ int agx_render(agx_ctx *c, const agx_render_params *p, const volatile int32_t *c
             st.guide_samples += std::min<uint32_t>(guide_samples_h, guide_batch);
             st.guide_trained += uint64_t(guide_valid_h) * uint64_t(guide_steps);
         }
-        if (stamps) {
-            auto ms = [&](int from, int to) { return double(c->h_stamps[to] - c->h_stamps[from]) / c->clock_khz; };
-            st.shade_ms += ms(0, 1);
-            for (int k = 0; k < bounces; ++k) {
-                const int shade = 3 * k + 3, shadow = had_shadow[size_t(k)] ? 3 * k + 2 : shade;
-                st.trace_closest_ms += ms(3 * k + 1, shadow);
-                st.trace_shadow_ms += ms(shadow, shade);
-                st.shade_ms += ms(shade, 3 * k + 4);
-            }
-        }
+        if (stamps) add_stamps();
         // sum the ray queue sizes of this pass (the last bounce's are complete: the pass has ended)
         for (int k = 0; k <= bounces; ++k) {
             const uint32_t *q = c->h_counters + 4 * k;

@@ -149,6 +149,8 @@ void launch_guide_gather(const RenderConst &rc, const PathBuffers &pb, float *sa
                          uint32_t *count, const uint32_t *ring, uint32_t *blk, hipStream_t st);
 // blocks of the sample gather (blk of launch_guide_gather holds this many entries)
 constexpr uint32_t GUIDE_GATHER_BLOCKS = uint32_t(GUIDE_REC_PATHS) * GUIDE_MAX_REC / 256 + 1;
+// notes the time in pb.stamp
+void launch_stamp(const PathBuffers &pb, hipStream_t st);
 void launch_reset_counters(uint32_t *c, hipStream_t st);
 void launch_copy_calibration(const float4 *src, float4 *dst, uint64_t n, hipStream_t st);
 // rays of the closest-hit (which = 0) or any-hit (1) queue appended to o/d (at most cap)

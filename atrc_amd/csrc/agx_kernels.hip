@@ -1841,6 +1841,9 @@ __device__ __forceinline__ void stamp_start(const PathBuffers &pb) {
     if (pb.stamp && blockIdx.x == 0 && threadIdx.x == 0) *pb.stamp = wall_clock64();
 }
 
+// the note alone, after the last kernel of a render that is cancelled
+__global__ void __launch_bounds__(64) k_stamp(PathBuffers pb) { stamp_start(pb); }
+
 // The dispatcher deals blocks to the eight XCDs round-robin by block index.
 // The traversal kernels map them so that XCD x takes the x-th contiguous
 // eighth of the queue: queues are in path (pixel) order, so an XCD's rays come
@@ -3808,6 +3811,7 @@ void launch_count_rays(const uint32_t *cin, unsigned long long *acc, hipStream_t
 void launch_copy_calibration(const float4 *src, float4 *dst, uint64_t n, hipStream_t st) {
     hipLaunchKernelGGL(k_copy_calibration, dim3(2048), dim3(256), 0, st, src, dst, n);
 }
+void launch_stamp(const PathBuffers &pb, hipStream_t st) { hipLaunchKernelGGL(k_stamp, dim3(1), dim3(64), 0, st, pb); }
 void launch_reset_counters(uint32_t *c, hipStream_t st) {
     hipLaunchKernelGGL(k_reset_counters, dim3(1), dim3(64), 0, st, c);
 }

@@ -3,6 +3,8 @@ roulette (queues counted on the device), scenes without lights (no shadow
 launches) and images of a few paths, path for path against the oracle; the ray
 counts are those of the queues and the same in every pass split.
 """
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -52,3 +54,24 @@ def test_ray_counts_add_up(gpu_ctx):
     gpu_ctx.render(scenes.render_params(70, 51, 3, cam, seed=3, **tr))
     st = gpu_ctx.stats()
     assert [st["closest_rays"], st["shadow_rays"], st["paths"]] == acc.tolist()
+
+
+@pytest.mark.parametrize("media", [False, True])
+def test_cancelled_renders_keep_their_times(gpu_ctx, media):
+    """A render cancelled after its first bounce: the times of the kernels that ran
+    are in its statistics, and the next render is a whole one."""
+    s, cam, tr = scenes.volumetric_room(n_clutter_tris=2000, grid_n=16) if media else scenes.cornell_box()
+    s.accel = capi.ACCEL_BVH4
+    desc, keep = s.to_desc()
+    gpu_ctx.upload_scene(desc)
+    print(f"[launches] cancelled render, media {media}", flush=True)
+    p = scenes.render_params(256, 256, 4, cam, seed=3, **tr)
+    whole = gpu_ctx.render(p, aovs=False)["image"]
+    full = gpu_ctx.stats()
+    g = gpu_ctx.render(p, cancel=C.c_int32(1), aovs=False)
+    st = gpu_ctx.stats()
+    assert g["cancelled"] and not g["image"].any()
+    assert st["trace_closest_launches"] == 1
+    assert 0 < st["trace_closest_ms"] < full["trace_closest_ms"] and 0 < st["shade_ms"] < full["shade_ms"]
+    assert st["trace_closest_ms"] + st["trace_shadow_ms"] + st["shade_ms"] <= 1.05 * st["total_ms"]
+    np.testing.assert_array_equal(gpu_ctx.render(p, aovs=False)["image"], whole)
