@@ -397,6 +397,11 @@ void fill_traversal_stats(const DevCounters hc[2], agx_stats_t *st) {
     st->shadow_bvh_bytes = hc[1].node_visits * st->node_bytes + hc[1].tri_tests * st->prim_bytes;
 }
 
+// materials whose bounces may extend a path by its specular depth
+bool is_delta(int32_t kind) {
+    return kind == AGX_MAT_GLASS || kind == AGX_MAT_MIRROR || kind == AGX_MAT_INVISIBLE_SURFACE;
+}
+
 // Paths of one wavefront pass.  Larger passes keep the late bounces of a pass
 // (fewer surviving paths) large enough to fill the chip: on the 1M-triangle
 // 1080p scene 4M -> 33.5M paths took the closest-hit time per 16 spp from 33.2
@@ -625,8 +630,7 @@ static int upload_host_scene(agx_ctx *c, const HostScene &hs) {
     if (hs.env_kind == AGX_ENV_IBL) ds.features |= SF_IBL;
     for (const DevMaterial &m : hs.mats) {
         if (m.kind == AGX_MAT_DISNEY) ds.features |= SF_DISNEY;
-        if (m.kind == AGX_MAT_GLASS || m.kind == AGX_MAT_MIRROR || m.kind == AGX_MAT_INVISIBLE_SURFACE)
-            ds.features |= SF_DELTA;
+        if (is_delta(m.kind)) ds.features |= SF_DELTA;
     }
     ds.n_ent = int32_t(hs.ents.size());
     ds.aggregate = hs.aggregate;
@@ -1373,6 +1377,14 @@ int agx_render_batch_graph(agx_ctx *c, agx_batch_item *items, uint32_t n, int32_
     for (uint32_t i = 0; i < n; ++i) {
         if (!items[i].scene || !items[i].params) return fail(AGX_E_INVALID_ARG, "batch item without scene or params");
         if (items[i].params->guide) return fail(AGX_E_UNSUPPORTED, "guided rendering is not available in batches");
+        // a path's depth record has 16 bits a count (agx_render holds depths to its ring);
+        // specular bounces come only from delta surfaces
+        bool delta = false;
+        for (uint32_t m = 0; items[i].scene->materials && m < items[i].scene->material_count; ++m)
+            delta = delta || is_delta(items[i].scene->materials[m].kind);
+        if (int64_t(items[i].params->max_depth) + (delta ? std::max(items[i].params->specular_depth, 0) : 0) > MAX_PATH_DEPTH)
+            return fail(AGX_E_UNSUPPORTED, "max_depth + specular_depth too large (at most " +
+                                               std::to_string(MAX_PATH_DEPTH) + ")");
         items[i].status = AGX_E_CANCELLED;
         items[i].worker = -1;
         items[i].rays = 0;

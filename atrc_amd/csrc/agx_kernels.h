@@ -50,6 +50,9 @@ struct PathBuffers {
                          // the segment ends at sh_o
 };
 
+// max_depth + specular_depth that PathBuffers::depth can count (two bounces more run)
+constexpr int64_t MAX_PATH_DEPTH = 65000;
+
 // Path guiding: one path in 2^guide_rec_shift keeps training records of its
 // first GUIDE_MAX_REC guided vertices: inputs[8], direction[3], mixture pdf,
 // throughput after the vertex[3], incident radiance estimate[3], luminance of

@@ -147,7 +147,7 @@ __device__ Rng rng_seed(unsigned long long seed, unsigned long long seq) {
 
 // A path's depth record: (depth, specular depth, medium scattering count,
 // shadow mask), 16 bits each.  Depths and counts grow by at most one a bounce,
-// and no render has 65,535 bounces.
+// and a render has at most MAX_PATH_DEPTH + 2 of them.
 __device__ __forceinline__ int4 unpack_depth(uint2 v) {
     return make_int4(int(v.x & 0xffffu), int(v.x >> 16), int(v.y & 0xffffu), int(v.y >> 16));
 }
@@ -155,6 +155,7 @@ __device__ __forceinline__ uint2 pack_depth(int4 d) {
     return make_uint2((uint32_t(d.x) & 0xffffu) | (uint32_t(d.y) << 16), (uint32_t(d.z) & 0xffffu) | (uint32_t(d.w) << 16));
 }
 static_assert(MAX_LIGHTS <= 16, "the shadow mask of a path is 16 bits");
+static_assert(MAX_PATH_DEPTH + 3 <= 0xffff, "the depths of a path are 16 bits");
 
 // ---------------------------------------------------------------- queues
 // Appends one entry for every active lane with `pred` set: a single atomic per

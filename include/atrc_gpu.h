@@ -427,7 +427,8 @@ int  agx_render_batch(agx_ctx *ctx, agx_batch_item *items, uint32_t n, int32_t w
  * group's graph time.  After a successful call the pooled contexts (their
  * path buffers and last scenes) stay with ctx for its next batch, so a call
  * neither starts by allocating them again nor ends by freeing them;
- * agx_destroy(ctx) releases them. */
+ * agx_destroy(ctx) releases them.  max_depth of an item (in scenes with delta
+ * surfaces plus specular_depth) may be at most 65000 (AGX_E_UNSUPPORTED above). */
 int  agx_render_batch_graph(agx_ctx *ctx, agx_batch_item *items, uint32_t n, int32_t branches,
                             agx_batch_report *report);
 

@@ -53,6 +53,28 @@ def test_batch_matches_single_renders(gpu_ctx, workers):
         assert rep["workers"] == workers and len({r["worker"] for r in recs}) > 1
 
 
+@pytest.mark.parametrize("max_depth,specular_depth", [(70_000, 0), (5, 70_000), (40_000, 40_000), (2**31 - 1, 2**31 - 1)])
+def test_graph_batch_rejects_depths_beyond_a_paths_record(gpu_ctx, max_depth, specular_depth):
+    """A path's depths are counted in 16 bits; a batch in graphs has no other bound on them."""
+    s, cam, tr = scenes.cornell_delta(False)
+    d, keep = s.to_desc()
+    p = scenes.render_params(16, 16, 1, cam, **dict(tr, max_depth=max_depth, specular_depth=specular_depth))
+    log(f"[batch] depth {max_depth} + {specular_depth}")
+    with pytest.raises(capi.AgxError) as e:
+        gpu_ctx.render_batch([d], [p], graph=True)
+    assert e.value.code == capi.AGX_E_UNSUPPORTED and "max_depth" in str(e.value)
+
+
+def test_graph_batch_without_delta_surfaces_takes_any_specular_depth(gpu_ctx):
+    s, cam, tr = scenes.cornell_box()
+    d, keep = s.to_desc()
+    a, b = (scenes.render_params(16, 16, 1, cam, **dict(tr, specular_depth=k)) for k in (0, 10**6))
+    log("[batch] specular depth 10^6 without delta surfaces")
+    imgs, _, _ = gpu_ctx.render_batch([d, d], [a, b], workers=1, graph=True)
+    assert imgs[0].any()
+    np.testing.assert_array_equal(imgs[0], imgs[1])
+
+
 def test_batch_rejects_guided_items(gpu_ctx):
     s, cam, tr = scenes.cornell_box()
     d, keep = s.to_desc()
