@@ -19,6 +19,7 @@
 #include "../../include/atrc_gpu_debug.h"
 #include "agx_guide.h"
 #include "agx_guide_kernels.h"
+#include "agx_budget.h"
 #include "agx_build.h"
 #include "agx_chunks.h"
 #include "agx_kernels.h"
@@ -76,10 +77,11 @@ struct agx_ctx {
     uint4 *qc_blk = nullptr;  // per-block counts / offsets of the queue compaction
     size_t cap_paths = 0;
     int cap_L = -1;
-    // paths per wavefront pass, chosen once per light count (the free-memory
+    // paths per wavefront pass, chosen once per light count and kind (the free-memory
     // query takes milliseconds, and the choice stays stable from call to call)
     size_t pass_paths = 0;
     int pass_paths_L = -1;
+    bool pass_paths_media = false;
     size_t pass_paths_limit = 0;  // 0: none; batch workers, which render side by side, use 2^22
     int trace_block = 128;        // threads per block of the BVH4 traversal launches (128 or 256)
     int64_t cap_wh = 0;
@@ -405,9 +407,9 @@ bool is_delta(int32_t kind) {
 // Paths of one wavefront pass.  Larger passes keep the late bounces of a pass
 // (fewer surviving paths) large enough to fill the chip: on the 1M-triangle
 // 1080p scene 4M -> 33.5M paths took the closest-hit time per 16 spp from 33.2
-// to 24.3 ms.  Default 2^25 paths (about 320 B + 53 B per light each, ~11 GB
-// with one light), limited to a quarter of the free device memory.
-size_t max_paths_in_flight(int lights) {
+// to 24.3 ms.  Default 2^25 paths (path_bytes each: 9.2 GB with one light, 11.4 GB
+// with media as well), limited to a quarter of the free device memory.
+size_t max_paths_in_flight(int lights, bool media) {
     if (const char *s = std::getenv("AGX_MAX_PATHS")) {
         const long long v = std::atoll(s);
         if (v >= 1024) return size_t(v);
@@ -415,10 +417,22 @@ size_t max_paths_in_flight(int lights) {
     size_t cap = size_t(1) << 25;
     size_t free_b = 0, total_b = 0;
     if (hipMemGetInfo(&free_b, &total_b) == hipSuccess && free_b > 0) {
-        const size_t per_path = 320 + 53 * size_t(std::max(lights, 1));
-        cap = std::min(cap, std::max<size_t>(size_t(1) << 20, free_b / 4 / per_path));
+        cap = std::min(cap, std::max<size_t>(size_t(1) << 20, free_b / 4 / path_bytes(lights, media)));
     }
     return cap;
+}
+
+// The context's pass size for scenes of L lights, with media or without: measured
+// once, and again when either changes.
+size_t pass_paths_of(agx_ctx *c, int L) {
+    const bool media = (c->ds.features & SF_MEDIA) != 0;
+    if (c->pass_paths_L != L || c->pass_paths_media != media) {
+        c->pass_paths = max_paths_in_flight(L, media);
+        if (c->pass_paths_limit) c->pass_paths = std::min(c->pass_paths, c->pass_paths_limit);
+        c->pass_paths_L = L;
+        c->pass_paths_media = media;
+    }
+    return c->pass_paths;
 }
 
 // Validation of a render's parameters and its RenderConst (image, depths,
@@ -692,12 +706,7 @@ int agx_render(agx_ctx *c, const agx_render_params *p, const volatile int32_t *c
     // paths per sample layer: the image, or the image and its border when samples splat
     const int64_t layer = rc.splat ? int64_t(rc.EW) * rc.EH : wh;
     const int64_t total = layer * p->spp;
-    if (c->pass_paths_L != rc.L) {
-        c->pass_paths = max_paths_in_flight(rc.L);
-        if (c->pass_paths_limit) c->pass_paths = std::min(c->pass_paths, c->pass_paths_limit);
-        c->pass_paths_L = rc.L;
-    }
-    const size_t cap = c->pass_paths;
+    const size_t cap = pass_paths_of(c, rc.L);
     int64_t per_pass;
     if (layer <= int64_t(cap)) per_pass = layer * std::min<int64_t>(p->spp, int64_t(cap) / layer);
     else per_pass = rc.splat ? layer : int64_t(cap);  // splatting needs whole layers in a pass
@@ -1210,12 +1219,7 @@ int run_batch(agx_ctx *c, agx_batch_item *items, const std::vector<uint32_t> &or
 // ---------------------------------------------------------------- graph-captured batch
 // Paths per wavefront pass of a render without guiding (agx_render's sizing).
 int64_t plain_pass_size(agx_ctx *c, const RenderConst &rc, int64_t layer, int spp) {
-    if (c->pass_paths_L != rc.L) {
-        c->pass_paths = max_paths_in_flight(rc.L);
-        if (c->pass_paths_limit) c->pass_paths = std::min(c->pass_paths, c->pass_paths_limit);
-        c->pass_paths_L = rc.L;
-    }
-    const int64_t cap = int64_t(c->pass_paths);
+    const int64_t cap = int64_t(pass_paths_of(c, rc.L));
     if (layer <= cap) return layer * std::min<int64_t>(spp, cap / layer);
     return rc.splat ? layer : cap;
 }
