@@ -1109,20 +1109,20 @@ int agx_trace_rays_noalloc(agx_ctx *c, const float *o, const float *d, const flo
     if (!base) return fail(AGX_E_HIP, "staging array not resolved on this device");
     const size_t M = NOALLOC_MAX_RAYS;
     auto word = [&](size_t k) { return base + 4 * M * k; };  // layout: launch_trace_rays_staged
-    hipError_t e = hipMemcpyAsync(word(8), o, size_t(n) * 12, hipMemcpyHostToDevice, c->stream);
-    if (e == hipSuccess) e = hipMemcpyAsync(word(11), d, size_t(n) * 12, hipMemcpyHostToDevice, c->stream);
-    if (e == hipSuccess) e = hipMemcpyAsync(word(14), tmin, size_t(n) * 4, hipMemcpyHostToDevice, c->stream);
-    if (e == hipSuccess) e = hipMemcpyAsync(word(15), tmax, size_t(n) * 4, hipMemcpyHostToDevice, c->stream);
+    hipError_t e = hipMemcpyAsync(word(0), o, size_t(n) * 12, hipMemcpyHostToDevice, c->stream);
+    if (e == hipSuccess) e = hipMemcpyAsync(word(3), d, size_t(n) * 12, hipMemcpyHostToDevice, c->stream);
+    if (e == hipSuccess) e = hipMemcpyAsync(word(6), tmin, size_t(n) * 4, hipMemcpyHostToDevice, c->stream);
+    if (e == hipSuccess) e = hipMemcpyAsync(word(7), tmax, size_t(n) * 4, hipMemcpyHostToDevice, c->stream);
     if (e == hipSuccess) e = hipEventRecord(c->ev[0], c->stream);
     if (e == hipSuccess) launch_trace_rays_staged(c->ds, base, n, any_hit, c->dcnt, c->stream);
     if (e == hipSuccess) e = hipGetLastError();
     if (e == hipSuccess) e = hipEventRecord(c->ev[1], c->stream);
-    if (e == hipSuccess) e = hipMemcpyAsync(entity_id, word(16), size_t(n) * 4, hipMemcpyDeviceToHost, c->stream);
+    if (e == hipSuccess) e = hipMemcpyAsync(entity_id, word(8), size_t(n) * 4, hipMemcpyDeviceToHost, c->stream);
     if (e == hipSuccess && !any_hit) {
-        if (prim_id) e = hipMemcpyAsync(prim_id, word(17), size_t(n) * 4, hipMemcpyDeviceToHost, c->stream);
-        if (e == hipSuccess && t) e = hipMemcpyAsync(t, word(18), size_t(n) * 4, hipMemcpyDeviceToHost, c->stream);
-        if (e == hipSuccess && u) e = hipMemcpyAsync(u, word(19), size_t(n) * 4, hipMemcpyDeviceToHost, c->stream);
-        if (e == hipSuccess && v) e = hipMemcpyAsync(v, word(20), size_t(n) * 4, hipMemcpyDeviceToHost, c->stream);
+        if (prim_id) e = hipMemcpyAsync(prim_id, word(9), size_t(n) * 4, hipMemcpyDeviceToHost, c->stream);
+        if (e == hipSuccess && t) e = hipMemcpyAsync(t, word(10), size_t(n) * 4, hipMemcpyDeviceToHost, c->stream);
+        if (e == hipSuccess && u) e = hipMemcpyAsync(u, word(11), size_t(n) * 4, hipMemcpyDeviceToHost, c->stream);
+        if (e == hipSuccess && v) e = hipMemcpyAsync(v, word(12), size_t(n) * 4, hipMemcpyDeviceToHost, c->stream);
     }
     DevCounters hc[2]{};
     if (e == hipSuccess) e = hipMemcpyAsync(hc, c->dcnt, sizeof(hc), hipMemcpyDeviceToHost, c->stream);

@@ -165,12 +165,12 @@ void launch_film_resolve(const RenderConst &rc, const PathBuffers &pb, int64_t w
                          float *normal, float *denoise, hipStream_t st);
 // parity hook: rays in device memory, results to device memory
 // Staging of agx_trace_rays_noalloc: a file-scope device array of
-// NOALLOC_MAX_RAYS rays (84 B each: packed rays, raw inputs, outputs) that the
+// NOALLOC_MAX_RAYS rays (52 B each: inputs and outputs) that the
 // library never allocates or frees.  noalloc_scratch_init resolves its address
 // on the current device (once per device; call with that device current);
 // noalloc_scratch returns it, or nullptr before init.
 constexpr uint32_t NOALLOC_MAX_RAYS = 1u << 17;
-constexpr size_t NOALLOC_BYTES_PER_RAY = 84;
+constexpr size_t NOALLOC_BYTES_PER_RAY = 52;
 hipError_t noalloc_scratch_init(int device);
 void *noalloc_scratch(int device);
 // trace_rays over raw host-layout inputs staged in the scratch: clears cnt with a

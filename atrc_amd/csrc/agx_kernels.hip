@@ -3844,13 +3844,12 @@ void launch_capture_rays(const PathBuffers &pb, int which, float4 *o, float4 *d,
 // ---------------------------------------------------------------- staging without allocation
 // The staging buffer of agx_trace_rays_noalloc.  Layout for n rays (n <=
 // NOALLOC_MAX_RAYS), offsets in units of NOALLOC_MAX_RAYS 4-byte words:
-//   [0, 8) unused
-//   [8, 11) o (3 floats per ray)     [11, 14) d   [14] tmin   [15] tmax
-//   [16] entity  [17] primitive  [18] t  [19] u  [20] v
+//   [0, 3) o (3 floats per ray)   [3, 6) d   [6] tmin   [7] tmax
+//   [8] entity  [9] primitive  [10] t  [11] u  [12] v
 // Every GPU holds its own copy until the process ends; host code uses the
 // address hipGetSymbolAddress gives on that device, never the array's name.
-static __device__ __align__(256) uint32_t scratch[21 * size_t(NOALLOC_MAX_RAYS)];
-static_assert(21 * 4 == NOALLOC_BYTES_PER_RAY, "staging layout");
+static __device__ __align__(256) uint32_t scratch[13 * size_t(NOALLOC_MAX_RAYS)];
+static_assert(13 * 4 == NOALLOC_BYTES_PER_RAY, "staging layout");
 
 namespace {
 constexpr int NOALLOC_MAX_DEVICES = 64;
@@ -3886,9 +3885,9 @@ void launch_trace_rays_staged(const DevScene &s, void *scratch_ptr, uint32_t n, 
     const size_t M = NOALLOC_MAX_RAYS;
     hipLaunchKernelGGL(k_zero_counters, dim3(1), dim3(64), 0, st, cnt);
     auto floats = [&](size_t word) { return reinterpret_cast<float *>(base + word * M); };
-    launch_trace_rays(s, RayArrays{floats(8), floats(11), floats(14), floats(15), 3, 1}, n, any_hit,
-                      reinterpret_cast<int32_t *>(base + 16 * M), reinterpret_cast<int32_t *>(base + 17 * M),
-                      floats(18), floats(19), floats(20), cnt + (any_hit ? 1 : 0), nullptr, st);
+    launch_trace_rays(s, RayArrays{floats(0), floats(3), floats(6), floats(7), 3, 1}, n, any_hit,
+                      reinterpret_cast<int32_t *>(base + 8 * M), reinterpret_cast<int32_t *>(base + 9 * M),
+                      floats(10), floats(11), floats(12), cnt + (any_hit ? 1 : 0), nullptr, st);
 }
 
 void launch_trace_rays(const DevScene &s, const RayArrays &in, uint32_t n, int any_hit, int32_t *ent, int32_t *prim,

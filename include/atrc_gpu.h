@@ -381,7 +381,7 @@ int  agx_trace_rays(agx_ctx *ctx, const float *o, const float *d,
  * harnesses that forbid hipMalloc.  Same arguments, results and statistics as
  * agx_trace_rays; rays and hits are staged in a fixed device array that the
  * library holds on every GPU it runs on until the process ends
- * (AGX_NOALLOC_MAX_RAYS rays, 84 bytes each, about 11 MB), so n above
+ * (AGX_NOALLOC_MAX_RAYS rays, 52 bytes each, about 7 MB), so n above
  * AGX_NOALLOC_MAX_RAYS returns AGX_E_LIMIT.  Every call on one GPU shares
  * that array: calls that overlap on one GPU (from several threads or
  * contexts) race, and must be serialised by the caller. */

@@ -37,6 +37,17 @@ def test_ray_counts(accel):
                 assert sa["total_ms"] > 0
 
 
+@pytest.mark.parametrize("any_hit", [False, True])
+def test_staging_without_allocation_at_its_capacity(gpu_ctx, any_hit):
+    n = 131072
+    _query_scene(gpu_ctx)
+    q = _query(n)
+    print(f"[ray sizes] {n} rays, any_hit {any_hit}", flush=True)
+    a, b = (gpu_ctx.trace_rays(*q, any_hit=any_hit, noalloc=k) for k in (False, True))
+    for k in ("entity",) if any_hit else ("entity", "prim", "t", "u", "v"):
+        np.testing.assert_array_equal(a[k].view(np.uint32), b[k].view(np.uint32))
+
+
 @pytest.mark.parametrize("n", [100, 40_000])
 def test_outputs_may_be_left_out(gpu_ctx, n):
     s, _, _ = scenes.cornell_box()
