@@ -125,7 +125,7 @@ class agx_stats_t(C.Structure):
         ("total_ms", C.c_double), ("trace_closest_ms", C.c_double), ("trace_shadow_ms", C.c_double),
         ("shade_ms", C.c_double), ("trace_closest_launches", C.c_uint64), ("trace_shadow_launches", C.c_uint64),
         ("guide_infer_ms", C.c_double), ("guide_train_ms", C.c_double), ("guide_samples", C.c_uint64),
-        ("guide_steps", C.c_uint64), ("guide_rows", C.c_uint64), ("guide_trained", C.c_uint64), ("node_bytes", C.c_uint32), ("prim_bytes", C.c_uint32), ("info_bytes", C.c_uint32), ("reserved", C.c_uint32),
+        ("guide_steps", C.c_uint64), ("guide_rows", C.c_uint64), ("guide_trained", C.c_uint64), ("node_bytes", C.c_uint32), ("prim_bytes", C.c_uint32), ("info_bytes", C.c_uint32), ("run_launches", C.c_uint32),
         ("host_ms", C.c_double), ("readback_ms", C.c_double),
     ]
 

@@ -816,7 +816,7 @@ int agx_render(agx_ctx *c, const agx_render_params *p, const volatile int32_t *c
                 if (!stamps && (r = mark(&e_last))) return r;
             }
             c->pb.stamp = stamp(3 * bounce + 1);
-            launch_trace_closest(c->ds, c->pb, n_closest, stats, c->dcnt, c->stream);
+            st.run_launches += launch_trace_closest(c->ds, c->pb, n_closest, stats, c->dcnt, c->stream) ? 1 : 0;
             c->pb.stamp = nullptr;
             if (!stamps && (r = mark(&e1))) return r;
             if (!stamps) timed.push_back({e_last, e1, 0});
@@ -825,7 +825,7 @@ int agx_render(agx_ctx *c, const agx_render_params *p, const volatile int32_t *c
             had_shadow.push_back(n_shadow ? 1 : 0);
             if (n_shadow) {
                 c->pb.stamp = stamp(3 * bounce + 2);
-                launch_trace_shadow(c->ds, c->pb, n_shadow, stats, c->dcnt + 1, c->stream);
+                st.run_launches += launch_trace_shadow(c->ds, c->pb, n_shadow, stats, c->dcnt + 1, c->stream) ? 1 : 0;
                 c->pb.stamp = nullptr;
                 if (!stamps) {
                     if ((r = mark(&e2))) return r;

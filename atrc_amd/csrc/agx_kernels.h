@@ -124,11 +124,13 @@ struct RenderConst {
 };
 
 void launch_raygen(const DevScene &s, const RenderConst &rc, const PathBuffers &pb, hipStream_t st);
-// The launch grids cover the capacity (max_n); each kernel reads its real
-// queue size from pb.cnt_in, so the host never waits between bounces.
-void launch_trace_closest(const DevScene &s, const PathBuffers &pb, uint32_t max_n, bool stats, DevCounters *cnt,
+// The launch grids cover max_n entries, a bound that the host knows (agx_render: by the queue
+// sizes it has read of earlier bounces; captured renders: the pass's capacity); each
+// kernel reads its real queue size from pb.cnt_in.  The result of the traversals'
+// launches: whether waves work through runs of rays (use_runs).
+bool launch_trace_closest(const DevScene &s, const PathBuffers &pb, uint32_t max_n, bool stats, DevCounters *cnt,
                           hipStream_t st);
-void launch_trace_shadow(const DevScene &s, const PathBuffers &pb, uint32_t max_n, bool stats, DevCounters *cnt,
+bool launch_trace_shadow(const DevScene &s, const PathBuffers &pb, uint32_t max_n, bool stats, DevCounters *cnt,
                          hipStream_t st);
 void launch_shade(const DevScene &s, const RenderConst &rc, const PathBuffers &pb, uint32_t max_n, hipStream_t st);
 // queues of the next bounce from the paths k_shade shaded (at most max_n of them);

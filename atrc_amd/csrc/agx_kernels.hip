@@ -3725,25 +3725,27 @@ inline bool use_runs(const DevScene &s, uint32_t max_n) {
     return (s.accel == AGX_ACCEL_BVH4 || s.accel == AGX_ACCEL_BVH4_WATERTIGHT) && max_n >= REFILL_MIN;
 }
 
-void launch_trace_closest(const DevScene &s, const PathBuffers &pb, uint32_t max_n, bool stats, DevCounters *cnt,
+bool launch_trace_closest(const DevScene &s, const PathBuffers &pb, uint32_t max_n, bool stats, DevCounters *cnt,
                           hipStream_t st) {
-    if (!max_n) return;
+    if (!max_n) return false;
     if (use_runs(s, max_n)) {
         AGX_LAUNCH_RUNS(k_trace_closest_runs, dim3(runs_grid(max_n)), st, s, pb, cnt);
-        return;
+        return true;
     }
     const unsigned tb = trace_block_of(s);
     AGX_LAUNCH_STACKED(k_trace_closest, tb, dim3(grid_of(max_n, tb) + 7), st, s, pb, cnt);
+    return false;
 }
-void launch_trace_shadow(const DevScene &s, const PathBuffers &pb, uint32_t max_n, bool stats, DevCounters *cnt,
+bool launch_trace_shadow(const DevScene &s, const PathBuffers &pb, uint32_t max_n, bool stats, DevCounters *cnt,
                          hipStream_t st) {
-    if (!max_n) return;
+    if (!max_n) return false;
     if (use_runs(s, max_n)) {
         AGX_LAUNCH_RUNS(k_trace_shadow_runs, dim3(runs_grid(max_n)), st, s, pb, cnt);
-        return;
+        return true;
     }
     const unsigned tb = trace_block_of(s);
     AGX_LAUNCH_STACKED(k_trace_shadow, tb, dim3(grid_of(max_n, tb) + 7), st, s, pb, cnt);
+    return false;
 }
 void launch_shade(const DevScene &s, const RenderConst &rc, const PathBuffers &pb, uint32_t max_n, hipStream_t st) {
     if (!max_n) return;

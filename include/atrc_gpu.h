@@ -304,7 +304,8 @@ typedef struct agx_stats_t {
     uint64_t guide_rows;       /* vertices the network evaluated */
     uint64_t guide_trained;    /* samples passed through training (ring size x Adam steps) */
     uint32_t node_bytes, prim_bytes, info_bytes; /* record sizes used for the byte counts */
-    uint32_t reserved;
+    uint32_t run_launches;     /* traversal launches of a render whose waves work through runs of rays (queues
+                                  that may hold 2^21 rays, BVH4 modes) */
     double   host_ms;          /* wall time of the agx_render call */
     double   readback_ms;      /* wall time from the end of the device work to the return
                                   (film resolve, copy to the host outputs) */

@@ -9,6 +9,7 @@ import numpy as np
 import pytest
 
 from atrc_amd import capi, scenes
+from oracle import py_oracle as po
 
 from test_gpu_render_parity import _path_parity
 
@@ -24,6 +25,25 @@ def test_small_images_path_parity(gpu_ctx, W, H, min_depth, accel):
     # a single path may round to another decision: small images must agree on all but one
     _path_parity(gpu_ctx, s, cam, dict(tr, min_depth=min_depth), W, H, f"small {W}x{H} min_depth {min_depth}",
                  min_frac=min(0.97, 1 - 1.5 / (W * H)))
+
+
+@pytest.mark.parametrize("accel", [capi.ACCEL_ATRC, capi.ACCEL_BVH4, capi.ACCEL_BVH4_WATERTIGHT])
+@pytest.mark.parametrize("min_depth", [0, 2])
+def test_images_of_one_path(gpu_ctx, min_depth, accel):
+    """Renders of a single path: of forty samples, asked for one by one, all but one agree with the oracle."""
+    s, cam, tr = scenes.cornell_box()
+    s.accel = accel
+    desc, keep = s.to_desc()
+    gpu_ctx.upload_scene(desc)
+    ref = po.OracleScene(desc, 32)
+    print(f"[launches] one path, min_depth {min_depth}, accel {accel}", flush=True)
+    off = lit = 0
+    for k in range(40):
+        p = scenes.render_params(1, 1, 1, cam, seed=1234, sample_begin=k, **dict(tr, min_depth=min_depth))
+        g, r = gpu_ctx.render(p)["image"].astype(np.float64), ref.render(p, threads=1)["image"]
+        off += bool((np.abs(g - r).max() > 1e-3 * (np.abs(r).max() + 1e-2)))
+        lit += bool(r.any())
+    assert off <= 1 and lit >= 10
 
 
 def test_no_lights(gpu_ctx):
