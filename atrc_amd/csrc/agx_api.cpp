@@ -1001,7 +1001,8 @@ int agx_trace_rays(agx_ctx *c, const float *o, const float *d, const float *tmin
     double ms = 0;
     // Small calls: one pinned buffer that the kernel reads the rays from and writes the hits
     // to over the link, so that a call is two host copies, one launch and one wait (1001 rays:
-    // 245 -> 106 us).  Larger ones: the callers' arrays to and from device
+    // 245 -> 106 us; 60 meshes, closest hit: 32,768 rays 139 us, one more, staged on the device,
+    // 276 us).  Larger ones: the callers' arrays to and from device
     // buffers that the context keeps, at most RAYS_CHUNK rays at a time
     // (2,000,003 rays: 12.5 -> 6.5 ms).
     bool pinned = false;
@@ -1886,7 +1887,9 @@ int agx_debug_scene_summary(const agx_scene_desc *desc, agx_debug_summary *out) 
     out->device_bytes = uint64_t(hs.ents.size() * sizeof(DevEntity) + hs.mats.size() * sizeof(DevMaterial) +
                                  (hs.blas_nodes.size() + hs.blas_prims.size() + hs.blas_info.size() +
                                   hs.tlas_nodes.size()) * sizeof(vec4) +
-                                 (hs.tlas_prims.size() + hs.alias_idx.size() + hs.alias_prob.size()) * 4);
+                                 (hs.alias_idx.size() + hs.alias_prob.size()) * 4);
+    if (hs.accel == AGX_ACCEL_ATRC)  // agg_refs
+        out->device_bytes += 16 * (hs.aggregate == AGX_AGGREGATE_BVH ? hs.tlas_prims.size() : hs.ents.size());
     out->world_centre_x = hs.world.x;
     out->world_centre_y = hs.world.y;
     out->world_centre_z = hs.world.z;

@@ -286,10 +286,10 @@ float bitsf(uint32_t u) {
     return f;
 }
 
-// Widens a box by a few ulps so that the rounded slab test of a ray that
-// meets a primitive exactly on its bound never culls it.
-// A child bound as the traversal decodes it: origin + byte x power-of-two step,
-// FP32 multiply then add (no contraction), exactly as b4_children evaluates it.
+// A child bound as its bytes encode it: origin + byte x power-of-two step, FP32
+// multiply then add (no contraction).  The traversal's box test (b4_children)
+// does not decode it: it puts the plane at byte x (step / d) + (origin - o) / d, which
+// differs from this by less than pad() and the test's own margins leave.
 float q_decode(float o, uint32_t q, float step) {
     const float m = float(q) * step;
     return o + m;
@@ -356,6 +356,8 @@ void decode_node(const vec4 *n, Box boxes[4], uint32_t codes[4]) {
         }
 }
 
+// Widens a box by 2^-20 of its coordinates, so that the rounded slab test of a
+// ray that meets a primitive exactly on its bound never culls it.
 void pad(Box *b) {
     for (int k = 0; k < 3; ++k) {
         const float m = std::max(std::fabs(b->lo[k]), std::fabs(b->hi[k]));

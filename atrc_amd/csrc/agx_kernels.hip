@@ -644,10 +644,10 @@ __device__ __forceinline__ float b4_byte(uint32_t w, int j) { return float((w >>
 // the 1M-triangle 1920x1080 frame at 64 samples 131.9 -> 122.5 ms, 1280x719 at 8 samples
 // in the watertight mode 10.7 -> 10.0 ms).
 // Conservative: step / d is exact up to 1/d's own rounding (step is a power of
-// two); the offset carries 2 ulp of its own size, so the near offset is
-// lowered and the far one raised by 2^-22 of it (4 ulp); the FMAs and the
-// axes' 1/d differ by at most 4 ulp of t, covered by widening the exit by
-// 2^-21.  Bounds carry the builder's own padding of 2^-20 of their coordinate, which
+// two); the offset carries two roundings (2^-23 of its size), so the near offset is
+// lowered and the far one raised by 2^-22 of it; the FMAs and the
+// axes' 1/d differ by less than 2^-21 of t, by which the exit is
+// widened.  Bounds carry the builder's own padding of 2^-20 of their coordinate, which
 // covers the decode's rounding that the builder emulates.  NaN axes (overflow)
 // are ignored by fminf / fmaxf and only cull less.
 __device__ __forceinline__ void b4_children(const B4Node &nd, const B4Ray &r, float tmin, float tmax, float t[4],
@@ -1863,7 +1863,7 @@ __device__ __forceinline__ int32_t xcd_block(uint32_t n) {
 
 // TM = traversal variant (TM_*).  Eight waves per SIMD: the traversal is bound by
 // the latency of its node fetches, and the default allocation (66 VGPRs) left
-// room for seven; eight fit in 64 without spilling.
+// room for seven; eight take 64, with two to four registers spilled.
 template <bool STATS, int TM, int TB>
 __global__ void __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(TM == TM_ATRC ? 5 : 8, 8))) k_trace_closest(DevScene s, PathBuffers pb, DevCounters *cnt) {
     stamp_start(pb);
@@ -1947,8 +1947,8 @@ __global__ void __launch_bounds__(TB) k_trace_shadow(DevScene s, PathBuffers pb,
 // Large BVH4 queues: a wave takes a run of 64 to 512 consecutive rays and gives
 // its idle lanes the run's next ones whenever at least REFILL_IDLE lanes have
 // finished (or all have).  With one ray a lane, a wave lasts as long as its
-// longest ray: on the 1M-triangle frame 14 of 64 lanes took part in the average vector instruction,
-// and these kernels are bound by those.  The run is the wave's own, so nothing
+// longest ray: on the 1M-triangle frame 16 (closest hit) and 14 (any hit) of 64 lanes took part in
+// the average vector instruction, and these kernels are bound by those.  The run is the wave's own, so nothing
 // is shared: no atomics, and rays stay in queue order within a wave.  A new ray
 // starts at the root like any lane at a node, so its first visit runs with the
 // others' (a root visit of its own for the few new lanes cost 4 ms a frame).  The state
@@ -1962,6 +1962,10 @@ __global__ void __launch_bounds__(TB) k_trace_shadow(DevScene s, PathBuffers pb,
 constexpr int REFILL_IDLE = 24;
 constexpr uint32_t REFILL_MIN = 1u << 21;
 constexpr unsigned REFILL_BLOCK = 128;
+// A captured render launches by its pass's capacity: passes of 2^20 paths or more take runs
+// in every bounce but the first, however few rays the late ones have.  That costs little: graph batches
+// of such passes, 16 to 24 bounces deep, take 0.93 to 0.98 of what they took without runs and before
+// the leaner box test and shading.
 __device__ __forceinline__ uint32_t refill_run(uint32_t n) { return 64u * min(8u, max(1u, n >> 19)); }
 
 // this wave's part [*first, *last) of a queue of n rays (empty past the queue);
@@ -3281,7 +3285,8 @@ __global__ void __launch_bounds__(QC_THREADS) k_queue_scatter(PathBuffers pb, ui
 
 // The three kernels above in one block, for queues of at most QS_MAX paths (the
 // last bounces of a pass, and small images): their work is a few microseconds and the
-// three launches take 20.  61x47 at 1 sample: 570 -> 497 us.
+// three launches take 20.  61x47 at 1 sample: 570 -> 497 us.  At the limit it still gains: 64x64 (one
+// block from the first bounce) 497 us, 65x64 (three launches there) 511 us.
 constexpr uint32_t QS_THREADS = 1024, QS_ITEMS = 4, QS_MAX = QS_THREADS * QS_ITEMS;
 __global__ void __launch_bounds__(QS_THREADS) k_queue_small(PathBuffers pb, uint32_t L, uint32_t *host, uint32_t seq) {
     const uint32_t n = min(pb.cnt_in[2], QS_MAX);
@@ -3753,7 +3758,7 @@ void launch_shade(const DevScene &s, const RenderConst &rc, const PathBuffers &p
     // unguided or guided; every other scene takes the full kernel
     const bool lean = (s.features & (SF_MEDIA | SF_DISNEY | SF_DELTA | SF_IBL)) == 0;
     // media and delta surfaces without Disney, IBL or guiding (the volumetric
-    // scenes): 199 VGPRs and no scratch against the full variant's spills
+    // scenes): 175 VGPRs and no scratch against the full variant's 208 and 256 bytes of it
     const bool media_delta = (s.features & (SF_DISNEY | SF_IBL)) == 0;
     if (lean && !rc.guide) hipLaunchKernelGGL(k_shade<0u>, dim3(grid_of(max_n, SHADE_BLOCK)), dim3(SHADE_BLOCK), 0, st, s, rc, pb);
     else if (lean) hipLaunchKernelGGL(k_shade<SF_GUIDE>, dim3(grid_of(max_n, SHADE_BLOCK)), dim3(SHADE_BLOCK), 0, st, s, rc, pb);

@@ -372,7 +372,11 @@ int  agx_render(agx_ctx *ctx, const agx_render_params *params,
  * any_hit = 0: closest hit; outputs entity id (-1 = miss), primitive id (mesh:
  * original triangle index; quad: 0 = ABC, 1 = ACD; others 0), t, and the
  * barycentric (u, v) of the hit triangle.  any_hit = 1: entity_id = 1 if
- * occluded else -1.  Output pointers other than entity_id may be NULL. */
+ * occluded else -1.  Output pointers other than entity_id may be NULL.
+ * Directions need not be of unit length (t is in units of them).  The context keeps
+ * the call's staging for its next one, until agx_destroy: pinned host memory for calls
+ * of up to 32,768 rays (at most 1.8 MB), device memory for larger ones (52
+ * bytes a ray of the largest, at most 218 MB: more rays than 2^22 are traced in parts). */
 int  agx_trace_rays(agx_ctx *ctx, const float *o, const float *d,
                     const float *tmin, const float *tmax, uint32_t n, int32_t any_hit,
                     int32_t *entity_id, int32_t *prim_id, float *t, float *u, float *v);
@@ -420,7 +424,8 @@ int  agx_render_batch(agx_ctx *ctx, agx_batch_item *items, uint32_t n, int32_t w
  * 2, plus specular_depth in scenes with delta surfaces; kernels of an empty
  * queue exit at once) and counts its rays on the device.  branches = 0: an
  * autotuner times the first group at 2 spp for 2, 4 and 8 branches, passes
- * of 2^21 / 2^22 / 2^23 paths and 128- / 256-thread traversal blocks
+ * of 2^21 / 2^22 / 2^23 paths and 128- / 256-thread traversal blocks (which
+ * traversals of queues that may hold 2^21 rays do not take: those use 128)
  * (coordinate descent; later groups build meanwhile) and renders the batch
  * with the fastest; otherwise `branches` branches, passes of at most 2^22
  * paths and 128-thread blocks.  Images are bit-identical to agx_render's for
