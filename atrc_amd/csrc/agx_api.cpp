@@ -87,7 +87,7 @@ struct agx_ctx {
     int64_t cap_wh = 0;
     uint32_t *counters = nullptr;    // device: two sets of 4 queue sizes (ping-pong)
     DevCounters *dcnt = nullptr;
-    uint32_t *h_counters = nullptr;  // pinned ring: RING x 4 queue sizes read back asynchronously
+    uint32_t *h_counters = nullptr;  // pinned ring: RING x (3 queue sizes, their sequence word) that kernels write
     float *d_resolve = nullptr;      // normalised film planes (10 floats per pixel), kept between renders
     float *h_resolve = nullptr;      // pinned staging of the planes the caller asked for
     size_t resolve_cap = 0;          // pixels both buffers hold
@@ -126,7 +126,7 @@ struct agx_ctx {
     float *rays_dev = nullptr;       // and the device staging of larger ones (at most RAYS_CHUNK rays, 218 MB)
     uint32_t rays_dev_cap = 0;
     hipEvent_t ev[8]{};
-    std::vector<hipEvent_t> pool;    // timing / readback events, reused across renders
+    std::vector<hipEvent_t> pool;    // timing events, reused across renders
     hipEvent_t event(size_t i) {
         while (pool.size() <= i) {
             hipEvent_t e = nullptr;
